@@ -249,10 +249,16 @@ void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far,
     VLB_REQUIRE(grid % 8 == 0, VLB_ERR_INVALID, "trace grid must be a multiple of 8");
     k_zero_ctr8<<<1, 64, 0, st>>>(a.wctr);
     // recording (hit ids are the same in any shadow order) and multi-bounce
-    // plans keep slot-order shadows
+    // plans keep slot-order shadows.  The multi-bounce kernel takes the
+    // variant's occupancy bound like the direct one: it is bound by the latency
+    // and issue of its eight corner rays per hit, so 8 waves/SIMD with spills
+    // outside the loops beat 3 without (2048 probes x 4096 rays of the
+    // 11k-triangle room: 2.9 ms per bounce at 64 VGPRs against 4.1 at 144).
     if (a.sp.ind.coeffs) {
         if (record) k_trace<true, false, 0, true><<<grid, 256, 0, st>>>(a);
         else if (count) k_trace<false, true, 0, true><<<grid, 256, 0, st>>>(a);
+        else if (occ == 8) k_trace<false, false, 8, true><<<grid, 256, 0, st>>>(a);
+        else if (occ == 6) k_trace<false, false, 6, true><<<grid, 256, 0, st>>>(a);
         else k_trace<false, false, 0, true><<<grid, 256, 0, st>>>(a);
     } else if (record) k_trace<true, false, 0, false><<<grid, 256, 0, st>>>(a);
     else if (count && far) k_trace<false, true, 0, false, true><<<grid, 256, 0, st>>>(a);

@@ -706,19 +706,28 @@ __device__ float3 grid_indirect(const SceneView& sc, const ProbeGridView& g, con
                                 uint32_t& nshadow)
 {
     const float p[3] = {P.x, P.y, P.z};
+    // visibility first, as a mask of hidden corners: only the hit point and
+    // the ray origin are live across the eight traversals, not the basis and
+    // the running sums.  Corners are then found again (same values).
+    uint32_t hidden = 0;
+    if (g.vis) {
+        const float3 org = make_float3(P.x + g.bias * N.x, P.y + g.bias * N.y, P.z + g.bias * N.z);
+        for (int v = 0; v < 8; ++v) {
+            const GridCorner c = grid_corner(g, p, v);
+            if (corner_needs_ray(g, c, sc.ntris)) {
+                ++nshadow;
+                const float3 dir = make_float3(c.dir[0] / c.dist, c.dir[1] / c.dist, c.dir[2] / c.dist);
+                if (trace_any<COUNT, FAR, STRI>(sc, org, dir, 0.0f, c.dist, st, cnt)) hidden |= 1u << v;
+            }
+        }
+    }
     const float n[3] = {N.x, N.y, N.z};
     float Y[16];
     grid_basis(g, n, Y);
     float sw = 0.0f, acc[3] = {0.0f, 0.0f, 0.0f};
     for (int v = 0; v < 8; ++v) {
         const GridCorner c = grid_corner(g, p, v);
-        float w = c.w;
-        if (corner_needs_ray(g, c, sc.ntris)) {
-            ++nshadow;
-            const float3 org = make_float3(P.x + g.bias * N.x, P.y + g.bias * N.y, P.z + g.bias * N.z);
-            const float3 dir = make_float3(c.dir[0] / c.dist, c.dir[1] / c.dist, c.dir[2] / c.dist);
-            if (trace_any<COUNT, FAR, STRI>(sc, org, dir, 0.0f, c.dist, st, cnt)) w = 0.0f;
-        }
+        const float w = (hidden >> v) & 1u ? 0.0f : c.w;
         if (w > 0.0f) {
             float val[3];
             corner_value(g, c.row, Y, val);
