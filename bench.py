@@ -44,6 +44,7 @@ sys.path.insert(0, os.path.join(ROOT, "vulkan-light-bakery_amd"))
 
 METRIC = "probes/sec & Grays/s at ≤1e-3 rel SH err vs FP64; p50/p99 rebake latency"
 HBM_PEAK_GBS = 8000.0
+NODE_BYTES = 64.0    # bytes per BVH4 node visit (4 x 16 B)
 TRI_BYTES = 48.0     # bytes per triangle test (3 x float4)
 
 
@@ -51,12 +52,6 @@ def is_fused(variant):
     """trace_variant 1..12 and 25..36 (far-first shadow queries) run the fused
     trace+shade kernel, 13..24 the wavefront kernels."""
     return not 13 <= variant <= 24
-
-
-def node_bytes(variant):
-    """Bytes fetched per BVH4 node visit: the fused kernels read float nodes
-    (7 x 16 B in use), the wavefront kernels quantized ones (4 x 16 B)."""
-    return 112.0 if is_fused(variant) else 64.0
 
 
 PREC = {"fp32": 0, "bf16": 1, "fp16": 2, "bf16_fast": 3, "fp16_fast": 4}
@@ -145,7 +140,7 @@ def trace_roofline(kernel, variant, cnt_nodes, cnt_tris, launch_s, launches, pro
     bytes are mostly served by L1/L2/MALL, so it can exceed the HBM peak.
     `issue` (from the profile's SQ counters) is the bound that does hold:
     the share of VALU issue slots used and the lanes busy per instruction."""
-    alg = (node_bytes(variant) * cnt_nodes + TRI_BYTES * cnt_tris) / launches
+    alg = (NODE_BYTES * cnt_nodes + TRI_BYTES * cnt_tris) / launches
     prof = None
     if profile:
         prof = profile.get("variants", {}).get(str(variant))
@@ -345,7 +340,7 @@ def served_roofline(ctx, sids, reqs, ps16, warm, server):
     b.destroy()
     steps = server["steps"]
     step_s = server["busy_ms"] / 1e3 / steps
-    alg = (node_bytes(v) * cnt["node_visits"] + TRI_BYTES * cnt["tri_tests"]) / steps
+    alg = (NODE_BYTES * cnt["node_visits"] + TRI_BYTES * cnt["tri_tests"]) / steps
     profile = load_traffic("served_c5_traffic.json")
     prof = (profile or {}).get("variants", {}).get(str(v))
     traffic = prof["hbm_bytes_per_launch"] if prof else None

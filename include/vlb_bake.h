@@ -241,7 +241,7 @@ vlb_status  vlb_debug_inject(vlb_ctx* ctx, int32_t site, int32_t count);
 /* Replaces SceneManager::pushScene + Scene_t::buildAccelerationStructures
  * (src/scene_manager.cpp:1013-1034, 339-443): world-space triangles are
  * uploaded and a BVH is built on the GPU (PLOC, Meister & Bittner 2018,
- * collapsed to a 4-wide BVH kept as float and as 8-bit quantized nodes).
+ * collapsed to a 4-wide BVH of 64-byte nodes).
  * xyz: nverts*3, finite with |x| <= 2^100 (else VLB_ERR_INVALID),
  * idx: ntris*3, normals: nverts*3 or NULL (geometric normals),
  * albedo_rgb: ntris*3 (base colour, env_map.rchit:36-49). */

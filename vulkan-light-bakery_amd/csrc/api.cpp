@@ -565,15 +565,8 @@ vlb_status vlb_scene_export_bvh(vlb_ctx* h, uint32_t scene, float* nodes, size_t
         }
         if (leaf_prims) {
             VLB_REQUIRE(leaf_len >= (size_t)s.ntris, VLB_ERR_INVALID, "leaf buffer too small");
-            std::vector<float4> t((size_t)s.ntris * 3);
-            VLB_HIP(hipMemcpyAsync(t.data(), s.tris.p, t.size() * sizeof(float4), hipMemcpyDeviceToHost,
-                                   c->stream));
-            VLB_HIP(hipStreamSynchronize(c->stream));
-            for (int i = 0; i < s.ntris; ++i) {
-                int32_t v;
-                memcpy(&v, &t[3 * (size_t)i].w, 4);
-                leaf_prims[i] = v;
-            }
+            VLB_HIP(hipMemcpyAsync(leaf_prims, s.leaf_prims.p, (size_t)s.ntris * sizeof(int32_t),
+                                   hipMemcpyDeviceToHost, c->stream));
         }
         VLB_HIP(hipStreamSynchronize(c->stream));
     });

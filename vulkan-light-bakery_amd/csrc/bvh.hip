@@ -195,18 +195,14 @@ __global__ void k_morton(const float4* __restrict__ cen, int n, const float* __r
 // the same time at 16-64.
 constexpr int kPlocRadius = 32;
 
-// Leaf-order triangles and the initial clusters (leaf j = ~j).
-__global__ void k_leaves(const uint32_t* __restrict__ order, int n,
-                         const float4* __restrict__ tri_raw, const float4* __restrict__ lo,
-                         const float4* __restrict__ hi, float4* __restrict__ tris,
-                         float4* __restrict__ clo, float4* __restrict__ chi, int* __restrict__ cid)
+// The initial clusters (leaf j = ~j).
+__global__ void k_leaves(const uint32_t* __restrict__ order, int n, const float4* __restrict__ lo,
+                         const float4* __restrict__ hi, float4* __restrict__ clo,
+                         float4* __restrict__ chi, int* __restrict__ cid)
 {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     uint32_t p = order[j];
-    tris[3 * j + 0] = tri_raw[3 * p + 0];
-    tris[3 * j + 1] = tri_raw[3 * p + 1];
-    tris[3 * j + 2] = tri_raw[3 * p + 2];
     clo[j] = lo[p];
     chi[j] = hi[p];
     cid[j] = ~j;
@@ -376,9 +372,12 @@ __global__ void k_depth(const int* __restrict__ iparent, const int* __restrict__
     atomicMax(depth, d);
 }
 
-// Depth of every inner node (root 0), for the BVH4 collapse.
-__global__ void k_inner_depth(const int* __restrict__ iparent, int nin, int* __restrict__ depth,
-                              int* __restrict__ even)
+// BVH2 -> BVH4: every even-depth BVH2 node becomes a BVH4 node whose
+// children are its grandchildren through inner children, or the child itself
+// when that is a leaf (2 to 4 entries).  Per BVH2 node: its BVH4 node's inner
+// children (low word) and leaves (high word), or 0 for an odd-depth node.
+__global__ void k_count4(const BNode* __restrict__ n2, const int* __restrict__ iparent, int nin,
+                         unsigned long long* __restrict__ count)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nin) return;
@@ -387,8 +386,40 @@ __global__ void k_inner_depth(const int* __restrict__ iparent, int nin, int* __r
         p = iparent[p] >> 1;
         ++d;
     }
-    depth[i] = d;
-    even[i] = (d & 1) == 0 ? 1 : 0;
+    unsigned long long c = 0;
+    if ((d & 1) == 0) {
+        const int4 a = n2[i].d;
+        const int kid[2] = {a.x, a.y};
+        for (int k = 0; k < 2; ++k) {
+            if (kid[k] < 0) {
+                c += 1ull << 32;
+                continue;
+            }
+            const int4 g = n2[kid[k]].d;
+            c += g.x < 0 ? 1ull << 32 : 1ull;
+            c += g.y < 0 ? 1ull << 32 : 1ull;
+        }
+    }
+    count[i] = c;
+}
+
+// BVH4 node ids: the inner children of a node are consecutive, after those of
+// the nodes before it (base = exclusive sum of the counts); the root is 0.
+__global__ void k_number4(const BNode* __restrict__ n2, const unsigned long long* __restrict__ count,
+                          const unsigned long long* __restrict__ base, int nin, int* __restrict__ id4)
+{
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) id4[0] = 0;
+    if (i >= nin || count[i] == 0) return;
+    int next = 1 + (int)(uint32_t)base[i];
+    const int4 a = n2[i].d;
+    const int kid[2] = {a.x, a.y};
+    for (int k = 0; k < 2; ++k) {
+        if (kid[k] < 0) continue;
+        const int4 g = n2[kid[k]].d;
+        if (g.x >= 0) id4[g.x] = next++;
+        if (g.y >= 0) id4[g.y] = next++;
+    }
 }
 
 __device__ __forceinline__ void child_box(const BNode& a, int k, float b[6])
@@ -400,124 +431,123 @@ __device__ __forceinline__ void child_box(const BNode& a, int k, float b[6])
     }
 }
 
-// Grid of one axis of a BVH4 node's box [lo, hi] (finite, |x| <= 2^100):
-// origin o = lo and the smallest float step s with fma(255, s, o) >= hi.  A
-// plane q decodes as fma(q, s, o) here and in the traversal (the same
-// correctly rounded operation, non-decreasing in q), so codes chosen by
-// comparing that decoded value with the float plane are conservative
-// whatever the rounding.
-__host__ __device__ void axis_grid(float lo, float hi, float& o, float& s)
+// FP16 x rounded towards -inf or +inf of the double v, never subnormal (so
+// no flush of subnormals anywhere can move a plane inwards).  |v| <= 65504.
+__host__ __device__ uint32_t half_outward(double v, bool up)
 {
-    o = lo;
-    const double want = ((double)hi - (double)lo) / 255.0;
-    s = (float)want;
-    if ((double)s < want) s = nextafterf(s, __builtin_huge_valf());
-    // s >= the exact extent / 255 makes fma(255, s, o) >= hi already; the
-    // loop only covers a rounded `want`, first in ulps, then by doubling
-    for (int i = 0; fmaf(255.0f, s, o) < hi; ++i)
-        s = i < 8 ? nextafterf(s, __builtin_huge_valf()) : fmaxf(2.0f * s, 0x1p-100f);
-}
-
-// 8-bit codes of one plane of the four children: the largest q whose plane
-// is <= the child's lo (UP false), or the smallest q whose plane is >= its
-// hi (UP true).
-template <bool UP>
-__host__ __device__ uint32_t plane_codes(const float v[4], int m, float o, float s)
-{
-    uint32_t w = 0;
-    for (int k = 0; k < m; ++k) {
-        const float x = v[k];
-        int q = 0;
-        if (s > 0.0f) {
-            const double r = ((double)x - (double)o) / (double)s;
-            q = (int)fmin(fmax(UP ? ceil(r) : floor(r), 0.0), 255.0);
-            if (UP) {
-                while (q < 255 && fmaf((float)q, s, o) < x) ++q;
-                while (q > 0 && fmaf((float)(q - 1), s, o) >= x) --q;
-            } else {
-                while (q > 0 && fmaf((float)q, s, o) > x) --q;
-                while (q < 255 && fmaf((float)(q + 1), s, o) <= x) ++q;
-            }
-        }
-        w |= (uint32_t)q << (8 * k);
+    const _Float16 h0 = (_Float16)(float)v;  // nearest (twice), then stepped
+    uint16_t u = __builtin_bit_cast(uint16_t, h0);
+    for (int i = 0; i < 4; ++i) {
+        const double x = (double)(float)__builtin_bit_cast(_Float16, u);
+        if (up ? x >= v : x <= v) break;
+        // next half towards +inf (up) or -inf
+        const bool neg = (u & 0x8000u) != 0;
+        if ((u & 0x7FFFu) == 0) u = up ? 0x0001u : 0x8001u;
+        else u = (uint16_t)(neg == up ? u - 1 : u + 1);
     }
-    return w;
+    if ((u & 0x7C00u) == 0 && (u & 0x03FFu) != 0) {
+        const bool neg = (u & 0x8000u) != 0;
+        u = up ? (neg ? 0x0000u : 0x0400u) : (neg ? 0x8400u : 0x0000u);
+    }
+    return u;
 }
 
-// BVH2 -> BVH4: every even-depth BVH2 node becomes a BVH4 node whose
-// children are its grandchildren through inner children, or the child
-// itself when that is a leaf (2 to 4 entries).  The float node copies the
-// boxes (exactly as conservative as the BVH2); the quantized node rounds
-// them outward on the node's grid.
-__global__ void k_collapse(const BNode* __restrict__ n2, const int* __restrict__ depth,
-                           const int* __restrict__ idx4, int nin, BNode4* __restrict__ n4,
-                           QNode4* __restrict__ q4)
+// Writes the BVH4 nodes (Node4) and their leaf triangles.  Boxes are widened
+// by `margin` (box_margin), taken relative to the node's origin (FP16) in
+// double, where the differences are exact, and rounded outwards: offsets of at
+// most 2^15 units (the scene's largest coordinate is at most 2^14).
+__global__ void k_collapse(const BNode* __restrict__ n2, const unsigned long long* __restrict__ count,
+                           const unsigned long long* __restrict__ base, const int* __restrict__ id4,
+                           int nin, int ntris, float margin, double per_unit,
+                           const uint32_t* __restrict__ order, const float4* __restrict__ tri_raw,
+                           Node4* __restrict__ n4, float4* __restrict__ tris)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nin || (depth[i] & 1)) return;
-    float bx[4][6];
-    int ch[4];
-    int m = 0;
+    if (i >= nin || count[i] == 0) return;
+    float bi[4][6], bl[4][6], b[6];
+    int leaf[4], ni = 0, nl = 0;
     const BNode a = n2[i];
     for (int k = 0; k < 2; ++k) {
         const int c = k == 0 ? a.d.x : a.d.y;
         if (c < 0) {
-            child_box(a, k, bx[m]);
-            ch[m++] = c;
+            child_box(a, k, b);
+            for (int t = 0; t < 6; ++t) bl[nl][t] = b[t];
+            leaf[nl++] = ~c;
             continue;
         }
         const BNode g = n2[c];
         for (int q = 0; q < 2; ++q) {
             const int gc = q == 0 ? g.d.x : g.d.y;
-            child_box(g, q, bx[m]);
-            ch[m++] = gc < 0 ? gc : idx4[gc];
+            child_box(g, q, b);
+            if (gc < 0) {
+                for (int t = 0; t < 6; ++t) bl[nl][t] = b[t];
+                leaf[nl++] = ~gc;
+            } else {
+                for (int t = 0; t < 6; ++t) bi[ni][t] = b[t];
+                ++ni;
+            }
         }
     }
-    const int used = m;
-    // Unused slots: in the float node an all-+inf box, which the slab test
-    // misses for every ray (each axis gives t = +inf or -inf, or NaN, which
-    // min/max drop, and a unit direction keeps one axis finite), with leaf 0
-    // as its id, so that even a box it did not miss would only re-test a
-    // real triangle; in the quantized node kEmpty (its decoded planes are
-    // finite, slab4<true> checks the id).
-    int chf[4];
-    for (int k = 0; k < used; ++k) chf[k] = ch[k];
-    for (; m < 4; ++m) {
-        for (int t = 0; t < 6; ++t) bx[m][t] = __builtin_huge_valf();
-        ch[m] = kEmpty;
-        chf[m] = ~0;
+    if (ntris == 1) nl = 1;  // the root's two children are the same leaf
+    const int first = (int)(base[i] >> 32);
+    for (int k = 0; k < nl; ++k) {
+        const uint32_t p = order[leaf[k]];
+        for (int t = 0; t < 3; ++t) tris[3 * (size_t)(first + k) + t] = tri_raw[3 * (size_t)p + t];
+        for (int t = 0; t < 6; ++t) bi[ni + k][t] = bl[k][t];
     }
-    BNode4 o;
-    o.lox = make_float4(bx[0][0], bx[1][0], bx[2][0], bx[3][0]);
-    o.loy = make_float4(bx[0][1], bx[1][1], bx[2][1], bx[3][1]);
-    o.loz = make_float4(bx[0][2], bx[1][2], bx[2][2], bx[3][2]);
-    o.hix = make_float4(bx[0][3], bx[1][3], bx[2][3], bx[3][3]);
-    o.hiy = make_float4(bx[0][4], bx[1][4], bx[2][4], bx[3][4]);
-    o.hiz = make_float4(bx[0][5], bx[1][5], bx[2][5], bx[3][5]);
-    o.child = make_int4(chf[0], chf[1], chf[2], chf[3]);
-    o.pad = make_int4(0, 0, 0, 0);
-    n4[idx4[i]] = o;
-    float org[3], stp[3];
-    uint32_t code[6];
-    for (int a = 0; a < 3; ++a) {
-        float lo[4], hi[4];
-        float blo = bx[0][a], bhi = bx[0][3 + a];
-        for (int k = 0; k < used; ++k) {
-            lo[k] = bx[k][a];
-            hi[k] = bx[k][3 + a];
-            blo = fminf(blo, lo[k]);
-            bhi = fmaxf(bhi, hi[k]);
+    const int used = ni + nl;
+    uint32_t org[3], lo[3][4], hi[3][4];
+    for (int x = 0; x < 3; ++x) {
+        float blo = bi[0][x], bhi = bi[0][3 + x];
+        for (int k = 1; k < used; ++k) {
+            blo = fminf(blo, bi[k][x]);
+            bhi = fmaxf(bhi, bi[k][3 + x]);
         }
-        axis_grid(blo, bhi, org[a], stp[a]);
-        code[a] = plane_codes<false>(lo, used, org[a], stp[a]);
-        code[3 + a] = plane_codes<true>(hi, used, org[a], stp[a]);
+        // origin: the node's centre or a child's, whichever lets the rounding
+        // (about 2^-11 of a plane's offset) thicken the children least in
+        // proportion.  Flat children decide: a wall's box must stay thinner
+        // than the offset a shadow ray leaves it with, or every such ray
+        // tests the wall again (centres alone: 19% more triangle tests in a
+        // room of boxes)
+        double best = 0.0, bo = 0.0;
+        for (int t = -1; t < used; ++t) {
+            const double at = t < 0 ? 0.5 * ((double)blo + (double)bhi)
+                                    : 0.5 * ((double)bi[t][x] + (double)bi[t][3 + x]);
+            _Float16 h = (_Float16)(float)(at * per_unit);
+            uint32_t u = __builtin_bit_cast(uint16_t, h);
+            if ((u & 0x7C00u) == 0) u = 0;  // no subnormal origin
+            const double o = (double)(float)__builtin_bit_cast(_Float16, (uint16_t)u) / per_unit;
+            double cost = 0.0;
+            for (int k = 0; k < used; ++k) {
+                const double l = (double)bi[k][x] - margin, g = (double)bi[k][3 + x] + margin;
+                cost += (fabs(l - o) + fabs(g - o)) / fmax(g - l, 1e-300);
+            }
+            if (t < 0 || cost < best) {
+                best = cost;
+                bo = o * per_unit;
+                org[x] = u;
+            }
+        }
+        for (int k = 0; k < 4; ++k) {
+            // unused slots: +inf planes, which no ray hits
+            lo[x][k] = k < used ? half_outward(((double)bi[k][x] - margin) * per_unit - bo, false) : 0x7C00u;
+            hi[x][k] = k < used ? half_outward(((double)bi[k][3 + x] + margin) * per_unit - bo, true) : 0x7C00u;
+        }
     }
-    QNode4 q;
-    q.a = make_float4(org[0], org[1], org[2], stp[0]);
-    q.b = make_float4(stp[1], stp[2], __uint_as_float(code[0]), __uint_as_float(code[1]));
-    q.q = make_uint4(code[2], code[3], code[4], code[5]);
-    q.child = make_int4(ch[0], ch[1], ch[2], ch[3]);
-    q4[idx4[i]] = q;
+    Node4 n;
+    n.oxy = org[0] | org[1] << 16;
+    n.ozn = org[2] | ((1u << used) - (1u << ni)) << 16 | (uint32_t)ni << 20;
+    n.inner = 1 + (int)(uint32_t)base[i];
+    n.leaf = first - ni;
+    for (int p = 0; p < 2; ++p) {
+        n.lox[p] = lo[0][2 * p] | lo[0][2 * p + 1] << 16;
+        n.loy[p] = lo[1][2 * p] | lo[1][2 * p + 1] << 16;
+        n.loz[p] = lo[2][2 * p] | lo[2][2 * p + 1] << 16;
+        n.hix[p] = hi[0][2 * p] | hi[0][2 * p + 1] << 16;
+        n.hiy[p] = hi[1][2 * p] | hi[1][2 * p + 1] << 16;
+        n.hiz[p] = hi[2][2 * p] | hi[2][2 * p + 1] << 16;
+    }
+    n4[id4[i]] = n;
 }
 
 inline int nblk(int n, int b = 256) { return (n + b - 1) / b; }
@@ -575,16 +605,16 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     DevBuf keys = dev_alloc(ctx, (size_t)n * sizeof(uint32_t));
     DevBuf vals = dev_alloc(ctx, (size_t)n * sizeof(uint32_t));
     DevBuf keys2 = dev_alloc(ctx, (size_t)n * sizeof(uint32_t));
-    DevBuf vals2 = dev_alloc(ctx, (size_t)n * sizeof(uint32_t));
+    s.leaf_prims = dev_alloc(ctx, (size_t)n * sizeof(uint32_t));
     k_morton<<<nblk(n), 256, 0, st>>>(cen.as<float4>(), n, bnd.as<float>(), keys.as<uint32_t>(),
                                       vals.as<uint32_t>());
     VLB_HIP(hipGetLastError());
     size_t tmp_bytes = 0;
     VLB_HIP(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys.as<uint32_t>(), keys2.as<uint32_t>(),
-                                      vals.as<uint32_t>(), vals2.as<uint32_t>(), (size_t)n, 0, 30, st));
+                                      vals.as<uint32_t>(), s.leaf_prims.as<uint32_t>(), (size_t)n, 0, 30, st));
     DevBuf tmp = dev_alloc(ctx, tmp_bytes > 0 ? tmp_bytes : 16);
     VLB_HIP(rocprim::radix_sort_pairs(tmp.p, tmp_bytes, keys.as<uint32_t>(), keys2.as<uint32_t>(),
-                                      vals.as<uint32_t>(), vals2.as<uint32_t>(), (size_t)n, 0, 30, st));
+                                      vals.as<uint32_t>(), s.leaf_prims.as<uint32_t>(), (size_t)n, 0, 30, st));
     // hierarchy (PLOC), one host round trip per pass for the cluster count
     const int nin = n > 1 ? n - 1 : 1;
     s.nodes = dev_alloc(ctx, (size_t)nin * sizeof(BNode));
@@ -597,8 +627,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
         chi[k] = dev_alloc(ctx, (size_t)n * sizeof(float4));
         cid[k] = dev_alloc(ctx, (size_t)n * sizeof(int));
     }
-    k_leaves<<<nblk(n), 256, 0, st>>>(vals2.as<uint32_t>(), n, tri_raw.as<float4>(),
-                                      lo.as<float4>(), hi.as<float4>(), s.tris.as<float4>(),
+    k_leaves<<<nblk(n), 256, 0, st>>>(s.leaf_prims.as<uint32_t>(), n, lo.as<float4>(), hi.as<float4>(),
                                       clo[0].as<float4>(), chi[0].as<float4>(), cid[0].as<int>());
     VLB_HIP(hipGetLastError());
     DevBuf dep = dev_alloc(ctx, sizeof(unsigned int));
@@ -652,39 +681,49 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
                                          dep.as<unsigned int>());
     }
     VLB_HIP(hipGetLastError());
-    // BVH4: even-depth BVH2 nodes, numbered by an exclusive scan
-    DevBuf idepth = dev_alloc(ctx, (size_t)nin * sizeof(int));
-    DevBuf even = dev_alloc(ctx, (size_t)nin * sizeof(int));
-    DevBuf idx4 = dev_alloc(ctx, (size_t)nin * sizeof(int));
-    if (n == 1) {
-        const int zero = 0, one = 1;
-        VLB_HIP(hipMemcpyAsync(idepth.p, &zero, sizeof zero, hipMemcpyHostToDevice, st));
-        VLB_HIP(hipMemcpyAsync(even.p, &one, sizeof one, hipMemcpyHostToDevice, st));
-    } else {
-        k_inner_depth<<<nblk(nin), 256, 0, st>>>(iparent.as<int>(), nin, idepth.as<int>(),
-                                                 even.as<int>());
-        VLB_HIP(hipGetLastError());
-    }
+    // BVH4: even-depth BVH2 nodes; an exclusive scan of their child counts
+    // places each one's inner children and leaves
+    DevBuf count = dev_alloc(ctx, (size_t)nin * sizeof(unsigned long long));
+    DevBuf base = dev_alloc(ctx, (size_t)nin * sizeof(unsigned long long));
+    DevBuf id4 = dev_alloc(ctx, (size_t)nin * sizeof(int));
+    k_count4<<<nblk(nin), 256, 0, st>>>(s.nodes.as<BNode>(), iparent.as<int>(), nin,
+                                        count.as<unsigned long long>());
+    VLB_HIP(hipGetLastError());
     size_t scan_bytes = 0;
-    VLB_HIP(rocprim::exclusive_scan(nullptr, scan_bytes, even.as<int>(), idx4.as<int>(), 0, (size_t)nin,
-                                    rocprim::plus<int>(), st));
+    VLB_HIP(rocprim::exclusive_scan(nullptr, scan_bytes, count.as<unsigned long long>(),
+                                    base.as<unsigned long long>(), 0ull, (size_t)nin,
+                                    rocprim::plus<unsigned long long>(), st));
     DevBuf scan_tmp = dev_alloc(ctx, scan_bytes > 0 ? scan_bytes : 16);
-    VLB_HIP(rocprim::exclusive_scan(scan_tmp.p, scan_bytes, even.as<int>(), idx4.as<int>(), 0, (size_t)nin,
-                                    rocprim::plus<int>(), st));
-    int last[2] = {0, 0};
-    VLB_HIP(hipMemcpyAsync(&last[0], idx4.as<int>() + (nin - 1), sizeof(int), hipMemcpyDeviceToHost, st));
-    VLB_HIP(hipMemcpyAsync(&last[1], even.as<int>() + (nin - 1), sizeof(int), hipMemcpyDeviceToHost, st));
+    VLB_HIP(rocprim::exclusive_scan(scan_tmp.p, scan_bytes, count.as<unsigned long long>(),
+                                    base.as<unsigned long long>(), 0ull, (size_t)nin,
+                                    rocprim::plus<unsigned long long>(), st));
+    unsigned long long last[2] = {0, 0};
+    float hb[16];
+    VLB_HIP(hipMemcpyAsync(&last[0], base.as<unsigned long long>() + (nin - 1), sizeof last[0],
+                           hipMemcpyDeviceToHost, st));
+    VLB_HIP(hipMemcpyAsync(&last[1], count.as<unsigned long long>() + (nin - 1), sizeof last[1],
+                           hipMemcpyDeviceToHost, st));
+    VLB_HIP(hipMemcpyAsync(hb, bnd.p, 13 * sizeof(float), hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
-    const int n4 = last[0] + last[1];
-    s.nodes4 = dev_alloc(ctx, (size_t)n4 * sizeof(BNode4));
-    s.qnodes4 = dev_alloc(ctx, (size_t)n4 * sizeof(QNode4));
-    k_collapse<<<nblk(nin), 256, 0, st>>>(s.nodes.as<BNode>(), idepth.as<int>(), idx4.as<int>(), nin,
-                                          s.nodes4.as<BNode4>(), s.qnodes4.as<QNode4>());
+    const int n4 = 1 + (int)(uint32_t)(last[0] + last[1]);
+    // node unit: the power of two that brings the largest coordinate to
+    // [2^13, 2^14) units, so that offsets stay within FP16's range
+    s.maxabs = hb[12];
+    int e = 0;
+    (void)frexpf(s.maxabs, &e);  // maxabs < 2^e; 0 gives e = 0
+    s.unit = ldexpf(1.0f, std::max(e - 14, -100));
+    s.nodes4 = dev_alloc(ctx, (size_t)n4 * sizeof(Node4));
+    k_number4<<<nblk(nin), 256, 0, st>>>(s.nodes.as<BNode>(), count.as<unsigned long long>(),
+                                         base.as<unsigned long long>(), nin, id4.as<int>());
+    VLB_HIP(hipGetLastError());
+    k_collapse<<<nblk(nin), 256, 0, st>>>(s.nodes.as<BNode>(), count.as<unsigned long long>(),
+                                          base.as<unsigned long long>(), id4.as<int>(), nin, n,
+                                          box_margin(s.maxabs), 1.0 / (double)s.unit,
+                                          s.leaf_prims.as<uint32_t>(), tri_raw.as<float4>(),
+                                          s.nodes4.as<Node4>(), s.tris.as<float4>());
     VLB_HIP(hipGetLastError());
     VLB_HIP(hipEventRecord(e1, st));
-    float hb[16];
     unsigned int depth = 0;
-    VLB_HIP(hipMemcpyAsync(hb, bnd.p, 13 * sizeof(float), hipMemcpyDeviceToHost, st));
     VLB_HIP(hipMemcpyAsync(&depth, dep.p, sizeof depth, hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
     float ms = 0.0f;
@@ -699,7 +738,6 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
         s.bmin[a] = hb[6 + a];
         s.bmax[a] = hb[9 + a];
     }
-    s.maxabs = hb[12];
 }
 
 }  // namespace vlb

@@ -31,37 +31,29 @@ struct __align__(16) BNode {
 };
 
 // The traversal kernels walk a 4-wide BVH collapsed from it (half the
-// dependent node fetches of the BVH2 per ray), stored twice with the same
-// node ids: the root is node 0; child ids >= 0 are inner BVH4 nodes, < 0
-// leaves (~ leaf-order triangle), kEmpty an unused slot.
-//
-// BNode4, 128 bytes (112 in use): the boxes of up to four children as float
-// structure-of-arrays (lo.x of child c in lox[c], ...) and their ids.  Read
-// by the fused kernels, which run at the 64-VGPR bound of 8 waves/SIMD where
-// a decode step costs more than the bytes it saves.
-//
-// QNode4, 64 bytes: per axis a grid origin o (the node box's lo) and step s
-// (its extent / 255, rounded up), the children's boxes as 8-bit grid
-// coordinates q (plane = fma(q, s, o); lo codes rounded down, hi codes
-// rounded up, each checked against that very decode when the node is
-// built), and the ids.  A decoded box contains the child's float box, so the
-// slab test sees conservative boxes, slightly larger than the BVH2's (2-6%
-// more node visits).  Read by the wavefront kernels, which have registers to
-// spare and whose node fetches are half the bytes through the texture path.
-struct __align__(16) BNode4 {
-    float4 lox, loy, loz;
-    float4 hix, hiy, hiz;
-    int4   child;
-    int4   pad;
+// dependent node fetches of the BVH2 per ray).  Node4 is 64 bytes, four
+// 16-byte loads, because a visit's cost is its loads as much as its
+// arithmetic (three more loads per divergent visit cost 18% on an 11k-triangle
+// room and 41% on a 1.15M-triangle terrain):
+//  - the children's boxes as FP16 offsets from the node's own origin, in
+//    units of the scene's power-of-two scale.  v_fma_mix_f32 reads an FP16
+//    operand inside an FP32 FMA, so a plane's ray parameter
+//    t = fma(offset, inv, fma(origin, inv, -o * inv)) costs no decode.  The
+//    offsets are rounded outwards from boxes already widened by the margin of
+//    the slab test, so a decoded box contains its child: boxes decide which
+//    nodes are visited, never which triangle is hit.
+//  - children are consecutive: the inner ones first (nodes inner, inner + 1,
+//    ...), then the leaves (triangle leaf + k for child k); unused slots have
+//    all-+inf boxes, which no ray hits.
+struct __align__(64) Node4 {
+    uint32_t oxy;      // origin x, y (FP16, low half first)
+    uint32_t ozn;      // origin z (FP16), leaf slots (4 bits) << 16, number
+                       // of inner children << 20
+    int32_t  inner;    // id of the first inner child
+    int32_t  leaf;     // leaf-order triangle of child k: leaf + k
+    uint32_t lox[2], loy[2], loz[2];  // FP16 offsets: children 0, 1 | 2, 3
+    uint32_t hix[2], hiy[2], hiz[2];
 };
-struct __align__(16) QNode4 {
-    float4 a;      // o.x, o.y, o.z, s.x
-    float4 b;      // s.y, s.z, lo.x codes, lo.y codes (as bits)
-    uint4  q;      // lo.z, hi.x, hi.y, hi.z codes
-    int4   child;
-};
-// (codes of one plane: child k in byte k)
-constexpr int kEmpty = (int)0x80000000;
 
 // Stack entries a BVH4 traversal can hold for a BVH2 of `depth` inner
 // levels: at most 3 pushes per BVH4 level, ceil(depth / 2) levels.
@@ -74,12 +66,12 @@ __host__ __device__ inline uint32_t stack_bound(uint32_t depth)
 // Shading record per prim id = 3 x float4: (n0, albedo.r) (n1, .g) (n2, .b).
 
 struct SceneView {
-    const BNode4* nodes;      // float BVH4 (fused kernels)
-    const QNode4* qnodes;     // quantized BVH4, same ids (wavefront kernels)
+    const Node4*  nodes;
     const float4* tris;
     const float4* shade;
     int           ntris;
     float         maxabs;  // max |coordinate| of the scene's vertices
+    float         unit;    // power of two: world length of a node's unit
 };
 
 struct ShadeParams {
@@ -218,42 +210,42 @@ __device__ __forceinline__ bool wt_hit(const WtRay& w, const float3& v0, const f
 }
 
 // -------------------------------------------------------------- slab test
-// Conservative: widened by 4e-6 relative plus an absolute margin of 64 ulps
-// of the largest coordinate in play, so a box holding an accepted triangle
-// is never culled.  Margins cost node visits, never change a result.
+// Conservative: a node's planes are stored widened by box_margin (128 float
+// roundings of the scene's largest coordinate), which covers the rounding of
+// the plane parameters, of the watertight test and of its t for rays whose
+// origin lies within several scene sizes; apad, in units of t, adds the same
+// margin of the origin's own magnitude for rays that start farther away.
+// Margins cost node visits, never change a result.
 struct SlabRay {
-    float3 inv;
-    float3 oinv;  // o * inv
+    float3 inv;         // node unit / direction
+    float3 oinv;        // origin / direction
     float  apad;
+    bool   nx, ny, nz;  // direction component negative: hi is the near plane
 };
 
-__device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, float maxabs)
+__host__ __device__ __forceinline__ float box_margin(float maxabs)
 {
-    SlabRay s;
-    float dx = d.x == 0.0f ? copysignf(1e-20f, d.x) : d.x;
-    float dy = d.y == 0.0f ? copysignf(1e-20f, d.y) : d.y;
-    float dz = d.z == 0.0f ? copysignf(1e-20f, d.z) : d.z;
-    s.inv = make_float3(1.0f / dx, 1.0f / dy, 1.0f / dz);
-    s.oinv = make_float3(o.x * s.inv.x, o.y * s.inv.y, o.z * s.inv.z);
-    float m = fmaxf(maxabs, fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))));
-    s.apad = m * (64.0f * 1.1920929e-7f);
-    return s;
+    return maxabs * (64.0f * 1.1920929e-7f);
 }
 
-// returns the (widened) entry distance, for near-first ordering, or +inf on
-// a miss
-__device__ __forceinline__ float slab(const SlabRay& s, float lox, float loy, float loz,
-                                      float hix, float hiy, float hiz, float tmin, float tbest)
+__device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, float maxabs, float unit)
 {
-    float t0x = fmaf(lox, s.inv.x, -s.oinv.x), t1x = fmaf(hix, s.inv.x, -s.oinv.x);
-    float t0y = fmaf(loy, s.inv.y, -s.oinv.y), t1y = fmaf(hiy, s.inv.y, -s.oinv.y);
-    float t0z = fmaf(loz, s.inv.z, -s.oinv.z), t1z = fmaf(hiz, s.inv.z, -s.oinv.z);
-    float tn = fmaxf(fmaxf(fminf(t0x, t1x), fminf(t0y, t1y)), fminf(t0z, t1z));
-    float tf = fminf(fminf(fmaxf(t0x, t1x), fmaxf(t0y, t1y)), fmaxf(t0z, t1z));
-    float hi = fminf(tf, tbest);
-    hi = fmaf(fabsf(hi), 4e-6f, hi) + s.apad;
-    const float lo = fmaf(-fabsf(tn), 4e-6f, tn) - s.apad;
-    return (lo <= hi && hi >= tmin) ? lo : __builtin_huge_valf();
+    SlabRay s;
+    // a component this small moves the ray by less than the margin over the
+    // whole scene, and keeps unit / d and o / d finite
+    const float dmin = fmaxf(1e-20f, unit * 0x1p-113f);
+    const float dx = fabsf(d.x) < dmin ? copysignf(dmin, d.x) : d.x;
+    const float dy = fabsf(d.y) < dmin ? copysignf(dmin, d.y) : d.y;
+    const float dz = fabsf(d.z) < dmin ? copysignf(dmin, d.z) : d.z;
+    const float3 r = make_float3(1.0f / dx, 1.0f / dy, 1.0f / dz);
+    s.oinv = make_float3(o.x * r.x, o.y * r.y, o.z * r.z);
+    s.inv = make_float3(unit * r.x, unit * r.y, unit * r.z);
+    s.nx = dx < 0.0f;
+    s.ny = dy < 0.0f;
+    s.nz = dz < 0.0f;
+    const float m = fmaxf(maxabs, fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))));
+    s.apad = box_margin(m);
+    return s;
 }
 
 // ------------------------------------------------------------- traversal
@@ -297,55 +289,11 @@ __device__ __forceinline__ void load_tri(const float4* tris, int leaf, float3& v
     prim = __float_as_int(a.w);
 }
 
-// Planes fma(q, s, o) of the four children for one code word (the decode
-// the node builder checked its codes against).
-__device__ __forceinline__ float4 decode4(uint32_t q, float s, float o)
-{
-    return make_float4(fmaf((float)(q & 255u), s, o), fmaf((float)((q >> 8) & 255u), s, o),
-                       fmaf((float)((q >> 16) & 255u), s, o), fmaf((float)(q >> 24), s, o));
-}
-
-// Float node fetch: the 112 bytes in use (7 x 16 B).
-__device__ __forceinline__ BNode4 load_node(const BNode4* nodes, uint32_t i)
-{
-    const BNode4* p = nodes + i;
-    BNode4 n;
-    n.lox = p->lox;
-    n.loy = p->loy;
-    n.loz = p->loz;
-    n.hix = p->hix;
-    n.hiy = p->hiy;
-    n.hiz = p->hiz;
-    n.child = p->child;
-    return n;
-}
-
-// Quantized node fetch (4 x 16 B) and decode to the float form.
-__device__ __forceinline__ BNode4 load_node(const QNode4* nodes, uint32_t i)
-{
-    const QNode4* p = nodes + i;
-    const float4 a = p->a;
-    const float4 b = p->b;
-    const uint4 q = p->q;
-    BNode4 n;
-    n.lox = decode4(__float_as_uint(b.z), a.w, a.x);
-    n.loy = decode4(__float_as_uint(b.w), b.x, a.y);
-    n.loz = decode4(q.x, b.y, a.z);
-    n.hix = decode4(q.y, a.w, a.x);
-    n.hiy = decode4(q.z, b.x, a.y);
-    n.hiz = decode4(q.w, b.y, a.z);
-    n.child = p->child;
-    return n;
-}
-
 // Node fetches of a wave whose active lanes are all at the same node (about
 // half of the fused kernel's visits on coherent probe rays) come through the
 // scalar cache into scalar registers, leaving the vector memory path, which
 // the divergent fetches keep busy, to those.  Nodes are read-only while any
-// trace kernel runs.  Used by the fused traversal (trace_closest, trace_any);
-// the wavefront kernels refill lanes with unrelated rays, rarely share a
-// node across a wave and measured slower with it (1.48 vs 1.41 ms on the
-// 11k-triangle room bake, 2048 probes x 4096 rays).
+// trace kernel runs.
 typedef int sgpr16_t __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void scalar_load64(unsigned long long addr, sgpr16_t& a)
@@ -357,37 +305,51 @@ __device__ __forceinline__ void scalar_load64(unsigned long long addr, sgpr16_t&
                          : "memory");
 }
 
-__device__ __forceinline__ BNode4 load_node_uniform(const BNode4* p)
+__device__ __forceinline__ Node4 load_node(const Node4* nodes, uint32_t i)
 {
-    const unsigned long long addr = (unsigned long long)p;
-    sgpr16_t a, b;
-    scalar_load64(addr, a);
-    scalar_load64(addr + 64, b);
-    BNode4 n;
-    n.lox = make_float4(__int_as_float(a[0]), __int_as_float(a[1]), __int_as_float(a[2]), __int_as_float(a[3]));
-    n.loy = make_float4(__int_as_float(a[4]), __int_as_float(a[5]), __int_as_float(a[6]), __int_as_float(a[7]));
-    n.loz = make_float4(__int_as_float(a[8]), __int_as_float(a[9]), __int_as_float(a[10]), __int_as_float(a[11]));
-    n.hix = make_float4(__int_as_float(a[12]), __int_as_float(a[13]), __int_as_float(a[14]), __int_as_float(a[15]));
-    n.hiy = make_float4(__int_as_float(b[0]), __int_as_float(b[1]), __int_as_float(b[2]), __int_as_float(b[3]));
-    n.hiz = make_float4(__int_as_float(b[4]), __int_as_float(b[5]), __int_as_float(b[6]), __int_as_float(b[7]));
-    n.child = make_int4(b[8], b[9], b[10], b[11]);
+    const uint4* p = reinterpret_cast<const uint4*>(nodes + i);
+    const uint4 m = p[0], a = p[1], b = p[2], c = p[3];
+    Node4 n;
+    n.oxy = m.x;
+    n.ozn = m.y;
+    n.inner = (int)m.z;
+    n.leaf = (int)m.w;
+    n.lox[0] = a.x;
+    n.lox[1] = a.y;
+    n.loy[0] = a.z;
+    n.loy[1] = a.w;
+    n.loz[0] = b.x;
+    n.loz[1] = b.y;
+    n.hix[0] = b.z;
+    n.hix[1] = b.w;
+    n.hiy[0] = c.x;
+    n.hiy[1] = c.y;
+    n.hiz[0] = c.z;
+    n.hiz[1] = c.w;
     return n;
 }
 
-__device__ __forceinline__ BNode4 load_node_uniform(const QNode4* p)
+__device__ __forceinline__ Node4 load_node_uniform(const Node4* nodes, uint32_t i)
 {
     sgpr16_t w;
-    scalar_load64((unsigned long long)p, w);
-    BNode4 n;
-    const float ox = __int_as_float(w[0]), oy = __int_as_float(w[1]), oz = __int_as_float(w[2]);
-    const float sx = __int_as_float(w[3]), sy = __int_as_float(w[4]), sz = __int_as_float(w[5]);
-    n.lox = decode4((uint32_t)w[6], sx, ox);
-    n.loy = decode4((uint32_t)w[7], sy, oy);
-    n.loz = decode4((uint32_t)w[8], sz, oz);
-    n.hix = decode4((uint32_t)w[9], sx, ox);
-    n.hiy = decode4((uint32_t)w[10], sy, oy);
-    n.hiz = decode4((uint32_t)w[11], sz, oz);
-    n.child = make_int4(w[12], w[13], w[14], w[15]);
+    scalar_load64((unsigned long long)(nodes + i), w);
+    Node4 n;
+    n.oxy = (uint32_t)w[0];
+    n.ozn = (uint32_t)w[1];
+    n.inner = w[2];
+    n.leaf = w[3];
+    n.lox[0] = (uint32_t)w[4];
+    n.lox[1] = (uint32_t)w[5];
+    n.loy[0] = (uint32_t)w[6];
+    n.loy[1] = (uint32_t)w[7];
+    n.loz[0] = (uint32_t)w[8];
+    n.loz[1] = (uint32_t)w[9];
+    n.hix[0] = (uint32_t)w[10];
+    n.hix[1] = (uint32_t)w[11];
+    n.hiy[0] = (uint32_t)w[12];
+    n.hiy[1] = (uint32_t)w[13];
+    n.hiz[0] = (uint32_t)w[14];
+    n.hiz[1] = (uint32_t)w[15];
     return n;
 }
 
@@ -443,75 +405,76 @@ __device__ __forceinline__ bool fetch_wt(const float4* tris, int leaf, const WtR
     return wt_test(w, v0, v1, v2, tmin, tmax, h);
 }
 
-// Child c[k] of a 4-way node with a runtime k, through selects (a register
-// array indexed at run time would be placed in scratch memory).
-__device__ __forceinline__ int pick4(const int c[4], int k)
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+
+// FP16 value k (0 or 1) of a packed pair: an operand of v_fma_mix_f32.
+__device__ __forceinline__ float half_of(uint32_t w, int k)
 {
-    const int a = (k & 1) ? c[1] : c[0];
-    const int b = (k & 1) ? c[3] : c[2];
-    return (k & 2) ? b : a;
+    return (float)__builtin_bit_cast(half2_t, w)[k];
 }
 
-// Hit leaf children as a 4-bit mask; their entry distances are cleared so
-// that only inner children are sorted and pushed.
-__device__ __forceinline__ uint32_t take_leaves(float e[4], const int c[4])
+// c ? a : b of a packed pair; the empty asm keeps the compiler from unpacking
+// the halves first (two selects and two shifts instead of one select).
+__device__ __forceinline__ uint32_t pick_pair(bool c, uint32_t a, uint32_t b)
 {
+    uint32_t r = c ? a : b;
+    __asm__("" : "+v"(r));
+    return r;
+}
+
+// What a visit found: entry distances e[k] of the hit inner children (+inf:
+// missed, leaf or unused), their ids c[k], and the hit leaf children as a
+// 4-bit mask, child k being leaf-order triangle leaf + k.
+struct NodeHits {
+    float    e[4];
+    int      c[4];
+    uint32_t leaves;
+    int      leaf;
+};
+
+__device__ __forceinline__ void slab4(const SlabRay& s, const Node4& n, float tmin, float tbest,
+                                      NodeHits& h)
+{
+    // near and far planes by the direction's signs: 12 selects of packed
+    // pairs instead of a min and a max per child and axis
+    const float ax = fmaf(half_of(n.oxy, 0), s.inv.x, -s.oinv.x);
+    const float ay = fmaf(half_of(n.oxy, 1), s.inv.y, -s.oinv.y);
+    const float az = fmaf(half_of(n.ozn, 0), s.inv.z, -s.oinv.z);
+    h.leaf = n.leaf;
     uint32_t m = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-        if (e[k] != __builtin_huge_valf() && c[k] < 0) {
-            m |= 1u << k;
-            e[k] = __builtin_huge_valf();
-        }
-    return m;
-}
-
-// Entry distances of the four children (+inf: missed or empty slot).
-// CHECK_EMPTY: the node's unused slots are marked kEmpty (quantized nodes);
-// a float node's unused slots hold all-+inf boxes that the slab test misses.
-template <bool CHECK_EMPTY>
-__device__ __forceinline__ void slab4(const SlabRay& s, const BNode4& n, float tmin, float tbest,
-                                      float e[4], int c[4])
-{
-    c[0] = n.child.x;
-    c[1] = n.child.y;
-    c[2] = n.child.z;
-    c[3] = n.child.w;
-    e[0] = slab(s, n.lox.x, n.loy.x, n.loz.x, n.hix.x, n.hiy.x, n.hiz.x, tmin, tbest);
-    e[1] = slab(s, n.lox.y, n.loy.y, n.loz.y, n.hix.y, n.hiy.y, n.hiz.y, tmin, tbest);
-    e[2] = slab(s, n.lox.z, n.loy.z, n.loz.z, n.hix.z, n.hiy.z, n.hiz.z, tmin, tbest);
-    e[3] = slab(s, n.lox.w, n.loy.w, n.loz.w, n.hix.w, n.hiy.w, n.hiz.w, tmin, tbest);
-    if (CHECK_EMPTY) {
+    for (int p = 0; p < 2; ++p) {
+        const uint32_t nx = pick_pair(s.nx, n.hix[p], n.lox[p]), fx = pick_pair(s.nx, n.lox[p], n.hix[p]);
+        const uint32_t ny = pick_pair(s.ny, n.hiy[p], n.loy[p]), fy = pick_pair(s.ny, n.loy[p], n.hiy[p]);
+        const uint32_t nz = pick_pair(s.nz, n.hiz[p], n.loz[p]), fz = pick_pair(s.nz, n.loz[p], n.hiz[p]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (c[k] == kEmpty) e[k] = __builtin_huge_valf();
+        for (int q = 0; q < 2; ++q) {
+            const int k = 2 * p + q;
+            const float tn = fmaxf(fmaxf(fmaf(half_of(nx, q), s.inv.x, ax), fmaf(half_of(ny, q), s.inv.y, ay)),
+                                   fmaf(half_of(nz, q), s.inv.z, az)) - s.apad;
+            const float tf = fminf(fminf(fminf(fmaf(half_of(fx, q), s.inv.x, ax),
+                                               fmaf(half_of(fy, q), s.inv.y, ay)),
+                                         fmaf(half_of(fz, q), s.inv.z, az)), tbest);
+            const bool hit = tn <= tf && tf >= tmin;
+            // inner children come first
+            h.e[k] = hit && n.ozn >= (uint32_t)(k + 1) << 20 ? tn : __builtin_huge_valf();
+            h.c[k] = n.inner + k;
+            m |= hit ? 1u << k : 0u;
+        }
     }
+    h.leaves = m & (n.ozn >> 16);
 }
 
-// Entry distances and ids of the children of node i, and its hit leaf
-// children as a 4-bit mask (take_leaves).  The node comes through
-// the scalar cache when its address is the same in every active lane (checked
-// on the address, so lanes of a multi-job wave on different scenes take the
-// vector path), else per lane.  Each path runs the slab tests on its own
-// registers: merging the two fetches first would copy the 28 scalar node
-// words into vector registers on every uniform visit.
-template <typename NodeT>
-__device__ __forceinline__ uint32_t fetch_slab4(const NodeT* nodes, uint32_t i, const SlabRay& s,
-                                                float tmin, float tbest, float e[4], int c[4])
+// Visits node i: through the scalar cache when every active lane is at it
+// (their base pointer is the same), else per lane.
+__device__ __forceinline__ void fetch_slab4(const Node4* nodes, uint32_t i, const SlabRay& s,
+                                            float tmin, float tbest, NodeHits& h)
 {
-    const NodeT* p = nodes + i;
-    const unsigned long long a = (unsigned long long)p;
-    const unsigned long long u =
-        ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32) |
-        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
-    if (__all(a == u)) {
-        const BNode4 n = load_node_uniform(reinterpret_cast<const NodeT*>(u));
-        slab4<std::is_same<NodeT, QNode4>::value>(s, n, tmin, tbest, e, c);
-        return take_leaves(e, c);
-    }
-    const BNode4 n = load_node(nodes, i);
-    slab4<std::is_same<NodeT, QNode4>::value>(s, n, tmin, tbest, e, c);
-    return take_leaves(e, c);
+    const uint32_t u = __builtin_amdgcn_readfirstlane(i);
+    Node4 n;
+    if (__all(i == u)) n = load_node_uniform(nodes, u);
+    else n = load_node(nodes, i);
+    slab4(s, n, tmin, tbest, h);
 }
 
 // Compare-exchange of two (entry distance, child id) pairs held as one 64-bit
@@ -624,24 +587,23 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
 {
     if (sc.ntris <= 0) return -1;
     const WtRay w = wt_setup(o, d);
-    const SlabRay s = slab_setup(o, d, sc.maxabs);
+    const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
     float tbest = tmax, bV = 0.0f, bW = 0.0f, bdet = 1.0f;
     int best = -1;
     int sp = 0;
     uint32_t node = 0;
     for (;;) {
         if (COUNT) ++cnt.nodes;
-        float e[4];
-        int c[4];
-        const uint32_t hit_leaves = fetch_slab4(sc.nodes, node, s, tmin, tbest, e, c);
+        NodeHits n;
+        fetch_slab4(sc.nodes, node, s, tmin, tbest, n);
         // leaves one at a time per lane: the wave runs as many tests as its
         // busiest lane has hit leaves, not one per child slot
-        for (uint32_t leaves = hit_leaves; leaves != 0; leaves &= leaves - 1) {
+        for (uint32_t leaves = n.leaves; leaves != 0; leaves &= leaves - 1) {
             int prim;
             if (COUNT) ++cnt.tris;
             WtHit h;
             // t <= tbest holds on acceptance; an equal t keeps the lower prim id
-            if (fetch_wt<STRI>(sc.tris, ~pick4(c, __builtin_ctz(leaves)), w, tmin, tbest, h, prim) &&
+            if (fetch_wt<STRI>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tbest, h, prim) &&
                 (best < 0 || h.t < tbest || prim < best)) {
                 tbest = h.t;
                 best = prim;
@@ -650,7 +612,7 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
                 bdet = h.det;
             }
         }
-        if (!next_node(e, c, st, sp, node)) break;
+        if (!next_node(n.e, n.c, st, sp, node)) break;
     }
     if (best >= 0) {
         t_out = tbest;
@@ -669,21 +631,20 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
 {
     if (sc.ntris <= 0) return false;
     const WtRay w = wt_setup(o, d);
-    const SlabRay s = slab_setup(o, d, sc.maxabs);
+    const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
     int sp = 0;
     uint32_t node = 0;
     for (;;) {
         if (COUNT) ++cnt.nodes;
-        float e[4];
-        int c[4];
-        const uint32_t hit_leaves = fetch_slab4(sc.nodes, node, s, tmin, tmax, e, c);
-        for (uint32_t leaves = hit_leaves; leaves != 0; leaves &= leaves - 1) {
+        NodeHits n;
+        fetch_slab4(sc.nodes, node, s, tmin, tmax, n);
+        for (uint32_t leaves = n.leaves; leaves != 0; leaves &= leaves - 1) {
             int prim;
             if (COUNT) ++cnt.tris;
             WtHit h;
-            if (fetch_wt<STRI>(sc.tris, ~pick4(c, __builtin_ctz(leaves)), w, tmin, tmax, h, prim)) return true;
+            if (fetch_wt<STRI>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tmax, h, prim)) return true;
         }
-        if (!next_node<FAR ? kOrderFar : kOrderSlot>(e, c, st, sp, node)) break;
+        if (!next_node<FAR ? kOrderFar : kOrderSlot>(n.e, n.c, st, sp, node)) break;
     }
     return false;
 }

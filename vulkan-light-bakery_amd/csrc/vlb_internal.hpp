@@ -87,8 +87,9 @@ struct Scene {
     int ntris = 0;
     int nnodes = 0;           // BVH2 inner nodes (build product, exported)
     int nnodes4 = 0;          // BVH4 nodes (traversed)
-    DevBuf nodes, nodes4, qnodes4, tris, shade;
-    float maxabs = 0.0f;
+    DevBuf nodes, nodes4, tris, shade;
+    DevBuf leaf_prims;        // triangle of each leaf of the BVH2
+    float maxabs = 0.0f, unit = 1.0f;
     float bmin[3] = {0, 0, 0}, bmax[3] = {0, 0, 0};
     uint32_t depth = 0;
     double build_ms = 0.0;
@@ -97,16 +98,16 @@ struct Scene {
     // the context's mutex (so a release cannot slip in between the lookup
     // and the raise), lowered from any thread.
     std::atomic<int> users{0};
-    size_t bytes() const { return nodes.bytes + nodes4.bytes + qnodes4.bytes + tris.bytes + shade.bytes; }
+    size_t bytes() const { return nodes.bytes + nodes4.bytes + tris.bytes + shade.bytes + leaf_prims.bytes; }
     SceneView view() const
     {
         SceneView v;
-        v.nodes = nodes4.as<BNode4>();
-        v.qnodes = qnodes4.as<QNode4>();
+        v.nodes = nodes4.as<Node4>();
         v.tris = tris.as<float4>();
         v.shade = shade.as<float4>();
         v.ntris = ntris;
         v.maxabs = maxabs;
+        v.unit = unit;
         return v;
     }
 };

@@ -89,7 +89,7 @@ __device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravSta
             return false;
         }
         const float4 pp = a.probes[probe];
-        trav_init(T, a.sc.maxabs, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z), a.tmin,
+        trav_init(T, a.sc, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z), a.tmin,
                   a.tmax);
         return true;
     }
@@ -117,7 +117,7 @@ __device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravSta
         *vis = 0;
         return false;
     }
-    trav_init(T, a.sc.maxabs, s.org, s.dir, 0.0f, s.dist);
+    trav_init(T, a.sc, s.org, s.dir, 0.0f, s.dist);
     return true;
 }
 
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(256) void k_rays(BakeArgs a, size_t nitems, unsigne
         }
         // --- one traversal step for active lanes
         if (act) {
-            if (trav_step<ANY, COUNT>(T, a.sc.qnodes, a.sc.tris, st, q, cnt)) {
+            if (trav_step<ANY, COUNT>(T, a.sc.nodes, a.sc.tris, st, q, cnt)) {
                 if (ANY) {
                     a.vis[(size_t)slot * a.nvis + light] = (uint8_t)(T.best == 0 ? 1 : 0);
                 } else if (T.best >= 0) {

@@ -133,11 +133,11 @@ struct TravState {
     bool live;  // `node` is still to be visited
 };
 
-__device__ __forceinline__ void trav_init(TravState& T, float maxabs, const float3& o,
+__device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, const float3& o,
                                           const float3& d, float tmin, float tmax)
 {
     T.w = wt_setup(o, d);
-    T.s = slab_setup(o, d, maxabs);
+    T.s = slab_setup(o, d, sc.maxabs, sc.unit);
     T.tmin = tmin;
     T.tb = tmax;
     T.best = -1;
@@ -155,21 +155,18 @@ __device__ __forceinline__ void trav_init(TravState& T, float maxabs, const floa
 // - 4, so a write past the end stays inside the queue), hit inner children
 // go on the stack.
 template <bool ANY, bool COUNT>
-__device__ __forceinline__ void visit_node(TravState& T, const QNode4* nodes, const Stack& st,
+__device__ __forceinline__ void visit_node(TravState& T, const Node4* nodes, const Stack& st,
                                            const LeafQueue& q, TraceCount& cnt)
 {
-    const BNode4 n = load_node(nodes, T.node);
     if (COUNT) ++cnt.nodes;
-    float e[4];
-    int c[4];
-    slab4<true>(T.s, n, T.tmin, T.tb, e, c);
-    const uint32_t leaves = take_leaves(e, c);
+    NodeHits n;
+    slab4(T.s, load_node(nodes, T.node), T.tmin, T.tb, n);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        q.lds[T.nq * 256] = (uint32_t)~c[k];
-        T.nq += (int)((leaves >> k) & 1u);
+        q.lds[T.nq * 256] = (uint32_t)(n.leaf + k);
+        T.nq += (int)((n.leaves >> k) & 1u);
     }
-    T.live = next_node<ANY ? kOrderSlot : kOrderNear>(e, c, st, T.sp, T.node);
+    T.live = next_node<ANY ? kOrderSlot : kOrderNear>(n.e, n.c, st, T.sp, T.node);
 }
 
 // Tests every queued triangle of the active lanes (the wave runs as many
@@ -206,7 +203,7 @@ __device__ __forceinline__ void test_queue(TravState& T, const float4* tris, con
 // a node visit, then (wave-uniform) the queued tests when due.  Returns true
 // when the ray is finished (ANY: T.best = 0 on an accepted triangle).
 template <bool ANY, bool COUNT>
-__device__ __forceinline__ bool trav_step(TravState& T, const QNode4* nodes, const float4* tris,
+__device__ __forceinline__ bool trav_step(TravState& T, const Node4* nodes, const float4* tris,
                                           const Stack& st, const LeafQueue& q, TraceCount& cnt)
 {
     if (T.live && T.nq <= kLeafQueue - 4) visit_node<ANY, COUNT>(T, nodes, st, q, cnt);
