@@ -45,7 +45,7 @@ sys.path.insert(0, os.path.join(ROOT, "vulkan-light-bakery_amd"))
 METRIC = "probes/sec & Grays/s at ≤1e-3 rel SH err vs FP64; p50/p99 rebake latency"
 HBM_PEAK_GBS = 8000.0
 NODE_BYTES = 64.0    # bytes per BVH4 node visit (4 x 16 B)
-TRI_BYTES = 48.0     # bytes per triangle test (3 x float4)
+TRI_BYTES = 36.0     # bytes per triangle test (3 x 12 B of a 64-byte record)
 
 
 def is_fused(variant):
@@ -135,8 +135,8 @@ def trace_roofline(kernel, variant, cnt_nodes, cnt_tris, launch_s, launches, pro
     measured by rocprofv3 (FETCH_SIZE x2 + WRITE_SIZE, committed under
     profiles/ for this kernel and workload) over the live event-timed launch
     duration, so frac <= 1 is a real HBM fraction.  `alg_rate_gbs` is the
-    algorithmic node + triangle byte rate (112 or 64 B per BVH4 node visit +
-    48 B per triangle test, counted by the kernels' counting pass): those
+    algorithmic node + triangle byte rate (64 B per BVH4 node visit +
+    36 B per triangle test, counted by the kernels' counting pass): those
     bytes are mostly served by L1/L2/MALL, so it can exceed the HBM peak.
     `issue` (from the profile's SQ counters) is the bound that does hold:
     the share of VALU issue slots used and the lanes busy per instruction."""

@@ -48,7 +48,8 @@ __global__ void k_zero_ctr8(unsigned long long* c)
 // OCC > 0 asks the compiler for OCC waves per SIMD (VGPR budget 512/OCC).
 // IND: plans with the multi-bounce term.  FAR: shadow queries visit children
 // far first (same radiance; fewer node visits on some scenes).
-template <bool RECORD, bool COUNT, int OCC, bool IND, bool FAR = false>
+template <bool RECORD, bool COUNT, int OCC, bool IND, bool FAR = false,
+          bool WIDE = RECORD || COUNT>
 __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_trace(BakeArgs a)
 {
     __shared__ uint32_t lds[kLdsDepth * 256];
@@ -110,7 +111,7 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_trace(BakeArgs a)
         if (probe < a.P && dd.w != 0.0f) {
             const float4 pp = a.probes[probe];
             int hp = -1;
-            L = shade_ray<COUNT, IND, FAR, kStriShadow>(a.sc, a.sp, make_float3(pp.x, pp.y, pp.z),
+            L = shade_ray<COUNT, IND, FAR, WIDE>(a.sc, a.sp, make_float3(pp.x, pp.y, pp.z),
                                  make_float3(dd.x, dd.y, dd.z), a.tmin, a.tmax, st, cnt, nshadow, hp);
             if (RECORD) {
                 const size_t ri = (size_t)a.probe_perm[probe] * a.R + a.dir_perm[r];
@@ -254,15 +255,18 @@ void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far,
     // and issue of its eight corner rays per hit, so 8 waves/SIMD with spills
     // outside the loops beat 3 without (2048 probes x 4096 rays of the
     // 11k-triangle room: 2.9 ms per bounce at 64 VGPRs against 4.1 at 144).
+    const bool wide = a.sc.ntris >= kNarrowTris;  // else record64's short form
     if (a.sp.ind.coeffs) {
         if (record) k_trace<true, false, 0, true><<<grid, 256, 0, st>>>(a);
         else if (count) k_trace<false, true, 0, true><<<grid, 256, 0, st>>>(a);
+        else if (wide) k_trace<false, false, 0, true, false, true><<<grid, 256, 0, st>>>(a);
         else if (occ == 8) k_trace<false, false, 8, true><<<grid, 256, 0, st>>>(a);
         else if (occ == 6) k_trace<false, false, 6, true><<<grid, 256, 0, st>>>(a);
         else k_trace<false, false, 0, true><<<grid, 256, 0, st>>>(a);
     } else if (record) k_trace<true, false, 0, false><<<grid, 256, 0, st>>>(a);
     else if (count && far) k_trace<false, true, 0, false, true><<<grid, 256, 0, st>>>(a);
     else if (count) k_trace<false, true, 0, false><<<grid, 256, 0, st>>>(a);
+    else if (wide) k_trace<false, false, 0, false, false, true><<<grid, 256, 0, st>>>(a);
     else if (far) {
         if (occ == 8) k_trace<false, false, 8, false, true><<<grid, 256, 0, st>>>(a);
         else if (occ == 6) k_trace<false, false, 6, false, true><<<grid, 256, 0, st>>>(a);

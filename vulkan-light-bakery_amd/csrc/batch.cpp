@@ -225,6 +225,7 @@ MultiArgs RoundBufs::args(const JobDesc* jobs, const uint8_t* table, const size_
     a.spill = spill.as<uint32_t>();
     a.focc = focc;
     a.far = focc >= 0 && far ? 1 : 0;
+    a.wide = wide ? 1 : 0;
     a.fgrid = focc < 0 ? 0 : fgrid[(focc == 8 ? 2 : (focc == 6 ? 1 : 0)) + 3 * a.far];
     a.spill_stride = (uint32_t)(focc < 0 ? grid : a.fgrid) * 256u;
     a.counters = counters.as<unsigned long long>();
@@ -480,6 +481,7 @@ void build_batch(Context& ctx, const vlb_batch_job* jobs, uint32_t njobs, const 
     }
     b.table = upload_vec(ctx, host);
     b.rb.alloc(ctx, std::max<size_t>(peak, 2), nvis, depth);
+    for (const Scene* sc : b.scenes) b.rb.wide = b.rb.wide || sc->ntris >= kNarrowTris;
     b.ev.assign(2 * Batch::kRing, nullptr);
     for (auto& e : b.ev) VLB_HIP(hipEventCreate(&e));
     b.info.jobs = njobs;

@@ -492,7 +492,12 @@ __global__ void k_collapse(const BNode* __restrict__ n2, const unsigned long lon
     const int first = (int)(base[i] >> 32);
     for (int k = 0; k < nl; ++k) {
         const uint32_t p = order[leaf[k]];
-        for (int t = 0; t < 3; ++t) tris[3 * (size_t)(first + k) + t] = tri_raw[3 * (size_t)p + t];
+        float4* out = tris + (size_t)(first + k) * (kTriWords / 4);
+        const float4 u = tri_raw[3 * (size_t)p], v = tri_raw[3 * (size_t)p + 1], w = tri_raw[3 * (size_t)p + 2];
+        out[0] = make_float4(u.x, u.y, u.z, u.x);
+        out[1] = make_float4(u.y, v.x, v.y, v.z);
+        out[2] = make_float4(v.x, v.y, w.x, w.y);
+        out[3] = make_float4(w.z, w.x, w.y, u.w);
         for (int t = 0; t < 6; ++t) bi[ni + k][t] = bl[k][t];
     }
     const int used = ni + nl;
@@ -618,7 +623,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     // hierarchy (PLOC), one host round trip per pass for the cluster count
     const int nin = n > 1 ? n - 1 : 1;
     s.nodes = dev_alloc(ctx, (size_t)nin * sizeof(BNode));
-    s.tris = dev_alloc(ctx, (size_t)n * 3 * sizeof(float4));
+    s.tris = dev_alloc(ctx, (size_t)n * kTriWords * sizeof(float));
     DevBuf iparent = dev_alloc(ctx, (size_t)nin * sizeof(int));
     DevBuf lparent = dev_alloc(ctx, (size_t)n * sizeof(int));
     DevBuf clo[2], chi[2], cid[2];

@@ -62,12 +62,18 @@ __host__ __device__ inline uint32_t stack_bound(uint32_t depth)
     return 3u * ((depth + 1u) / 2u) + 1u;
 }
 
-// Leaf-order triangle = 3 x float4: (v0, prim id bits) (v1, 0) (v2, 0).
+// Leaf-order triangle = 16 words, one 64-byte line: per vertex x y z x y, so
+// that the three coordinates in any cyclic order are consecutive (the
+// watertight test reads them in its ray's order with one load per vertex,
+// instead of reordering them with 24 selects), and the prim id.
+constexpr int kTriWords = 16;
+constexpr int kTriPrim = 15;
+
 // Shading record per prim id = 3 x float4: (n0, albedo.r) (n1, .g) (n2, .b).
 
 struct SceneView {
     const Node4*  nodes;
-    const float4* tris;
+    const float*  tris;       // kTriWords per leaf
     const float4* shade;
     int           ntris;
     float         maxabs;  // max |coordinate| of the scene's vertices
@@ -111,37 +117,26 @@ __device__ __forceinline__ float dot3(const float3& a, const float3& b)
 // Woop, Benthin, Wald, "Watertight Ray/Triangle Intersection", JCGT 2(1),
 // 2013: shear the triangle into ray space along the dominant axis kz, take
 // the 2D edge functions U, V, W (recomputed in double when one is zero), and
-// accept when they share a sign.
+// accept when they share a sign.  The paper also exchanges kx and ky where
+// d[kz] < 0, to keep the winding; without culling that only negates U, V, W,
+// their sum and T together, exactly, so it is left out.
 struct WtRay {
-    float3 o;
-    // axis permutation (kx, ky, kz) as select masks: kz = 0 -> r1, kz = 1 ->
-    // r2, kz = 2 -> neither; swp exchanges kx and ky (d[kz] < 0)
-    bool  r1, r2, swp;
-    float Sx, Sy, Sz;
+    float3   o;    // origin (kx, ky, kz)
+    float    Sx, Sy, Sz;
+    uint32_t rot;  // byte offset of (kx, ky, kz) in a vertex's x y z x y
 };
-
-// (v[kx], v[ky], v[kz]) with selects only (no indexed access: a runtime
-// component index would be lowered to divergent branches).
-__device__ __forceinline__ float3 wt_perm(const WtRay& w, const float3& v)
-{
-    const float a = w.r1 ? v.y : (w.r2 ? v.z : v.x);
-    const float b = w.r1 ? v.z : (w.r2 ? v.x : v.y);
-    const float c = w.r1 ? v.x : (w.r2 ? v.y : v.z);
-    return make_float3(w.swp ? b : a, w.swp ? a : b, c);
-}
 
 __device__ __forceinline__ WtRay wt_setup(const float3& o, const float3& d)
 {
-    WtRay w;
-    w.o = o;
     const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
-    const int kz = (ax > ay) ? ((ax > az) ? 0 : 2) : ((ay > az) ? 1 : 2);
-    w.r1 = kz == 0;
-    w.r2 = kz == 1;
-    w.swp = false;
-    const float3 pd0 = wt_perm(w, d);
-    w.swp = pd0.z < 0.0f;
-    const float3 pd = wt_perm(w, d);
+    const bool zx = ax > ay && ax > az;             // kz = x: order y z x
+    const bool zy = !(ax > ay) && ay > az;          // kz = y: order z x y
+    const float3 pd = make_float3(zx ? d.y : (zy ? d.z : d.x), zx ? d.z : (zy ? d.x : d.y),
+                                  zx ? d.x : (zy ? d.y : d.z));
+    WtRay w;
+    w.o = make_float3(zx ? o.y : (zy ? o.z : o.x), zx ? o.z : (zy ? o.x : o.y),
+                      zx ? o.x : (zy ? o.y : o.z));
+    w.rot = zx ? 4u : (zy ? 8u : 0u);
     w.Sx = pd.x / pd.z;
     w.Sy = pd.y / pd.z;
     w.Sz = 1.0f / pd.z;
@@ -155,12 +150,13 @@ struct WtHit {
     float t, V, W, det;
 };
 
+// v0, v1, v2: the vertices in the ray's coordinate order.
 __device__ __forceinline__ bool wt_test(const WtRay& w, const float3& v0, const float3& v1,
                                         const float3& v2, float tmin, float tmax, WtHit& h)
 {
-    const float3 A = wt_perm(w, make_float3(v0.x - w.o.x, v0.y - w.o.y, v0.z - w.o.z));
-    const float3 B = wt_perm(w, make_float3(v1.x - w.o.x, v1.y - w.o.y, v1.z - w.o.z));
-    const float3 C = wt_perm(w, make_float3(v2.x - w.o.x, v2.y - w.o.y, v2.z - w.o.z));
+    const float3 A = make_float3(v0.x - w.o.x, v0.y - w.o.y, v0.z - w.o.z);
+    const float3 B = make_float3(v1.x - w.o.x, v1.y - w.o.y, v1.z - w.o.z);
+    const float3 C = make_float3(v2.x - w.o.x, v2.y - w.o.y, v2.z - w.o.z);
     const float Ax = A.x - w.Sx * A.z;
     const float Ay = A.y - w.Sy * A.z;
     const float Bx = B.x - w.Sx * B.z;
@@ -194,18 +190,6 @@ __device__ __forceinline__ bool wt_test(const WtRay& w, const float3& v0, const 
     h.V = V;
     h.W = W;
     h.det = det;
-    return true;
-}
-
-__device__ __forceinline__ bool wt_hit(const WtRay& w, const float3& v0, const float3& v1,
-                                       const float3& v2, float tmin, float tmax, float& t_out,
-                                       float& u_out, float& v_out)
-{
-    WtHit h;
-    if (!wt_test(w, v0, v1, v2, tmin, tmax, h)) return false;
-    t_out = h.t;
-    u_out = h.V / h.det;
-    v_out = h.W / h.det;
     return true;
 }
 
@@ -277,16 +261,35 @@ struct TraceCount {
     uint32_t tris = 0;
 };
 
-__device__ __forceinline__ void load_tri(const float4* tris, int leaf, float3& v0, float3& v1,
-                                         float3& v2, int& prim)
+// Address of byte `byte` (< 64) of 64-byte record i (nodes and triangles).
+// WIDE: any scene.  Without it the byte offset is kept in 32 bits, the form
+// the vector loads take next to a scalar base (one instruction instead of
+// two 64-bit ones and a register pair): for scenes with less than 2^26
+// triangles (kNarrowTris), so that every offset is below 2^32.
+constexpr int kNarrowTris = 1 << 26;
+
+template <bool WIDE>
+__device__ __forceinline__ const char* record64(const void* base, uint32_t i, uint32_t byte)
 {
-    const float4 a = tris[3 * leaf + 0];
-    const float4 b = tris[3 * leaf + 1];
-    const float4 c = tris[3 * leaf + 2];
-    v0 = make_float3(a.x, a.y, a.z);
-    v1 = make_float3(b.x, b.y, b.z);
-    v2 = make_float3(c.x, c.y, c.z);
-    prim = __float_as_int(a.w);
+    if (WIDE) return static_cast<const char*>(base) + (((size_t)i << 6) + byte);
+    return static_cast<const char*>(base) + (size_t)((i << 6) + byte);
+}
+
+// The vertices of triangle `leaf` in the ray's coordinate order: three 12-byte
+// loads from one line.
+template <bool WIDE>
+__device__ __forceinline__ void load_tri(const float* tris, int leaf, const WtRay& w, float3& v0,
+                                         float3& v1, float3& v2)
+{
+    const char* p = record64<WIDE>(tris, (uint32_t)leaf, w.rot);
+    v0 = *reinterpret_cast<const float3*>(p);
+    v1 = *reinterpret_cast<const float3*>(p + 20);
+    v2 = *reinterpret_cast<const float3*>(p + 40);
+}
+
+__device__ __forceinline__ int tri_prim(const float* tris, int leaf)
+{
+    return __float_as_int(tris[(size_t)leaf * kTriWords + kTriPrim]);
 }
 
 // Node fetches of a wave whose active lanes are all at the same node (about
@@ -305,9 +308,10 @@ __device__ __forceinline__ void scalar_load64(unsigned long long addr, sgpr16_t&
                          : "memory");
 }
 
+template <bool WIDE>
 __device__ __forceinline__ Node4 load_node(const Node4* nodes, uint32_t i)
 {
-    const uint4* p = reinterpret_cast<const uint4*>(nodes + i);
+    const uint4* p = reinterpret_cast<const uint4*>(record64<WIDE>(nodes, i, 0));
     const uint4 m = p[0], a = p[1], b = p[2], c = p[3];
     Node4 n;
     n.oxy = m.x;
@@ -353,55 +357,17 @@ __device__ __forceinline__ Node4 load_node_uniform(const Node4* nodes, uint32_t 
     return n;
 }
 
-// Watertight test of triangle `leaf` for the fused traversal.  SCALAR: when
-// every active lane tests the same triangle, its record comes through the
-// scalar cache (32 + 16 bytes, exactly the record) and the test runs on the
-// scalar operands, sparing the vector memory path three 16-byte loads per
-// lane; else, and without SCALAR, each lane loads its own.  Each path runs
-// its own test, so the scalar words are never copied into vector registers.
-// The multi-job kernel takes SCALAR in both queries (a batch of 64 jobs over
-// four scenes: 196.4 vs 202.9 ms per trace stage; 200.0 with the shadow
-// queries alone).  The single-bake kernel takes it in the shadow queries
-// only (1.15M-triangle terrain, 16,384 probes x 16,384 rays: 38.25 vs 39.27
-// ms; the 11k-triangle room bake unchanged): in its closest-hit query the
-// extra scalar registers spill into vector-register lanes read back in the
-// loop, and the room bake ran 1.03-1.04 vs 0.99-1.00 ms.
-typedef int sgpr8_t __attribute__((ext_vector_type(8)));
-typedef int sgpr4_t __attribute__((ext_vector_type(4)));
-
-template <bool SCALAR>
-__device__ __forceinline__ bool fetch_wt(const float4* tris, int leaf, const WtRay& w, float tmin,
-                                         float tmax, WtHit& h, int& prim)
+// Watertight test of triangle `leaf`.  Always through the vector path: a
+// record that every active lane reads in the same order could come through
+// the scalar cache, but the compare, the branch and the scalar registers cost
+// more than the three 12-byte loads (24-job batch 72.5 ms with the scalar
+// form, 71.0 without; 11k-triangle room plan 0.974 against 0.923 ms).
+template <bool WIDE>
+__device__ __forceinline__ bool fetch_wt(const float* tris, int leaf, const WtRay& w, float tmin,
+                                         float tmax, WtHit& h)
 {
-    if (!SCALAR) {
-        float3 v0, v1, v2;
-        load_tri(tris, leaf, v0, v1, v2, prim);
-        return wt_test(w, v0, v1, v2, tmin, tmax, h);
-    }
-    const float4* p = tris + 3 * leaf;
-    const unsigned long long a = (unsigned long long)p;
-    const unsigned long long u =
-        ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32) |
-        (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a);
-    if (__all(a == u)) {
-        sgpr8_t x;
-        sgpr4_t y;
-        // early-clobber: the first load's destination never overlaps the
-        // address the second one reads
-        __asm__ __volatile__("s_load_dwordx8 %0, %2, 0x0\n\t"
-                             "s_load_dwordx4 %1, %2, 0x20\n\t"
-                             "s_waitcnt lgkmcnt(0)"
-                             : "=&s"(x), "=&s"(y)
-                             : "s"(u)
-                             : "memory");
-        prim = x[3];
-        return wt_test(w, make_float3(__int_as_float(x[0]), __int_as_float(x[1]), __int_as_float(x[2])),
-                       make_float3(__int_as_float(x[4]), __int_as_float(x[5]), __int_as_float(x[6])),
-                       make_float3(__int_as_float(y[0]), __int_as_float(y[1]), __int_as_float(y[2])),
-                       tmin, tmax, h);
-    }
     float3 v0, v1, v2;
-    load_tri(tris, leaf, v0, v1, v2, prim);
+    load_tri<WIDE>(tris, leaf, w, v0, v1, v2);
     return wt_test(w, v0, v1, v2, tmin, tmax, h);
 }
 
@@ -467,13 +433,14 @@ __device__ __forceinline__ void slab4(const SlabRay& s, const Node4& n, float tm
 
 // Visits node i: through the scalar cache when every active lane is at it
 // (their base pointer is the same), else per lane.
+template <bool WIDE>
 __device__ __forceinline__ void fetch_slab4(const Node4* nodes, uint32_t i, const SlabRay& s,
                                             float tmin, float tbest, NodeHits& h)
 {
     const uint32_t u = __builtin_amdgcn_readfirstlane(i);
     Node4 n;
     if (__all(i == u)) n = load_node_uniform(nodes, u);
-    else n = load_node(nodes, i);
+    else n = load_node<WIDE>(nodes, i);
     slab4(s, n, tmin, tbest, h);
 }
 
@@ -580,7 +547,9 @@ __device__ __forceinline__ bool next_node(float e[4], int c[4], const Stack& st,
 // triangles in [tmin, tmax].  Returns the prim id or -1.  Any BVH whose
 // boxes are conservative gives the same answer: every triangle that could
 // beat the current best is tested, and ties go to the lower prim id.
-template <bool COUNT, bool STRI = false>
+// The best triangle is held as its leaf; prim ids are read for the rare equal
+// distances and once at the end.
+template <bool COUNT, bool WIDE = true>
 __device__ int trace_closest(const SceneView& sc, const float3& o, const float3& d, float tmin,
                              float tmax, float& t_out, float& u_out, float& v_out,
                              const Stack& st, TraceCount& cnt)
@@ -595,18 +564,18 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
     for (;;) {
         if (COUNT) ++cnt.nodes;
         NodeHits n;
-        fetch_slab4(sc.nodes, node, s, tmin, tbest, n);
+        fetch_slab4<WIDE>(sc.nodes, node, s, tmin, tbest, n);
         // leaves one at a time per lane: the wave runs as many tests as its
         // busiest lane has hit leaves, not one per child slot
         for (uint32_t leaves = n.leaves; leaves != 0; leaves &= leaves - 1) {
-            int prim;
             if (COUNT) ++cnt.tris;
+            const int leaf = n.leaf + __builtin_ctz(leaves);
             WtHit h;
             // t <= tbest holds on acceptance; an equal t keeps the lower prim id
-            if (fetch_wt<STRI>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tbest, h, prim) &&
-                (best < 0 || h.t < tbest || prim < best)) {
+            if (fetch_wt<WIDE>(sc.tris, leaf, w, tmin, tbest, h) &&
+                (best < 0 || h.t < tbest || tri_prim(sc.tris, leaf) < tri_prim(sc.tris, best))) {
                 tbest = h.t;
-                best = prim;
+                best = leaf;
                 bV = h.V;
                 bW = h.W;
                 bdet = h.det;
@@ -618,14 +587,14 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
         t_out = tbest;
         u_out = bV / bdet;
         v_out = bW / bdet;
+        best = tri_prim(sc.tris, best);
     }
     return best;
 }
 
 // Shadow query: true if any triangle is accepted in [tmin, tmax].  FAR: the
 // inner children far first, else in slot order (same answer either way).
-// STRI: uniform triangle records through the scalar cache (fetch_wt).
-template <bool COUNT, bool FAR = false, bool STRI = false>
+template <bool COUNT, bool FAR = false, bool WIDE = true>
 __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d, float tmin,
                           float tmax, const Stack& st, TraceCount& cnt)
 {
@@ -637,12 +606,11 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
     for (;;) {
         if (COUNT) ++cnt.nodes;
         NodeHits n;
-        fetch_slab4(sc.nodes, node, s, tmin, tmax, n);
+        fetch_slab4<WIDE>(sc.nodes, node, s, tmin, tmax, n);
         for (uint32_t leaves = n.leaves; leaves != 0; leaves &= leaves - 1) {
-            int prim;
             if (COUNT) ++cnt.tris;
             WtHit h;
-            if (fetch_wt<STRI>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tmax, h, prim)) return true;
+            if (fetch_wt<WIDE>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tmax, h)) return true;
         }
         if (!next_node<FAR ? kOrderFar : kOrderSlot>(n.e, n.c, st, sp, node)) break;
     }
@@ -679,7 +647,7 @@ __device__ __forceinline__ float unorm8(float x)
 // Indirect term of a multi-bounce bake at hit point P with the two-sided
 // shading normal N: the grid lookup of probe_grid.hpp (visibility rays to the
 // corner probes traced here, counted as shadow rays), times g.scale.
-template <bool COUNT, bool FAR = false, bool STRI = false>
+template <bool COUNT, bool FAR = false, bool WIDE = true>
 __device__ float3 grid_indirect(const SceneView& sc, const ProbeGridView& g, const float3& P,
                                 const float3& N, const Stack& st, TraceCount& cnt,
                                 uint32_t& nshadow)
@@ -696,7 +664,7 @@ __device__ float3 grid_indirect(const SceneView& sc, const ProbeGridView& g, con
             if (corner_needs_ray(g, c, sc.ntris)) {
                 ++nshadow;
                 const float3 dir = make_float3(c.dir[0] / c.dist, c.dir[1] / c.dist, c.dir[2] / c.dist);
-                if (trace_any<COUNT, FAR, STRI>(sc, org, dir, 0.0f, c.dist, st, cnt)) hidden |= 1u << v;
+                if (trace_any<COUNT, FAR, WIDE>(sc, org, dir, 0.0f, c.dist, st, cnt)) hidden |= 1u << v;
             }
         }
     }
@@ -750,7 +718,7 @@ __device__ __forceinline__ float3 shadow_origin(const ShadeParams& sp, const flo
 // Lambert term of light j at hit point P with the two-sided normal N: the
 // contribution E cos is formed before the shadow query, so only it (not E
 // and the cosine) is live across the traversal; added to acc when unoccluded.
-template <bool COUNT, bool FAR = false, bool STRI = false>
+template <bool COUNT, bool FAR = false, bool WIDE = true>
 __device__ __forceinline__ void light_term(const SceneView& sc, const ShadeParams& sp, int j,
                                            const float3& P, const float3& N, float3& acc,
                                            const Stack& st, TraceCount& cnt, uint32_t& nshadow)
@@ -763,7 +731,7 @@ __device__ __forceinline__ void light_term(const SceneView& sc, const ShadeParam
         const float3 c = make_float3(E.x * cosNL, E.y * cosNL, E.z * cosNL);
         const float3 org = shadow_origin(sp, P, N);
         ++nshadow;
-        if (!trace_any<COUNT, FAR, STRI>(sc, org, Ld, 0.0f, dist, st, cnt)) {
+        if (!trace_any<COUNT, FAR, WIDE>(sc, org, Ld, 0.0f, dist, st, cnt)) {
             acc.x = acc.x + c.x;
             acc.y = acc.y + c.y;
             acc.z = acc.z + c.z;
@@ -792,19 +760,14 @@ __device__ __forceinline__ void hit_point_normal(const SceneView& sc, int prim, 
 // Radiance carried by one primary ray.  `nshadow` counts traced shadow rays.
 // IND compiles the multi-bounce term in (used only when sp.ind.coeffs is
 // set); direct-only kernels are built without it and keep its registers free.
-// FAR: shadow queries visit children far first (same radiance).  STRI:
-// where uniform triangle records come through the scalar cache (fetch_wt):
-// kStriClosest in the closest-hit query, kStriShadow in the shadow queries.
-enum : int { kStriClosest = 1, kStriShadow = 2 };
-
-template <bool COUNT, bool IND = false, bool FAR = false, int STRI = 0>
+// FAR: shadow queries visit children far first (same radiance).
+template <bool COUNT, bool IND = false, bool FAR = false, bool WIDE = true>
 __device__ float3 shade_ray(const SceneView& sc, const ShadeParams& sp, const float3& o,
                             const float3& d, float tmin, float tmax, const Stack& st,
                             TraceCount& cnt, uint32_t& nshadow, int& hit_prim)
 {
     float t = 0.0f, u = 0.0f, v = 0.0f;
-    constexpr bool kShadowScalar = (STRI & kStriShadow) != 0;
-    const int prim = trace_closest<COUNT, (STRI & kStriClosest) != 0>(sc, o, d, tmin, tmax, t, u, v, st, cnt);
+    const int prim = trace_closest<COUNT, WIDE>(sc, o, d, tmin, tmax, t, u, v, st, cnt);
     hit_prim = prim;
     const bool ref = sp.mode == VLB_SHADE_REFERENCE;
     if (prim < 0) {
@@ -840,7 +803,7 @@ __device__ float3 shade_ray(const SceneView& sc, const ShadeParams& sp, const fl
         bool in_shadow = true;
         if (sDotN != 0.0f) {
             ++nshadow;
-            in_shadow = trace_any<COUNT, FAR, kShadowScalar>(sc, org, Ln, 0.0f, Llen, st, cnt);
+            in_shadow = trace_any<COUNT, FAR, WIDE>(sc, org, Ln, 0.0f, Llen, st, cnt);
         }
         float diffuse = 0.0f, spec = 0.0f;
         if (!in_shadow) {
@@ -880,8 +843,8 @@ __device__ float3 shade_ray(const SceneView& sc, const ShadeParams& sp, const fl
     // (unless the indirect term needs them)
     const int nl = sp.nlights;
     for (int j = 0; j + 1 < nl; ++j)
-        light_term<COUNT, FAR, kShadowScalar>(sc, sp, j, P, N, acc, st, cnt, nshadow);
-    if (nl > 0) light_term<COUNT, FAR, kShadowScalar>(sc, sp, nl - 1, P, N, acc, st, cnt, nshadow);
+        light_term<COUNT, FAR, WIDE>(sc, sp, j, P, N, acc, st, cnt, nshadow);
+    if (nl > 0) light_term<COUNT, FAR, WIDE>(sc, sp, nl - 1, P, N, acc, st, cnt, nshadow);
     // albedo read after the shadow queries rather than held across them (the
     // compiler barrier keeps it from reusing the loads of the normals, which
     // it would otherwise keep in scratch across the traversals)
@@ -891,7 +854,7 @@ __device__ float3 shade_ray(const SceneView& sc, const ShadeParams& sp, const fl
     const float kInvPi = 0.318309886183790671538f;
     if (!IND || !sp.ind.coeffs)
         return make_float3(alb.x * acc.x * kInvPi, alb.y * acc.y * kInvPi, alb.z * acc.z * kInvPi);
-    const float3 E = grid_indirect<COUNT, FAR, kShadowScalar>(sc, sp.ind, P, N, st, cnt, nshadow);
+    const float3 E = grid_indirect<COUNT, FAR, WIDE>(sc, sp.ind, P, N, st, cnt, nshadow);
     return make_float3(alb.x * acc.x * kInvPi + alb.x * E.x, alb.y * acc.y * kInvPi + alb.y * E.y,
                        alb.z * acc.z * kInvPi + alb.z * E.z);
 }

@@ -79,7 +79,7 @@ __device__ __forceinline__ void decode_slot(const JobDesc& J, int tb, int pt0, i
 struct LaneRay {
     TravState T;
     const Node4* nodes;
-    const float4* tris;
+    const float* tris;
     int slot, light;
 };
 
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void k_rays_jobs(MultiArgs a, const JobDesc* _
                 if (ANY) {
                     a.vis[(size_t)R.slot * a.nvis + R.light] = (uint8_t)(R.T.best == 0 ? 1 : 0);
                 } else if (R.T.best >= 0) {
-                    a.hits[R.slot] = make_int4(R.T.best, __float_as_int(R.T.tb),
+                    a.hits[R.slot] = make_int4(tri_prim(R.tris, R.T.best), __float_as_int(R.T.tb),
                                                __float_as_int(R.T.bV / R.T.bdet),
                                                __float_as_int(R.T.bW / R.T.bdet));
                 } else {
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(256) void k_rays_jobs(MultiArgs a, const JobDesc* _
 // wave fetches 64 items at a time (a chunk lies within a pair of trace tiles,
 // hence one segment and one job).  Same values as the wavefront passes, bit
 // for bit.
-template <bool COUNT, int OCC, bool FAR = false>
+template <bool COUNT, int OCC, bool FAR = false, bool WIDE = COUNT>
 __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs a,
                                                                        const JobDesc* __restrict__ jobs,
                                                                        const Segment* __restrict__ seg,
@@ -323,7 +323,7 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs
         if (probe < J.P && dd.w != 0.0f) {
             const float4 pp = J.probes[probe];
             int hp = -1;
-            L = shade_ray<COUNT, false, FAR, kStriClosest | kStriShadow>(J.sc, J.sp, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z),
+            L = shade_ray<COUNT, false, FAR, WIDE>(J.sc, J.sp, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z),
                                  J.tmin, J.tmax, st, cnt, nshadow, hp);
         }
         float* out = a.rad + (size_t)tile * 1536 + l * 8 + e;
@@ -476,6 +476,7 @@ void launch_multi_trace(const MultiArgs& a, bool count, int grid, int shade_grid
         VLB_REQUIRE(a.fgrid % 8 == 0 && a.fgrid > 0, VLB_ERR_INVALID, "fused grid must be a multiple of 8");
         if (count && a.far) k_fused_jobs<true, 0, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
         else if (count) k_fused_jobs<true, 0><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
+        else if (a.wide) k_fused_jobs<false, 0, false, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
         else if (a.far) {
             if (a.focc == 8) k_fused_jobs<false, 8, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
             else if (a.focc == 6) k_fused_jobs<false, 6, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);

@@ -80,6 +80,7 @@ struct RoundBufs {
     int nvis = 0;             // visibility bytes per ray
     uint32_t depth = 0;       // deepest BVH served
     int grid = 0, shade_grid = 0, pgrid = 0, mgrid = 0;
+    bool wide = false;          // a job's scene has kNarrowTris triangles or more
     int fgrid[6] = {};          // fused kernel grids at occupancy 0, 6, 8 (+3: far-first shadows)
     DevBuf rad, hits, vis, wctr, spill, counters;
     void alloc(Context& ctx, size_t cap_tiles, int nvis, uint32_t depth);

@@ -284,6 +284,18 @@ bool Server::admit_one(Request* r, size_t& upload_used, std::vector<Upload>& ups
         // lock order: the server's mutex, then the context's
         std::lock_guard<std::recursive_mutex> lk(ctx->mtx);
         Scene& sc = find_scene(*ctx, r->scene);
+        if (sc.ntris >= kNarrowTris && !rb.wide) {
+            // the first request on such a scene: capture the step again with
+            // the kernel for it
+            rb.wide = true;
+            if (gexec) {
+                VLB_HIP(hipStreamSynchronize(stream));
+                (void)hipGraphExecDestroy(gexec);
+                (void)hipGraphDestroy(graph);
+                gexec = nullptr;
+                graph = nullptr;
+            }
+        }
         bool built = false;
         js.rt = cache.get(*ctx, p, K, RS, &built);
         if (built) VLB_HIP(hipStreamSynchronize(ctx->stream));

@@ -103,7 +103,7 @@ struct Scene {
     {
         SceneView v;
         v.nodes = nodes4.as<Node4>();
-        v.tris = tris.as<float4>();
+        v.tris = tris.as<float>();
         v.shade = shade.as<float4>();
         v.ntris = ntris;
         v.maxabs = maxabs;
@@ -385,6 +385,7 @@ struct MultiArgs {
                               // occupancy (0 = compiler's choice, 6, 8 waves/SIMD)
     int fgrid;                // grid of the fused kernel
     int far;                  // fused kernel: far-first shadow queries
+    int wide;                 // fused kernel: 64-bit record offsets (record64)
 };
 
 // ------------------------------------------------------ probe-grid lookup

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void k_rays(BakeArgs a, size_t nitems, unsigne
                 if (ANY) {
                     a.vis[(size_t)slot * a.nvis + light] = (uint8_t)(T.best == 0 ? 1 : 0);
                 } else if (T.best >= 0) {
-                    a.hits[slot] = make_int4(T.best, __float_as_int(T.tb), __float_as_int(T.bV / T.bdet),
+                    a.hits[slot] = make_int4(tri_prim(a.sc.tris, T.best), __float_as_int(T.tb), __float_as_int(T.bV / T.bdet),
                                              __float_as_int(T.bW / T.bdet));
                 } else {
                     a.hits[slot] = make_int4(-1, 0, 0, 0);

@@ -125,7 +125,7 @@ struct TravState {
     WtRay w;
     SlabRay s;
     float tmin, tb;
-    int best;
+    int best;   // leaf of the closest hit so far, -1 none (ANY: 0 = hit)
     float bV, bW, bdet;
     uint32_t node;
     int sp;
@@ -160,7 +160,7 @@ __device__ __forceinline__ void visit_node(TravState& T, const Node4* nodes, con
 {
     if (COUNT) ++cnt.nodes;
     NodeHits n;
-    slab4(T.s, load_node(nodes, T.node), T.tmin, T.tb, n);
+    slab4(T.s, load_node<true>(nodes, T.node), T.tmin, T.tb, n);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         q.lds[T.nq * 256] = (uint32_t)(n.leaf + k);
@@ -172,23 +172,23 @@ __device__ __forceinline__ void visit_node(TravState& T, const Node4* nodes, con
 // Tests every queued triangle of the active lanes (the wave runs as many
 // rounds as its longest queue) and empties the queues.
 template <bool ANY, bool COUNT>
-__device__ __forceinline__ void test_queue(TravState& T, const float4* tris, const LeafQueue& q,
+__device__ __forceinline__ void test_queue(TravState& T, const float* tris, const LeafQueue& q,
                                            TraceCount& cnt)
 {
     for (int i = 0; __any(i < T.nq); ++i) {
         if (i < T.nq && !(ANY && T.best == 0)) {
             float3 v0, v1, v2;
-            int prim;
-            load_tri(tris, (int)q.lds[i * 256], v0, v1, v2, prim);
+            const int leaf = (int)q.lds[i * 256];
+            load_tri<true>(tris, leaf, T.w, v0, v1, v2);
             if (COUNT) ++cnt.tris;
             WtHit h;
             if (ANY) {
                 if (wt_test(T.w, v0, v1, v2, T.tmin, T.tb, h)) T.best = 0;
             } else if (wt_test(T.w, v0, v1, v2, T.tmin, T.tb, h) &&
-                       (T.best < 0 || h.t < T.tb || prim < T.best)) {
+                       (T.best < 0 || h.t < T.tb || tri_prim(tris, leaf) < tri_prim(tris, T.best))) {
                 // t <= tbest holds on acceptance; an equal t keeps the lower prim id
                 T.tb = h.t;
-                T.best = prim;
+                T.best = leaf;
                 T.bV = h.V;
                 T.bW = h.W;
                 T.bdet = h.det;
@@ -203,7 +203,7 @@ __device__ __forceinline__ void test_queue(TravState& T, const float4* tris, con
 // a node visit, then (wave-uniform) the queued tests when due.  Returns true
 // when the ray is finished (ANY: T.best = 0 on an accepted triangle).
 template <bool ANY, bool COUNT>
-__device__ __forceinline__ bool trav_step(TravState& T, const Node4* nodes, const float4* tris,
+__device__ __forceinline__ bool trav_step(TravState& T, const Node4* nodes, const float* tris,
                                           const Stack& st, const LeafQueue& q, TraceCount& cnt)
 {
     if (T.live && T.nq <= kLeafQueue - 4) visit_node<ANY, COUNT>(T, nodes, st, q, cnt);
