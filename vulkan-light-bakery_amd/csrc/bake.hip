@@ -52,14 +52,10 @@ template <bool RECORD, bool COUNT, int OCC, bool IND, bool FAR = false,
           bool WIDE = RECORD || COUNT>
 __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_trace(BakeArgs a)
 {
-    __shared__ uint32_t lds[kLdsDepth * 256];
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    Stack st;
-    st.lds = &lds[tid];
-    st.spill = a.spill + (size_t)blockIdx.x * 256 + tid;
-    st.spill_stride = a.spill_stride;
-    st.depth = kLdsDepth;
+    Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
     TraceCount cnt;
     uint32_t nshadow = 0;
     // 32 64-aligned ranges, range 4x + w owned by wave w of the workgroups on
@@ -182,12 +178,8 @@ __global__ __launch_bounds__(256) void k_trace_closest(SceneView sc, const float
                                                        float* tout, float* uout, float* vout,
                                                        uint32_t* spill, uint32_t stride)
 {
-    __shared__ uint32_t lds[kLdsDepth * 256];
-    Stack st;
-    st.lds = &lds[threadIdx.x];
-    st.spill = spill + (size_t)blockIdx.x * 256 + threadIdx.x;
-    st.spill_stride = stride;
-    st.depth = kLdsDepth;
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
+    Stack st = make_stack(lds, kLdsDepth, spill + (size_t)blockIdx.x * 256 + threadIdx.x, stride);
     TraceCount cnt;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const float3 o = make_float3(org[3 * i], org[3 * i + 1], org[3 * i + 2]);
@@ -207,12 +199,8 @@ __global__ __launch_bounds__(256) void k_trace_occluded(SceneView sc, const floa
                                                         float tmin, uint8_t* occ,
                                                         uint32_t* spill, uint32_t stride)
 {
-    __shared__ uint32_t lds[kLdsDepth * 256];
-    Stack st;
-    st.lds = &lds[threadIdx.x];
-    st.spill = spill + (size_t)blockIdx.x * 256 + threadIdx.x;
-    st.spill_stride = stride;
-    st.depth = kLdsDepth;
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
+    Stack st = make_stack(lds, kLdsDepth, spill + (size_t)blockIdx.x * 256 + threadIdx.x, stride);
     TraceCount cnt;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const float3 o = make_float3(org[3 * i], org[3 * i + 1], org[3 * i + 2]);

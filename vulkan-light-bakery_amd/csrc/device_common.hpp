@@ -221,7 +221,9 @@ __device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, 
     const float dx = fabsf(d.x) < dmin ? copysignf(dmin, d.x) : d.x;
     const float dy = fabsf(d.y) < dmin ? copysignf(dmin, d.y) : d.y;
     const float dz = fabsf(d.z) < dmin ? copysignf(dmin, d.z) : d.z;
-    const float3 r = make_float3(1.0f / dx, 1.0f / dy, 1.0f / dz);
+    // hardware reciprocals (1 ulp, far inside the margin): 30 instructions
+    // fewer per ray than correctly rounded divides
+    const float3 r = make_float3(__builtin_amdgcn_rcpf(dx), __builtin_amdgcn_rcpf(dy), __builtin_amdgcn_rcpf(dz));
     s.oinv = make_float3(o.x * r.x, o.y * r.y, o.z * r.z);
     s.inv = make_float3(unit * r.x, unit * r.y, unit * r.z);
     s.nx = dx < 0.0f;
@@ -233,27 +235,53 @@ __device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, 
 }
 
 // ------------------------------------------------------------- traversal
-// Stack: entries [0, depth) in LDS at lds[i * 256] (lane-interleaved,
-// conflict-free), deeper entries in a global spill area at
-// spill[(i - depth) * spill_stride].
+// Stack of one lane: entries [0, depth) in LDS, 256 words apart (lane-
+// interleaved, conflict-free), deeper ones in a global spill area at
+// spill[(i - depth) * spill_stride].  The position is the LDS address of the
+// next free entry, counted on past the last row for spilled entries.  The row
+// below entry 0 holds kStackEnd, so popping an empty stack yields it and needs
+// no test of its own (with addresses kept instead of indexes, 2% of every
+// trace stage: 24-job batch 71.1 -> 69.3 ms).
+typedef __attribute__((address_space(3))) uint32_t lds_u32;
+constexpr uint32_t kStackEnd = 0xFFFFFFFFu;
+constexpr int stack_words(int depth) { return (depth + 1) * 256; }  // LDS of a workgroup
+
 struct Stack {
-    uint32_t* lds;
+    lds_u32*  lds;     // entry 0
     uint32_t* spill;
     uint32_t  spill_stride;
-    int       depth = kLdsDepth;  // LDS entries per lane (a constant of the kernel)
+    uint32_t  full;    // LDS address (row base) where fewer than 3 rows are left
+    int       depth;   // LDS entries per lane (a constant of the kernel)
 };
 
-__device__ __forceinline__ void push(const Stack& st, int& sp, uint32_t v)
+// `lds` is the workgroup's array of stack_words(depth) words, `spill` this
+// lane's first spill entry.
+__device__ __forceinline__ Stack make_stack(uint32_t* lds, int depth, uint32_t* spill, uint32_t stride)
 {
-    if (sp < st.depth) st.lds[sp * 256] = v;
-    else st.spill[(size_t)(sp - st.depth) * st.spill_stride] = v;
-    ++sp;
+    Stack st;
+    lds_u32* row0 = (lds_u32*)lds;
+    row0[threadIdx.x] = kStackEnd;
+    st.lds = row0 + 256 + threadIdx.x;
+    st.spill = spill;
+    st.spill_stride = stride;
+    st.full = (uint32_t)(uintptr_t)(row0 + 256 * (depth - 1));
+    st.depth = depth;
+    return st;
 }
-__device__ __forceinline__ uint32_t pop(const Stack& st, int& sp)
+
+__device__ __forceinline__ void push(const Stack& st, lds_u32*& top, uint32_t v)
 {
-    --sp;
-    if (sp < st.depth) return st.lds[sp * 256];
-    return st.spill[(size_t)(sp - st.depth) * st.spill_stride];
+    const int i = (int)(top - st.lds) >> 8;
+    if (i < st.depth) *top = v;
+    else st.spill[(size_t)(i - st.depth) * st.spill_stride] = v;
+    top += 256;
+}
+__device__ __forceinline__ uint32_t pop(const Stack& st, lds_u32*& top)
+{
+    top -= 256;
+    const int i = (int)(top - st.lds) >> 8;  // -1: the kStackEnd row
+    if (i < st.depth) return *top;
+    return st.spill[(size_t)(i - st.depth) * st.spill_stride];
 }
 
 struct TraceCount {
@@ -398,37 +426,53 @@ struct NodeHits {
     int      leaf;
 };
 
-__device__ __forceinline__ void slab4(const SlabRay& s, const Node4& n, float tmin, float tbest,
-                                      NodeHits& h)
+// The slab tests of a node's four children, their near and far planes picked.
+struct NodePlanes {
+    uint32_t nx[2], ny[2], nz[2], fx[2], fy[2], fz[2];
+};
+
+__device__ __forceinline__ void slab4(const SlabRay& s, const Node4& n, const NodePlanes& b, float tmin,
+                                      float tbest, NodeHits& h)
 {
-    // near and far planes by the direction's signs: 12 selects of packed
-    // pairs instead of a min and a max per child and axis
     const float ax = fmaf(half_of(n.oxy, 0), s.inv.x, -s.oinv.x);
     const float ay = fmaf(half_of(n.oxy, 1), s.inv.y, -s.oinv.y);
     const float az = fmaf(half_of(n.ozn, 0), s.inv.z, -s.oinv.z);
     h.leaf = n.leaf;
     uint32_t m = 0;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const uint32_t nx = pick_pair(s.nx, n.hix[p], n.lox[p]), fx = pick_pair(s.nx, n.lox[p], n.hix[p]);
-        const uint32_t ny = pick_pair(s.ny, n.hiy[p], n.loy[p]), fy = pick_pair(s.ny, n.loy[p], n.hiy[p]);
-        const uint32_t nz = pick_pair(s.nz, n.hiz[p], n.loz[p]), fz = pick_pair(s.nz, n.loz[p], n.hiz[p]);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int k = 2 * p + q;
-            const float tn = fmaxf(fmaxf(fmaf(half_of(nx, q), s.inv.x, ax), fmaf(half_of(ny, q), s.inv.y, ay)),
-                                   fmaf(half_of(nz, q), s.inv.z, az)) - s.apad;
-            const float tf = fminf(fminf(fminf(fmaf(half_of(fx, q), s.inv.x, ax),
-                                               fmaf(half_of(fy, q), s.inv.y, ay)),
-                                         fmaf(half_of(fz, q), s.inv.z, az)), tbest);
-            const bool hit = tn <= tf && tf >= tmin;
-            // inner children come first
-            h.e[k] = hit && n.ozn >= (uint32_t)(k + 1) << 20 ? tn : __builtin_huge_valf();
-            h.c[k] = n.inner + k;
-            m |= hit ? 1u << k : 0u;
-        }
+    for (int k = 0; k < 4; ++k) {
+        const int p = k >> 1, q = k & 1;
+        const float tn = fmaxf(fmaxf(fmaf(half_of(b.nx[p], q), s.inv.x, ax), fmaf(half_of(b.ny[p], q), s.inv.y, ay)),
+                               fmaf(half_of(b.nz[p], q), s.inv.z, az)) - s.apad;
+        const float tf = fminf(fminf(fminf(fmaf(half_of(b.fx[p], q), s.inv.x, ax),
+                                           fmaf(half_of(b.fy[p], q), s.inv.y, ay)),
+                                     fmaf(half_of(b.fz[p], q), s.inv.z, az)), tbest);
+        const bool hit = (tn <= tf) & (tf >= tmin);
+        // inner children come first
+        const bool inner = n.ozn >= (uint32_t)(k + 1) << 20;
+        h.e[k] = (hit & inner) ? tn : __builtin_huge_valf();
+        h.c[k] = n.inner + k;
+        m |= hit ? 1u << k : 0u;
     }
     h.leaves = m & (n.ozn >> 16);
+}
+
+// Near and far planes by each lane's direction signs: 12 selects of packed
+// pairs instead of a min and a max per child and axis.
+__device__ __forceinline__ void slab4(const SlabRay& s, const Node4& n, float tmin, float tbest,
+                                      NodeHits& h)
+{
+    NodePlanes b;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        b.nx[p] = pick_pair(s.nx, n.hix[p], n.lox[p]);
+        b.fx[p] = pick_pair(s.nx, n.lox[p], n.hix[p]);
+        b.ny[p] = pick_pair(s.ny, n.hiy[p], n.loy[p]);
+        b.fy[p] = pick_pair(s.ny, n.loy[p], n.hiy[p]);
+        b.nz[p] = pick_pair(s.nz, n.hiz[p], n.loz[p]);
+        b.fz[p] = pick_pair(s.nz, n.loz[p], n.hiz[p]);
+    }
+    slab4(s, n, b, tmin, tbest, h);
 }
 
 // Visits node i: through the scalar cache when every active lane is at it
@@ -439,8 +483,11 @@ __device__ __forceinline__ void fetch_slab4(const Node4* nodes, uint32_t i, cons
 {
     const uint32_t u = __builtin_amdgcn_readfirstlane(i);
     Node4 n;
-    if (__all(i == u)) n = load_node_uniform(nodes, u);
-    else n = load_node<WIDE>(nodes, i);
+    if (__all(i == u)) {
+        n = load_node_uniform(nodes, u);
+    } else {
+        n = load_node<WIDE>(nodes, i);
+    }
     slab4(s, n, tmin, tbest, h);
 }
 
@@ -487,7 +534,7 @@ enum : int {
 // build's) it runs level with slot order or 1% behind.  The pushes below
 // are right for any order (a missed child is written and then overwritten).
 template <int ORDER = kOrderNear>
-__device__ __forceinline__ bool next_node(float e[4], int c[4], const Stack& st, int& sp,
+__device__ __forceinline__ bool next_node(float e[4], int c[4], const Stack& st, lds_u32*& top,
                                           uint32_t& node)
 {
     if (ORDER == kOrderFar) {
@@ -510,37 +557,30 @@ __device__ __forceinline__ bool next_node(float e[4], int c[4], const Stack& st,
         }
     }
     const float inf = __builtin_huge_valf();
-    if (__all(sp + 3 <= st.depth)) {
+    const bool go = e[0] != inf;
+    if (__all((uint32_t)(uintptr_t)top < st.full)) {
         // Every active lane has three free LDS entries (one wave-uniform
-        // test): straight-line pushes with conditional increments.  A write
-        // past the top lands at most where the all-hit case writes, and is
-        // overwritten by the next push or left unused, so the pushes are the
-        // same as below in any order.
-        st.lds[sp * 256] = (uint32_t)c[3];
-        sp += e[3] != inf ? 1 : 0;
-        st.lds[sp * 256] = (uint32_t)c[2];
-        sp += e[2] != inf ? 1 : 0;
-        st.lds[sp * 256] = (uint32_t)c[1];
-        sp += e[1] != inf ? 1 : 0;
-        if (e[0] != inf) {
-            node = (uint32_t)c[0];
-            return true;
-        }
-        if (sp == 0) return false;
-        --sp;
-        node = st.lds[sp * 256];
-        return true;
+        // test): straight-line pushes with conditional increments, and a pop
+        // that every lane reads.  A write past the top lands at most where the
+        // all-hit case writes, and is overwritten by the next push or left
+        // unused, so the pushes are the same as below in any order.
+        *top = (uint32_t)c[3];
+        top += e[3] != inf ? 256 : 0;
+        *top = (uint32_t)c[2];
+        top += e[2] != inf ? 256 : 0;
+        *top = (uint32_t)c[1];
+        top += e[1] != inf ? 256 : 0;
+        const uint32_t below = top[-256];
+        node = go ? (uint32_t)c[0] : below;
+        top -= go ? 0 : 256;
+        return node != kStackEnd;
     }
-    if (e[3] != inf) push(st, sp, (uint32_t)c[3]);
-    if (e[2] != inf) push(st, sp, (uint32_t)c[2]);
-    if (e[1] != inf) push(st, sp, (uint32_t)c[1]);
-    if (e[0] != inf) {
-        node = (uint32_t)c[0];
-        return true;
-    }
-    if (sp == 0) return false;
-    node = pop(st, sp);
-    return true;
+    if (e[3] != inf) push(st, top, (uint32_t)c[3]);
+    if (e[2] != inf) push(st, top, (uint32_t)c[2]);
+    if (e[1] != inf) push(st, top, (uint32_t)c[1]);
+    node = (uint32_t)c[0];
+    if (!go) node = pop(st, top);
+    return node != kStackEnd;
 }
 
 // Closest hit: lexicographic minimum of (t, prim id) over accepted
@@ -559,7 +599,7 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
     const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
     float tbest = tmax, bV = 0.0f, bW = 0.0f, bdet = 1.0f;
     int best = -1;
-    int sp = 0;
+    lds_u32* top = st.lds;
     uint32_t node = 0;
     for (;;) {
         if (COUNT) ++cnt.nodes;
@@ -581,7 +621,7 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
                 bdet = h.det;
             }
         }
-        if (!next_node(n.e, n.c, st, sp, node)) break;
+        if (!next_node(n.e, n.c, st, top, node)) break;
     }
     if (best >= 0) {
         t_out = tbest;
@@ -601,7 +641,7 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
     if (sc.ntris <= 0) return false;
     const WtRay w = wt_setup(o, d);
     const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
-    int sp = 0;
+    lds_u32* top = st.lds;
     uint32_t node = 0;
     for (;;) {
         if (COUNT) ++cnt.nodes;
@@ -612,7 +652,7 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
             WtHit h;
             if (fetch_wt<WIDE>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tmax, h)) return true;
         }
-        if (!next_node<FAR ? kOrderFar : kOrderSlot>(n.e, n.c, st, sp, node)) break;
+        if (!next_node<FAR ? kOrderFar : kOrderSlot>(n.e, n.c, st, top, node)) break;
     }
     return false;
 }

@@ -17,12 +17,8 @@ namespace {
 
 __global__ __launch_bounds__(256) void k_lookup(LookupArgs a)
 {
-    __shared__ uint32_t lds[kLdsDepth * 256];
-    Stack st;
-    st.lds = &lds[threadIdx.x];
-    st.spill = a.spill + (size_t)blockIdx.x * 256 + threadIdx.x;
-    st.spill_stride = a.spill_stride;
-    st.depth = kLdsDepth;
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
+    Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + threadIdx.x, a.spill_stride);
     TraceCount cnt;
     const ProbeGridView& g = a.g;
     const size_t total = (size_t)a.n * 8;

@@ -84,7 +84,7 @@ struct LaneRay {
 };
 
 template <bool ANY>
-__device__ __forceinline__ bool setup_item(const MultiArgs& a, const JobDesc& J, int tb, int pt0,
+__device__ __forceinline__ bool setup_item(const MultiArgs& a, const JobDesc& J, const Stack& st, int tb, int pt0,
                                            size_t it, size_t nslots, LaneRay& R)
 {
     if (!ANY) {
@@ -99,7 +99,7 @@ __device__ __forceinline__ bool setup_item(const MultiArgs& a, const JobDesc& J,
             return false;
         }
         const float4 pp = J.probes[probe];
-        trav_init(R.T, J.sc, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z),
+        trav_init(R.T, J.sc, st, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z),
                   J.tmin, J.tmax);
         R.nodes = J.sc.nodes;
         R.tris = J.sc.tris;
@@ -133,7 +133,7 @@ __device__ __forceinline__ bool setup_item(const MultiArgs& a, const JobDesc& J,
         *vis = 0;
         return false;
     }
-    trav_init(R.T, J.sc, s.org, s.dir, 0.0f, s.dist);
+    trav_init(R.T, J.sc, st, s.org, s.dir, 0.0f, s.dist);
     R.nodes = J.sc.nodes;
     R.tris = J.sc.tris;
     return true;
@@ -144,17 +144,13 @@ __global__ __launch_bounds__(256) void k_rays_jobs(MultiArgs a, const JobDesc* _
                                                    const Segment* __restrict__ seg,
                                                    const WorkHeader* __restrict__ hdr)
 {
-    __shared__ uint32_t lds[kLdsDepthWave * 256];
+    __shared__ uint32_t lds[stack_words(kLdsDepthWave)];
     __shared__ uint32_t qlds[kLeafQueue * 256];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    Stack st;
-    st.lds = &lds[tid];
+    Stack st = make_stack(lds, kLdsDepthWave, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
     LeafQueue q;
     q.lds = &qlds[tid];
-    st.spill = a.spill + (size_t)blockIdx.x * 256 + tid;
-    st.spill_stride = a.spill_stride;
-    st.depth = kLdsDepthWave;
     TraceCount cnt;
     uint32_t ntraced = 0;
 
@@ -223,7 +219,7 @@ __global__ __launch_bounds__(256) void k_rays_jobs(MultiArgs a, const JobDesc* _
                 const bool mine = !act && rank < avail;
                 const size_t take = min((size_t)__popcll(idle), avail);
                 if (mine) {
-                    act = setup_item<ANY>(a, jobs[cj], ctb, cpt0, pnext + rank, nslots, R);
+                    act = setup_item<ANY>(a, jobs[cj], st, ctb, cpt0, pnext + rank, nslots, R);
                     if (act && ANY) ++ntraced;
                 }
                 pnext += take;
@@ -271,14 +267,10 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs
                                                                        const Segment* __restrict__ seg,
                                                                        const WorkHeader* __restrict__ hdr)
 {
-    __shared__ uint32_t lds[kLdsDepth * 256];
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    Stack st;
-    st.lds = &lds[tid];
-    st.spill = a.spill + (size_t)blockIdx.x * 256 + tid;
-    st.spill_stride = a.spill_stride;
-    st.depth = kLdsDepth;
+    Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
     TraceCount cnt;
     uint32_t nshadow = 0;
     const int nseg = hdr->nseg;

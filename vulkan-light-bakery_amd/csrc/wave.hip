@@ -76,7 +76,7 @@ constexpr int kChunk = 256;
 // Sets up item `it` for this lane.  Returns false when the item needs no
 // traversal (its result is written here).
 template <bool ANY, bool CORNERS>
-__device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravState& T, int& slot_out,
+__device__ __forceinline__ bool item_setup(const BakeArgs& a, const Stack& st, size_t it, TravState& T, int& slot_out,
                                            int& light_out)
 {
     if (!ANY) {
@@ -89,7 +89,7 @@ __device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravSta
             return false;
         }
         const float4 pp = a.probes[probe];
-        trav_init(T, a.sc, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z), a.tmin,
+        trav_init(T, a.sc, st, make_float3(pp.x, pp.y, pp.z), make_float3(dd.x, dd.y, dd.z), a.tmin,
                   a.tmax);
         return true;
     }
@@ -117,7 +117,7 @@ __device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravSta
         *vis = 0;
         return false;
     }
-    trav_init(T, a.sc, s.org, s.dir, 0.0f, s.dist);
+    trav_init(T, a.sc, st, s.org, s.dir, 0.0f, s.dist);
     return true;
 }
 
@@ -126,17 +126,13 @@ __device__ __forceinline__ bool item_setup(const BakeArgs& a, size_t it, TravSta
 template <bool ANY, bool COUNT, bool CORNERS>
 __global__ __launch_bounds__(256) void k_rays(BakeArgs a, size_t nitems, unsigned long long* ctr)
 {
-    __shared__ uint32_t lds[kLdsDepthWave * 256];
+    __shared__ uint32_t lds[stack_words(kLdsDepthWave)];
     __shared__ uint32_t qlds[kLeafQueue * 256];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    Stack st;
-    st.lds = &lds[tid];
+    Stack st = make_stack(lds, kLdsDepthWave, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
     LeafQueue q;
     q.lds = &qlds[tid];
-    st.spill = a.spill + (size_t)blockIdx.x * 256 + tid;
-    st.spill_stride = a.spill_stride;
-    st.depth = kLdsDepthWave;
     TraceCount cnt;
     uint32_t ntraced = 0;
     // eight kChunk-aligned ranges of the item space, one per XCD; a wave
@@ -190,7 +186,7 @@ __global__ __launch_bounds__(256) void k_rays(BakeArgs a, size_t nitems, unsigne
                 const bool mine = !act && rank < avail;
                 const size_t take = min((size_t)__popcll(idle), avail);
                 if (mine) {
-                    act = item_setup<ANY, CORNERS>(a, pnext + rank, T, slot, light);
+                    act = item_setup<ANY, CORNERS>(a, st, pnext + rank, T, slot, light);
                     if (act && ANY) ++ntraced;
                 }
                 pnext += take;

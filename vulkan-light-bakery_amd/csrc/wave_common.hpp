@@ -128,12 +128,12 @@ struct TravState {
     int best;   // leaf of the closest hit so far, -1 none (ANY: 0 = hit)
     float bV, bW, bdet;
     uint32_t node;
-    int sp;
+    lds_u32* top;  // stack position
     int nq;     // queued triangles
     bool live;  // `node` is still to be visited
 };
 
-__device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, const float3& o,
+__device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, const Stack& st, const float3& o,
                                           const float3& d, float tmin, float tmax)
 {
     T.w = wt_setup(o, d);
@@ -145,7 +145,7 @@ __device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, con
     T.bW = 0.0f;
     T.bdet = 1.0f;
     T.node = 0;
-    T.sp = 0;
+    T.top = st.lds;
     T.nq = 0;
     T.live = true;
 }
@@ -166,7 +166,7 @@ __device__ __forceinline__ void visit_node(TravState& T, const Node4* nodes, con
         q.lds[T.nq * 256] = (uint32_t)(n.leaf + k);
         T.nq += (int)((n.leaves >> k) & 1u);
     }
-    T.live = next_node<ANY ? kOrderSlot : kOrderNear>(n.e, n.c, st, T.sp, T.node);
+    T.live = next_node<ANY ? kOrderSlot : kOrderNear>(n.e, n.c, st, T.top, T.node);
 }
 
 // Tests every queued triangle of the active lanes (the wave runs as many
