@@ -143,6 +143,12 @@ __device__ __forceinline__ WtRay wt_setup(const float3& o, const float3& d)
     return w;
 }
 
+// A ray with a direction component below 2^-16 of its largest (box_agrees).
+__device__ __forceinline__ bool wt_thin(const WtRay& w)
+{
+    return fminf(fabsf(w.Sx), fabsf(w.Sy)) < 0x1p-16f;
+}
+
 // Edge-function part of the test.  On acceptance returns t (correctly
 // rounded T / det) with the numerators V, W and det kept for the
 // barycentrics, which are divided out once for the final hit only.
@@ -212,7 +218,8 @@ __host__ __device__ __forceinline__ float box_margin(float maxabs)
     return maxabs * (64.0f * 1.1920929e-7f);
 }
 
-__device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, float maxabs, float unit)
+__device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, bool thin, float maxabs,
+                                              float unit)
 {
     SlabRay s;
     // a component this small moves the ray by less than the margin over the
@@ -221,9 +228,11 @@ __device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, 
     const float dx = fabsf(d.x) < dmin ? copysignf(dmin, d.x) : d.x;
     const float dy = fabsf(d.y) < dmin ? copysignf(dmin, d.y) : d.y;
     const float dz = fabsf(d.z) < dmin ? copysignf(dmin, d.z) : d.z;
-    // hardware reciprocals (1 ulp, far inside the margin): 30 instructions
-    // fewer per ray than correctly rounded divides
-    const float3 r = make_float3(__builtin_amdgcn_rcpf(dx), __builtin_amdgcn_rcpf(dy), __builtin_amdgcn_rcpf(dz));
+    // hardware reciprocals (1 ulp, far inside the margin; 30 instructions fewer
+    // than correctly rounded ones), but exact for the waves with a thin ray,
+    // where box_agrees looks at their last bit
+    float3 r = make_float3(__builtin_amdgcn_rcpf(dx), __builtin_amdgcn_rcpf(dy), __builtin_amdgcn_rcpf(dz));
+    if (__any(thin)) r = make_float3(1.0f / dx, 1.0f / dy, 1.0f / dz);
     s.oinv = make_float3(o.x * r.x, o.y * r.y, o.z * r.z);
     s.inv = make_float3(unit * r.x, unit * r.y, unit * r.z);
     s.nx = dx < 0.0f;
@@ -385,18 +394,56 @@ __device__ __forceinline__ Node4 load_node_uniform(const Node4* nodes, uint32_t 
     return n;
 }
 
+// Whether the slab test of a triangle's own box, on its exact bounds, agrees
+// that the ray meets it before tbest.  Asked for accepted triangles of thin
+// rays: a ray that runs in the plane of an axis-aligned triangle (a probe on a
+// wall) has a determinant of rounding errors only, and whether such a hit
+// counts has always been decided by the box of the triangle; a widened box
+// does not decide it.  All other rays meet the exact box of any triangle they
+// are accepted by.
+__device__ __forceinline__ void box_axis(const char* p, float per_unit, float inv, float oinv, float& tn,
+                                         float& tf)
+{
+    // one axis at a time: the check is rare, its registers are not
+    __asm__ __volatile__("" ::: "memory");
+    const float a = *reinterpret_cast<const float*>(p), b = *reinterpret_cast<const float*>(p + 20),
+                c = *reinterpret_cast<const float*>(p + 40);
+    const float t0 = fmaf(fminf(a, fminf(b, c)) * per_unit, inv, -oinv);
+    const float t1 = fmaf(fmaxf(a, fmaxf(b, c)) * per_unit, inv, -oinv);
+    tn = fmaxf(tn, fminf(t0, t1));
+    tf = fminf(tf, fmaxf(t0, t1));
+}
+
+template <bool WIDE>
+__device__ __forceinline__ bool box_agrees(const float* tris, float unit, int leaf, const WtRay& w,
+                                           const SlabRay& s, float tmin, float tbest)
+{
+    if (!wt_thin(w)) return true;
+    __asm__ __volatile__("" : "+v"(unit));  // nothing of this block before the loop
+    const float per_unit = 1.0f / unit;     // exact: a power of two
+    const char* p = record64<WIDE>(tris, (uint32_t)leaf, 0);
+    float tn = -__builtin_huge_valf(), tf = __builtin_huge_valf();
+    box_axis(p, per_unit, s.inv.x, s.oinv.x, tn, tf);
+    box_axis(p + 4, per_unit, s.inv.y, s.oinv.y, tn, tf);
+    box_axis(p + 8, per_unit, s.inv.z, s.oinv.z, tn, tf);
+    float hi = fminf(tf, tbest);
+    hi = fmaf(fabsf(hi), 4e-6f, hi) + s.apad;
+    const float lo = fmaf(-fabsf(tn), 4e-6f, tn) - s.apad;
+    return lo <= hi && hi >= tmin;
+}
+
 // Watertight test of triangle `leaf`.  Always through the vector path: a
 // record that every active lane reads in the same order could come through
 // the scalar cache, but the compare, the branch and the scalar registers cost
 // more than the three 12-byte loads (24-job batch 72.5 ms with the scalar
 // form, 71.0 without; 11k-triangle room plan 0.974 against 0.923 ms).
 template <bool WIDE>
-__device__ __forceinline__ bool fetch_wt(const float* tris, int leaf, const WtRay& w, float tmin,
-                                         float tmax, WtHit& h)
+__device__ __forceinline__ bool fetch_wt(const float* tris, float unit, int leaf, const WtRay& w,
+                                         const SlabRay& s, float tmin, float tmax, WtHit& h)
 {
     float3 v0, v1, v2;
     load_tri<WIDE>(tris, leaf, w, v0, v1, v2);
-    return wt_test(w, v0, v1, v2, tmin, tmax, h);
+    return wt_test(w, v0, v1, v2, tmin, tmax, h) && box_agrees<WIDE>(tris, unit, leaf, w, s, tmin, tmax);
 }
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
@@ -596,7 +643,7 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
 {
     if (sc.ntris <= 0) return -1;
     const WtRay w = wt_setup(o, d);
-    const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
+    const SlabRay s = slab_setup(o, d, wt_thin(w), sc.maxabs, sc.unit);
     float tbest = tmax, bV = 0.0f, bW = 0.0f, bdet = 1.0f;
     int best = -1;
     lds_u32* top = st.lds;
@@ -612,7 +659,7 @@ __device__ int trace_closest(const SceneView& sc, const float3& o, const float3&
             const int leaf = n.leaf + __builtin_ctz(leaves);
             WtHit h;
             // t <= tbest holds on acceptance; an equal t keeps the lower prim id
-            if (fetch_wt<WIDE>(sc.tris, leaf, w, tmin, tbest, h) &&
+            if (fetch_wt<WIDE>(sc.tris, sc.unit, leaf, w, s, tmin, tbest, h) &&
                 (best < 0 || h.t < tbest || tri_prim(sc.tris, leaf) < tri_prim(sc.tris, best))) {
                 tbest = h.t;
                 best = leaf;
@@ -640,7 +687,7 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
 {
     if (sc.ntris <= 0) return false;
     const WtRay w = wt_setup(o, d);
-    const SlabRay s = slab_setup(o, d, sc.maxabs, sc.unit);
+    const SlabRay s = slab_setup(o, d, wt_thin(w), sc.maxabs, sc.unit);
     lds_u32* top = st.lds;
     uint32_t node = 0;
     for (;;) {
@@ -650,7 +697,7 @@ __device__ bool trace_any(const SceneView& sc, const float3& o, const float3& d,
         for (uint32_t leaves = n.leaves; leaves != 0; leaves &= leaves - 1) {
             if (COUNT) ++cnt.tris;
             WtHit h;
-            if (fetch_wt<WIDE>(sc.tris, n.leaf + __builtin_ctz(leaves), w, tmin, tmax, h)) return true;
+            if (fetch_wt<WIDE>(sc.tris, sc.unit, n.leaf + __builtin_ctz(leaves), w, s, tmin, tmax, h)) return true;
         }
         if (!next_node<FAR ? kOrderFar : kOrderSlot>(n.e, n.c, st, top, node)) break;
     }

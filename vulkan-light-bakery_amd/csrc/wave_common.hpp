@@ -124,7 +124,7 @@ struct LeafQueue {
 struct TravState {
     WtRay w;
     SlabRay s;
-    float tmin, tb;
+    float tmin, tb, unit;
     int best;   // leaf of the closest hit so far, -1 none (ANY: 0 = hit)
     float bV, bW, bdet;
     uint32_t node;
@@ -137,8 +137,9 @@ __device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, con
                                           const float3& d, float tmin, float tmax)
 {
     T.w = wt_setup(o, d);
-    T.s = slab_setup(o, d, sc.maxabs, sc.unit);
+    T.s = slab_setup(o, d, wt_thin(T.w), sc.maxabs, sc.unit);
     T.tmin = tmin;
+    T.unit = sc.unit;
     T.tb = tmax;
     T.best = -1;
     T.bV = 0.0f;
@@ -177,14 +178,12 @@ __device__ __forceinline__ void test_queue(TravState& T, const float* tris, cons
 {
     for (int i = 0; __any(i < T.nq); ++i) {
         if (i < T.nq && !(ANY && T.best == 0)) {
-            float3 v0, v1, v2;
             const int leaf = (int)q.lds[i * 256];
-            load_tri<true>(tris, leaf, T.w, v0, v1, v2);
             if (COUNT) ++cnt.tris;
             WtHit h;
             if (ANY) {
-                if (wt_test(T.w, v0, v1, v2, T.tmin, T.tb, h)) T.best = 0;
-            } else if (wt_test(T.w, v0, v1, v2, T.tmin, T.tb, h) &&
+                if (fetch_wt<true>(tris, T.unit, leaf, T.w, T.s, T.tmin, T.tb, h)) T.best = 0;
+            } else if (fetch_wt<true>(tris, T.unit, leaf, T.w, T.s, T.tmin, T.tb, h) &&
                        (T.best < 0 || h.t < T.tb || tri_prim(tris, leaf) < tri_prim(tris, T.best))) {
                 // t <= tbest holds on acceptance; an equal t keeps the lower prim id
                 T.tb = h.t;
