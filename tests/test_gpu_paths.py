@@ -80,3 +80,71 @@ def test_small_trees_at_extreme_scales(ctx, ntris, scale):
     occ = ctx.trace_occluded(sid, org, d, tmax, 0.0)
     assert np.array_equal(occ, o.trace_occluded(org, d, np.full(n, tmax, np.float32), 0.0))
     ctx.release_scene(sid)
+
+
+def test_probes_on_walls_agree_across_kernels(ctx, room):
+    """Rays that run in the plane of a wall (probes on the scene bounds, an
+    equirect grid with columns along the axes): the check that decides those
+    hits gives the same bits in every kernel family, with point queries on the
+    same rays in agreement."""
+    s, sid, o = room
+    probes, _ = vlb.probe_grid([0, 0, 0], [10, 4, 10], [3, 2, 3], vlb.ORDER_REFERENCE_BFS)
+    p = vlb.Params(probes=probes, dir_mode=vlb.DIRS_EQUIRECT, equirect_w=157, equirect_h=50, sh_order=3,
+                   sh_constants=vlb.SH_LITERAL, shade_mode=vlb.SHADE_REFERENCE)
+    ref = None
+    for v in (12, 4, 16, 20, 36):
+        p.trace_variant = v
+        got = ctx.bake(sid, p)
+        ref = got if ref is None else ref
+        assert np.array_equal(_bits(got), _bits(ref)), v
+    p.trace_variant = 0
+    _, hits = ctx.bake_radiance(sid, p, want_radiance=False)
+    xyz, _ = vlb.directions(p.dir_mode, 0, 157, 50)
+    for i in (0, 5, 17):
+        prim = ctx.trace_closest(sid, np.repeat(probes[i:i + 1], len(xyz), 0), xyz)[0]
+        assert np.array_equal(prim, hits[i])
+
+
+@pytest.mark.parametrize("mode,n", [("fib", 1), ("fib", 63), ("fib", 1000), ("fib", 16384), ("eq", (7, 3)),
+                                    ("eq", (64, 32)), ("eq", (157, 50))])
+@pytest.mark.parametrize("prec", [vlb.PREC_FP32, vlb.PREC_BF16, vlb.PREC_FP16])
+def test_device_ray_tables_project_like_the_oracle(ctx, mode, n, prec):
+    """The direction and basis tables built on the device, through a sky-only
+    bake: every ray's radiance is a function of its direction (so a wrong
+    direction, order or weight shows), and the coefficients are the FP64
+    oracle's within the bar of the precision (1e-5, split 16-bit forms 1e-4)."""
+    sid = ctx.upload_scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32))
+    o = orc.Scene(np.zeros((0, 3)), np.zeros((0, 3), np.uint32))
+    probes = np.zeros((3, 3), np.float32)
+    sun = vlb.sun_direction(np.random.default_rng(3)).tolist()
+    if mode == "fib":
+        p = vlb.Params(probes=probes, rays=n, sun_dir=sun, precision=prec, sh_order=3)
+    else:
+        p = vlb.Params(probes=probes, dir_mode=vlb.DIRS_EQUIRECT, equirect_w=n[0], equirect_h=n[1],
+                       sun_dir=sun, precision=prec, sh_order=3, sh_constants=vlb.SH_LITERAL)
+    rad, hit = ctx.bake_radiance(sid, p)
+    assert (hit == -1).all()
+    xyz, _ = vlb.directions(p.dir_mode, p.rays, p.equirect_w, p.equirect_h)
+    d = xyz.astype(np.float64)
+    want = 0.5 + 1.5 * np.maximum(d[:, 1], 0.0) + 50.0 * np.exp(200.0 * (d @ np.asarray(sun) - 1.0))
+    np.testing.assert_allclose(rad[0, :, 0], want, rtol=3e-5)
+    got = ctx.bake(sid, p)
+    ref = o.bake(p, mode64=True)["coeffs"]
+    assert rel_err(got, ref).max() <= (1e-5 if prec == vlb.PREC_FP32 else 1e-4)
+    ctx.release_scene(sid)
+
+
+@pytest.mark.parametrize("P", [1, 15, 16, 17, 1000, 20000])
+def test_device_probe_order_keeps_every_probe(ctx, room, P):
+    """Probes sorted on the device come back in the caller's order: each
+    probe's coefficients are those of a bake of that probe alone."""
+    s, sid, o = room
+    rng = np.random.default_rng(P)
+    probes = rng.uniform([1, 0.5, 1], [9, 3.5, 9], (P, 3)).astype(np.float32)
+    if P > 16:
+        probes[5:9] = probes[4]                        # equal keys: a stable order
+    p = vlb.Params(probes=probes, rays=64, lights=[(vlb.LIGHT_DIRECTIONAL, (0.0, -1.0, 0.0), (3.0, 3.0, 3.0))])
+    got = ctx.bake(sid, p)
+    for i in rng.integers(0, P, 4):
+        p.probes = probes[i:i + 1]
+        assert rel_err(ctx.bake(sid, p), got[i:i + 1]).max() <= 1e-6

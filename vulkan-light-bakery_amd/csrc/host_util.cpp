@@ -1,9 +1,11 @@
 // host_util.cpp -- host helpers of the C ABI: direction sets, probe grid,
-// double-precision SH basis, base64.
+// SH constants, base64.
 #include <math.h>
 #include <string.h>
 
 #include <vector>
+
+#include <hip/hip_runtime.h>
 
 #include "../../include/vlb_bake.h"
 
@@ -25,75 +27,60 @@ void fibonacci_dirs(uint32_t R, float* xyz)
     }
 }
 
-// shaders/env_map.rgen:21 with sh_common.h:8-22 (float, PI = 3.1415926538f),
-// weight of shaders/sh.comp:32-33.
-void equirect_dirs(uint32_t W, uint32_t H, float* xyz, float* weight)
+// Angles of an equirect grid, shaders/env_map.rgen:21 with sh_common.h:8-22
+// (float, PI = 3.1415926538f): tab[x] = (cos, sin) of column x's phi, tab[W +
+// y] = (sin, cos) of row y's theta; weight[y] as shaders/sh.comp:32-33.
+void equirect_angles(uint32_t W, uint32_t H, float2* tab, float* weight)
 {
     const float PI = 3.1415926538f;
     const float area = (2.0f * PI / (float)W) * (PI / (float)H);
+    for (uint32_t x = 0; x < W; ++x) {
+        const float phi = 2.f * PI * ((float)x + 0.5f) / (float)W;
+        tab[x] = make_float2(cosf(phi), sinf(phi));
+    }
     for (uint32_t y = 0; y < H; ++y) {
         const float theta = PI * ((float)y + 0.5f) / (float)H;
-        const float wgt = area * sinf(theta);
+        tab[W + y] = make_float2(sinf(theta), cosf(theta));
+        weight[y] = area * sinf(theta);
+    }
+}
+
+void equirect_dirs(uint32_t W, uint32_t H, float* xyz, float* weight)
+{
+    std::vector<float2> tab((size_t)W + H);
+    std::vector<float> wrow(H);
+    equirect_angles(W, H, tab.data(), wrow.data());
+    for (uint32_t y = 0; y < H; ++y)
         for (uint32_t x = 0; x < W; ++x) {
-            const float phi = 2.f * PI * ((float)x + 0.5f) / (float)W;
-            const float r = sinf(theta);
-            const float a = r * cosf(phi), b = r * sinf(phi), c = cosf(theta);
+            const float2 cp = tab[x], st = tab[W + y];
+            const float a = st.x * cp.x, b = st.x * cp.y, c = st.y;
             const float l = sqrtf(a * a + b * b + c * c);
             const size_t i = (size_t)y * W + x;
             xyz[3 * i + 0] = a / l;
             xyz[3 * i + 1] = c / l;
             xyz[3 * i + 2] = b / l;
-            if (weight) weight[i] = wgt;
+            if (weight) weight[i] = wrow[y];
         }
-    }
 }
 
-// Real SH basis of shaders/sh_common.h:26-152 (l <= 3 here), double.
-void sh_eval_double(int K, bool exact, const double d[3], double* out)
+// Constants of the real SH basis of shaders/sh_common.h:26-152 (l <= 3), in
+// the order of the basis table's terms: closed forms, or the shader's six
+// digits.
+void sh_constants(bool exact, double c[10])
 {
-    const double x = d[0], y = d[1], z = d[2];
-    double c0, c1, c2a, c20, c22, c33, c32, c31, c30, c3p2;
-    if (exact) {
-        c0 = 0.5 * sqrt(1.0 / kPi);
-        c1 = sqrt(3.0 / (4.0 * kPi));
-        c2a = 0.5 * sqrt(15.0 / kPi);
-        c20 = 0.25 * sqrt(5.0 / kPi);
-        c22 = 0.25 * sqrt(15.0 / kPi);
-        c33 = 0.25 * sqrt(35.0 / (2.0 * kPi));
-        c32 = 0.5 * sqrt(105.0 / kPi);
-        c31 = 0.25 * sqrt(21.0 / (2.0 * kPi));
-        c30 = 0.25 * sqrt(7.0 / kPi);
-        c3p2 = 0.25 * sqrt(105.0 / kPi);
-    } else {
-        c0 = 0.282095;
-        c1 = 0.488603;
-        c2a = 1.092548;
-        c20 = 0.315392;
-        c22 = 0.546274;
-        c33 = 0.590044;
-        c32 = 2.890611;
-        c31 = 0.457046;
-        c30 = 0.373176;
-        c3p2 = 1.445306;
-    }
-    double v[16];
-    v[0] = c0;
-    v[1] = -c1 * y;
-    v[2] = c1 * z;
-    v[3] = -c1 * x;
-    v[4] = c2a * x * y;
-    v[5] = -c2a * y * z;
-    v[6] = c20 * (-x * x - y * y + 2.0 * z * z);
-    v[7] = -c2a * x * z;
-    v[8] = c22 * (x * x - y * y);
-    v[9] = -c33 * y * (3.0 * x * x - y * y);
-    v[10] = c32 * x * y * z;
-    v[11] = -c31 * y * (4.0 * z * z - x * x - y * y);
-    v[12] = c30 * z * (2.0 * z * z - 3.0 * x * x - 3.0 * y * y);
-    v[13] = -c31 * x * (4.0 * z * z - x * x - y * y);
-    v[14] = c3p2 * z * (x * x - y * y);
-    v[15] = -c33 * x * (x * x - 3.0 * y * y);
-    for (int k = 0; k < K && k < 16; ++k) out[k] = v[k];
+    const double lit[10] = {0.282095, 0.488603, 1.092548, 0.315392, 0.546274,
+                            0.590044, 2.890611, 0.457046, 0.373176, 1.445306};
+    const double ex[10] = {0.5 * sqrt(1.0 / kPi),
+                           sqrt(3.0 / (4.0 * kPi)),
+                           0.5 * sqrt(15.0 / kPi),
+                           0.25 * sqrt(5.0 / kPi),
+                           0.25 * sqrt(15.0 / kPi),
+                           0.25 * sqrt(35.0 / (2.0 * kPi)),
+                           0.5 * sqrt(105.0 / kPi),
+                           0.25 * sqrt(21.0 / (2.0 * kPi)),
+                           0.25 * sqrt(7.0 / kPi),
+                           0.25 * sqrt(105.0 / kPi)};
+    for (int i = 0; i < 10; ++i) c[i] = exact ? ex[i] : lit[i];
 }
 
 }  // namespace vlb

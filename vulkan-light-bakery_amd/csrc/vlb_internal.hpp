@@ -237,7 +237,6 @@ void build_probe_set(Context& ctx, const float* xyz, uint32_t P, ProbeSet& s);
 ShadeParams shade_params(const vlb_bake_params& p);
 size_t scene_spill_bytes(const Scene& s, uint32_t stride);
 std::vector<uint32_t> morton_order(const float* xyz, size_t n);
-std::vector<uint32_t> direction_order(const float* xyz, size_t n);
 
 // ------------------------------------------------------------ bake plan
 struct BakeArgs {
@@ -454,7 +453,8 @@ void launch_read(const void* src, size_t bytes, int grid, hipStream_t st);
 // host_util.cpp
 void fibonacci_dirs(uint32_t R, float* xyz);
 void equirect_dirs(uint32_t W, uint32_t H, float* xyz, float* weight);
-void sh_eval_double(int K, bool exact, const double d[3], double* out);
+void equirect_angles(uint32_t W, uint32_t H, float2* tab, float* weight);
+void sh_constants(bool exact, double c[10]);
 void geometric_normal(const float* v0, const float* v1, const float* v2, float g[3]);
 
 }  // namespace vlb
