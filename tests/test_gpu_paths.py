@@ -1,5 +1,7 @@
 """GPU tests of the launch paths picked by size or option: each path against
 the same work on the path it stands in for, or against the oracle."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -148,3 +150,53 @@ def test_device_probe_order_keeps_every_probe(ctx, room, P):
     for i in rng.integers(0, P, 4):
         p.probes = probes[i:i + 1]
         assert rel_err(ctx.bake(sid, p), got[i:i + 1]).max() <= 1e-6
+
+
+def _mixed_calls(c, sid, probes):
+    """One-shot calls of different buffer sizes: their results in a fixed order."""
+    sun = [(vlb.LIGHT_DIRECTIONAL, (0.2, -1.0, 0.1), (3.0, 3.0, 3.0))]
+    rng = np.random.default_rng(len(probes))
+    res = []
+    for rays, order in ((48, 2), (700, 3), (129, 2)):
+        res.append(c.bake(sid, vlb.Params(probes=probes, rays=rays, sh_order=order, lights=sun)))
+    d = rng.normal(size=(777, 3)).astype(np.float32)
+    o = np.tile(probes[:1], (777, 1))
+    res += list(c.trace_closest(sid, o, d))
+    res.append(c.project_equirect(rng.integers(0, 256, (40, 80, 4), dtype=np.uint8)))
+    return res
+
+
+@pytest.mark.parametrize("budget", [0, 64 << 20])
+def test_reused_device_blocks_hold_nothing_over(budget):
+    """Calls whose buffers are blocks freed by other calls (larger, smaller,
+    from two threads at once; with a budget that some of the kept blocks have
+    to make room for) return what the first call on a fresh context returns."""
+    s = vlb.generate_scene(vlb.SCENE_ROOM, 2)
+    rng = np.random.default_rng(5)
+    sets = [rng.uniform([1, 0.5, 1], [9, 3.5, 9], (n, 3)).astype(np.float32) for n in (300, 37)]
+    want = []
+    for p in sets:
+        with vlb.Context() as c:
+            want.append(_mixed_calls(c, c.upload_scene_dict(s), p))
+    with vlb.Context(hbm_budget=budget) as c:
+        sid = c.upload_scene_dict(s)
+        errors = []
+
+        def work(k):
+            try:
+                for _ in range(3):
+                    got = _mixed_calls(c, sid, sets[k])
+                    assert all(np.array_equal(a, b) for a, b in zip(got, want[k]))
+            except BaseException as e:  # reported by the main thread
+                errors.append(e)
+
+        ts = [threading.Thread(target=work, args=(k,)) for k in (0, 1)]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        assert not errors, errors
+        c.release_scene(sid)
+        again = c.upload_scene_dict(s)  # a scene built in kept blocks
+        got = _mixed_calls(c, again, sets[0])
+        assert all(np.array_equal(a, b) for a, b in zip(got, want[0]))

@@ -17,7 +17,7 @@ using namespace vlb;
 
 namespace vlb {
 
-DevBuf dev_alloc(Context& ctx, size_t bytes)
+DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
 {
     if (bytes == 0) bytes = 16;
     const uint64_t now = ctx.in_use.load();
@@ -27,13 +27,30 @@ DevBuf dev_alloc(Context& ctx, size_t bytes)
                                         std::to_string(now) + " of " + std::to_string(ctx.budget) +
                                         " in use)"};
     DevBuf b;
-    hipError_t e = hipMalloc(&b.p, bytes);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        throw Error{VLB_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e)};
+    // capacities in steps of 1/16 (4 KiB at least, 2 MiB from 64 MiB on), so
+    // that blocks fit the next call of about the same size
+    size_t step = 4096;
+    while (step * 16 < bytes && step < (2u << 20)) step *= 2;
+    b.cap = (bytes + step - 1) / step * step;
+    if (pooled) b.p = ctx.pool.take(bytes, b.cap);
+    if (!b.p) {
+        if (ctx.budget && now + ctx.pool.kept() + b.cap > ctx.budget) ctx.pool.trim();
+        hipError_t e = hipMalloc(&b.p, b.cap);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            ctx.pool.trim();
+            b.cap = bytes;
+            e = hipMalloc(&b.p, b.cap);
+        }
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            b.p = nullptr;
+            throw Error{VLB_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e)};
+        }
     }
     b.bytes = bytes;
     b.acct = &ctx.in_use;
+    b.pool = pooled ? &ctx.pool : nullptr;
     ctx.in_use.fetch_add(bytes);
     return b;
 }
@@ -267,7 +284,6 @@ void build_plan(Context& ctx, Scene& sc, const vlb_bake_params& p, Plan& pl)
     apply_variant(ctx, pl, tv);
     pl.stats.rays_per_slice = pl.rt.RS;
     pl.stats.slices = (uint32_t)nslices;
-    VLB_HIP(hipStreamSynchronize(ctx.stream));
 }
 
 void plan_sync(Plan& pl);
@@ -419,6 +435,7 @@ vlb_status vlb_ctx_create(int32_t device, uint64_t hbm_budget_bytes, vlb_ctx** o
         size_t freeb = 0, total = 0;
         VLB_HIP(hipMemGetInfo(&freeb, &total));
         c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)freeb;
+        c->pool.set_limit(total / kPoolShare);
         VLB_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         for (auto& e : c->ev) VLB_HIP(hipEventCreate(&e));
         c->sky_scratch = skybox_scratch_init(device);
@@ -642,6 +659,7 @@ vlb_status vlb_plan_create(vlb_ctx* h, uint32_t scene, const vlb_bake_params* p,
         VLB_HIP(hipSetDevice(c->device));
         auto pl = std::make_unique<Plan>();
         build_plan(*c, s, *p, *pl);
+        VLB_HIP(hipStreamSynchronize(c->stream));  // the caller's probes are read
         *out = reinterpret_cast<vlb_plan*>(pl.release());
         ++s.users;
         ++c->children;
@@ -916,6 +934,7 @@ static void ensure_wtab(Context& c, int N)
     if (c.wtab_n == N && c.wtab.p) return;
     std::vector<float> w = solid_angle_table(N);
     c.wtab = upload_vec(c, w);
+    VLB_HIP(hipStreamSynchronize(c.stream));  // w is read
     c.sky_tab.release();
     const size_t tab_bytes = (size_t)6 * N * N * sizeof(float4);
     if (tab_bytes <= (2u << 20)) {
@@ -1133,7 +1152,8 @@ vlb_status vlb_device_alloc(vlb_ctx* h, size_t bytes, void** dptr)
     std::lock_guard<std::recursive_mutex> lk(c->mtx);
     return guard(c, [&] {
         VLB_HIP(hipSetDevice(c->device));
-        DevBuf b = dev_alloc(*c, bytes);
+        // the caller may use it on streams of its own: not from the pool
+        DevBuf b = dev_alloc(*c, bytes, false);
         *dptr = b.p;
         c->user_bufs[b.p] = std::move(b);
     });

@@ -333,6 +333,7 @@ void build_ray_table(Context& ctx, const vlb_bake_params& p, int K, uint32_t RS,
         k_dirs_equirect<<<blocks(R), 256, 0, st>>>(W, R, trig.as<float2>(), trig.as<float2>() + W,
                                                    xyz.as<float>(), s.key.as<uint32_t>(),
                                                    s.val.as<uint32_t>());
+        VLB_HIP(hipStreamSynchronize(st));  // tab and wrow are read
     }
     VLB_HIP(hipGetLastError());
     s.sort(R, 32, st);
@@ -353,8 +354,6 @@ void build_ray_table(Context& ctx, const vlb_bake_params& p, int K, uint32_t RS,
                                              xyz.as<float>(), s.val2.as<uint32_t>(), t.dirs.as<float4>(),
                                              t.dir_perm.as<int>(), t.ytab.p);
     VLB_HIP(hipGetLastError());
-    // the scratch is freed on return
-    VLB_HIP(hipStreamSynchronize(st));
 }
 
 void build_probe_set(Context& ctx, const float* xyz, uint32_t P, ProbeSet& s)
@@ -378,7 +377,6 @@ void build_probe_set(Context& ctx, const float* xyz, uint32_t P, ProbeSet& s)
     k_probe_rows<<<blocks(Ppad), 256, 0, st>>>(raw.as<float>(), P, Ppad, sb.val2.as<uint32_t>(),
                                                s.probes.as<float4>(), s.probe_perm.as<int>());
     VLB_HIP(hipGetLastError());
-    VLB_HIP(hipStreamSynchronize(st));
 }
 
 }  // namespace vlb

@@ -677,6 +677,8 @@ vlb_status vlb_server_create(vlb_ctx* h, const vlb_server_options* o, vlb_server
         s->jobtab.assign(op.max_active, JobDesc{});
         for (int i = (int)op.max_active - 1; i >= 0; --i) s->free_slots.push_back(i);
         s->rb.alloc(*c, s->cap_tiles, (int)op.max_lights, op.max_depth);
+        // blocks from the pool may still be in use on the context's stream
+        VLB_HIP(hipStreamSynchronize(c->stream));
         s->t0 = std::chrono::steady_clock::now();
         s->thr = std::thread([s] { s->run(); });
     });

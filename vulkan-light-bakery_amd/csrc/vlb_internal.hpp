@@ -5,10 +5,12 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/vlb_bake.h"
@@ -36,50 +38,121 @@ struct Error {
     } while (0)
 
 // --------------------------------------------------------- device buffers
+// Freed device blocks of a context, kept for its next allocations: a one-shot
+// call makes and drops a dozen buffers, and hipMalloc/hipFree of them cost
+// 0.3-0.5 ms per call, 20 ms and more with a radiance buffer of gigabytes.
+// Bounded (kPoolShare of the device's memory), emptied when an allocation
+// would not fit the context's budget or the device, and with the context.
+//
+// A block may come back while kernels on the context's stream still use it;
+// later work on that stream is ordered behind them.  Work on any other stream
+// (the server's, the user's) first waits for the context's stream
+// (vlb_server_create, Server::admit_one) or has its blocks outside the pool
+// (vlb_device_alloc); every release of a block used on another stream follows
+// a wait for that stream.  While an exception unwinds, blocks are freed, which
+// waits for the device.
+class DevPool {
+public:
+    ~DevPool() { trim(); }
+    void set_limit(size_t bytes) { limit_ = bytes; }
+    // The smallest kept block of at least `bytes` and little more, or null.
+    void* take(size_t bytes, size_t& cap)
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        auto it = free_.lower_bound(bytes);
+        if (it == free_.end() || it->first > bytes + bytes / 4 + (64u << 10)) return nullptr;
+        void* p = it->second;
+        cap = it->first;
+        kept_ -= cap;
+        free_.erase(it);
+        return p;
+    }
+    void put(void* p, size_t cap) noexcept
+    {
+        if (cap <= limit_) {
+            if (kept() + cap > limit_) trim();
+            try {
+                std::lock_guard<std::mutex> lk(mu_);
+                if (kept_ + cap <= limit_) {
+                    free_.emplace(cap, p);
+                    kept_ += cap;
+                    return;
+                }
+            } catch (...) {  // no host memory for the entry
+            }
+        }
+        (void)hipFree(p);
+    }
+    void trim()
+    {
+        std::multimap<size_t, void*> drop;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            drop.swap(free_);
+            kept_ = 0;
+        }
+        for (auto& kv : drop) (void)hipFree(kv.second);
+    }
+    size_t kept()
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        return kept_;
+    }
+
+private:
+    std::mutex mu_;
+    std::multimap<size_t, void*> free_;  // capacity -> block
+    size_t kept_ = 0, limit_ = 0;
+};
+constexpr size_t kPoolShare = 32;  // of the device's memory: 9 of 288 GB
+
 // Device allocation owned by RAII; `acct` is the owning context's byte
-// counter (HBM budget admission).
+// counter (HBM budget admission), `pool` where the block goes back (null:
+// freed).
 struct DevBuf {
     void* p = nullptr;
-    size_t bytes = 0;
+    size_t bytes = 0, cap = 0;
     std::atomic<uint64_t>* acct = nullptr;
+    DevPool* pool = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), acct(o.acct)
-    {
-        o.p = nullptr;
-        o.bytes = 0;
-        o.acct = nullptr;
-    }
+    DevBuf(DevBuf&& o) noexcept { swap(o); }
     DevBuf& operator=(DevBuf&& o) noexcept
     {
         if (this != &o) {
             release();
-            p = o.p;
-            bytes = o.bytes;
-            acct = o.acct;
-            o.p = nullptr;
-            o.bytes = 0;
-            o.acct = nullptr;
+            swap(o);
         }
         return *this;
     }
     ~DevBuf() { release(); }
+    void swap(DevBuf& o) noexcept
+    {
+        std::swap(p, o.p);
+        std::swap(bytes, o.bytes);
+        std::swap(cap, o.cap);
+        std::swap(acct, o.acct);
+        std::swap(pool, o.pool);
+    }
     void release()
     {
         if (p) {
-            (void)hipFree(p);
+            if (pool && std::uncaught_exceptions() == 0) pool->put(p, cap);
+            else (void)hipFree(p);
             if (acct) acct->fetch_sub(bytes);
         }
         p = nullptr;
-        bytes = 0;
+        bytes = cap = 0;
         acct = nullptr;
+        pool = nullptr;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
 struct Context;
-DevBuf dev_alloc(Context& ctx, size_t bytes);
+// `pooled` false: a block of its own, freed on release (see DevPool).
+DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled = true);
 
 // ------------------------------------------------------------------ scene
 struct Scene {
@@ -120,6 +193,7 @@ struct Context {
     hipStream_t stream = nullptr;
     uint64_t budget = 0;                  // bytes
     std::atomic<uint64_t> in_use{0};      // bytes allocated through dev_alloc
+    DevPool pool;                         // before every member that holds blocks
     // message of the last failure on this context, from any thread (the
     // serving entry points may fail concurrently): written and copied out
     // under err_mu only (set_error / get_error)
