@@ -200,3 +200,72 @@ def test_reused_device_blocks_hold_nothing_over(budget):
         again = c.upload_scene_dict(s)  # a scene built in kept blocks
         got = _mixed_calls(c, again, sets[0])
         assert all(np.array_equal(a, b) for a, b in zip(got, want[0]))
+
+
+@pytest.mark.parametrize("layout", ["scattered", "coincident", "line"])
+@pytest.mark.parametrize("n", [1, 2, 255, 257, 960, 1024, 1025, 1920, 1921, 3000])
+def test_exported_tree_is_whole_at_the_pass_boundaries(ctx, n, layout):
+    """Triangle counts around the sizes where the clustering passes change
+    (one launch to 256 clusters, 960 per block of the windowed passes, 1024):
+    every leaf once, every box the exact union of its triangles, the depth
+    that of the longest path."""
+    rng = np.random.default_rng(n)
+    v = rng.uniform(-1, 1, (n, 3, 3)).astype(np.float32)
+    if layout == "coincident":
+        v[:] = v[0]
+    if layout == "line":
+        v *= np.float32(0.01)
+        v[..., 0] += np.arange(n, dtype=np.float32)[:, None]
+    sid = ctx.upload_scene(v.reshape(-1, 3), np.arange(3 * n, dtype=np.uint32).reshape(n, 3))
+    nodes, leaf = ctx.export_bvh(sid)
+    info = ctx.scene_info(sid)
+    ctx.release_scene(sid)
+    assert sorted(leaf) == list(range(n))
+    tlo, thi = v.min(1), v.max(1)
+    kids = nodes.view(np.int32)[:, 12:14]
+    boxes = [(nodes[:, 0:3], nodes[:, 3:6]), (nodes[:, 6:9], nodes[:, 9:12])]
+    seen = np.zeros(n, int)
+    ulo, uhi, height = {}, {}, {}
+    order, stack = [], [0]
+    while stack:                       # parents before children
+        k = stack.pop()
+        order.append(k)
+        stack += [c for c in kids[k] if c >= 0]
+    assert len(order) == len(set(order)) == len(nodes) == max(1, n - 1)
+    for k in reversed(order):
+        lo, hi, h = [], [], 0
+        for side, c in enumerate(kids[k]):
+            if c < 0:
+                seen[~c] += 1
+                l, u = tlo[leaf[~c]], thi[leaf[~c]]
+            else:
+                l, u, h = ulo[c], uhi[c], max(h, height[c])
+            assert np.array_equal(boxes[side][0][k], l) and np.array_equal(boxes[side][1][k], u)
+            lo.append(l)
+            hi.append(u)
+        ulo[k], uhi[k], height[k] = np.minimum(*lo), np.maximum(*hi), h + 1
+    assert (seen == (2 if n == 1 else 1)).all()
+    assert info["depth"] == height[0]
+
+
+def test_exported_tree_of_many_blocks_is_whole(ctx):
+    """1.6M triangles: more clustering blocks than one block adds up the counts
+    of.  Every leaf and inner node is a child once, and every child's box is
+    the union of its own two."""
+    n = 1_600_000
+    rng = np.random.default_rng(1)
+    v = rng.uniform(-1, 1, (n, 1, 3)).astype(np.float32) + rng.uniform(-.01, .01, (n, 3, 3)).astype(np.float32)
+    sid = ctx.upload_scene(v.reshape(-1, 3), np.arange(3 * n, dtype=np.uint32).reshape(n, 3))
+    nodes, leaf = ctx.export_bvh(sid)
+    ctx.release_scene(sid)
+    kids = nodes.view(np.int32)[:, 12:14].T.reshape(-1).astype(np.int64)
+    lo = np.concatenate([nodes[:, 0:3], nodes[:, 6:9]])
+    hi = np.concatenate([nodes[:, 3:6], nodes[:, 9:12]])
+    assert np.array_equal(np.sort(kids), np.r_[np.arange(-n, 0), np.arange(1, n - 1)])
+    assert np.array_equal(np.sort(leaf), np.arange(n))
+    inner = kids >= 0
+    c = kids[inner]
+    assert np.array_equal(lo[inner], np.minimum(nodes[c, 0:3], nodes[c, 6:9]))
+    assert np.array_equal(hi[inner], np.maximum(nodes[c, 3:6], nodes[c, 9:12]))
+    prim = leaf[~kids[~inner]]
+    assert np.array_equal(lo[~inner], v.min(1)[prim]) and np.array_equal(hi[~inner], v.max(1)[prim])

@@ -195,7 +195,7 @@ __global__ void k_morton(const float4* __restrict__ cen, int n, const float* __r
 // the same time at 16-64.
 constexpr int kPlocRadius = 32;
 
-// The initial clusters (leaf j = ~j).
+// The initial clusters (leaf j = ~j; no inner node below).
 __global__ void k_leaves(const uint32_t* __restrict__ order, int n, const float4* __restrict__ lo,
                          const float4* __restrict__ hi, float4* __restrict__ clo,
                          float4* __restrict__ chi, int* __restrict__ cid)
@@ -203,140 +203,487 @@ __global__ void k_leaves(const uint32_t* __restrict__ order, int n, const float4
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     uint32_t p = order[j];
-    clo[j] = lo[p];
+    const float4 l = lo[p];
+    clo[j] = make_float4(l.x, l.y, l.z, 0.0f);
     chi[j] = hi[p];
     cid[j] = ~j;
 }
 
-// Candidate j = i + o against the best so far.  A NaN area (non-finite
-// input) counts as +inf so the pair order stays total.  Tie key for this i:
-// distance, then the lower position's parity, then the lower position (the
-// left candidate is the lower one).
-__device__ __forceinline__ void ploc_consider(const float4& a, const float4& b, const float4& l,
-                                              const float4& h, int i, int o, float& best,
-                                              int& bj, int& bk)
+// fminf/fmaxf of numbers that were loaded get a canonicalizing instruction
+// per operand first (12 of the 24 of a union's box); these do not.
+__device__ __forceinline__ float min_f32(float a, float b)
 {
-    const float dx = fmaxf(b.x, h.x) - fminf(a.x, l.x);
-    const float dy = fmaxf(b.y, h.y) - fminf(a.y, l.y);
-    const float dz = fmaxf(b.z, h.z) - fminf(a.z, l.z);
-    float ar = dx * dy + dy * dz + dz * dx;
-    ar = ar == ar ? ar : __builtin_huge_valf();
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max_f32(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+// Surface area (its half) of the union of two boxes, each axis as (lower,
+// upper).  One fixed operation order: both clusters of a pair, on whichever
+// path, see the same bits.
+__device__ __forceinline__ float ploc_area(float2 ax, float2 ay, float2 az, float2 bx, float2 by,
+                                           float2 bz)
+{
+    const float dx = max_f32(ax.y, bx.y) - min_f32(ax.x, bx.x);
+    const float dy = max_f32(ay.y, by.y) - min_f32(ay.x, by.x);
+    const float dz = max_f32(az.y, bz.y) - min_f32(az.x, bz.x);
+    return dx * dy + dy * dz + dz * dx;
+}
+
+// Candidate j = i + o of area `ar` as a sort key: the area's bits, then the
+// tie key (distance, then the lower position's parity, then the lower
+// position: the left candidate is the lower one), unique per candidate, so
+// the pair order is total.  A NaN area (non-finite input) counts as +inf.
+// The key is also a positive finite double of the same order (v_min_f64), and
+// kNoKey, +inf, is above all of them.
+constexpr unsigned long long kNoKey = 0x7ff0000000000000ull;
+__device__ __forceinline__ unsigned long long ploc_key(float ar, int i, int o)
+{
     const int k = 4 * abs(o) + 2 * (min(i, i + o) & 1) + (o > 0 ? 1 : 0);
-    if (bj < 0 || ar < best || (ar == best && k < bk)) {
-        best = ar;
-        bj = i + o;
-        bk = k;
-    }
+    const float a = min_f32(ar, __builtin_huge_valf());
+    return ((unsigned long long)__float_as_uint(a) << 32) | (unsigned)k;
 }
-
-// Nearest neighbour of every cluster within kPlocRadius positions; the
-// block's window of boxes is staged in LDS.
-__global__ __launch_bounds__(256) void k_ploc_nn(const float4* __restrict__ clo,
-                                                 const float4* __restrict__ chi, int m,
-                                                 int* __restrict__ nn)
+__device__ __forceinline__ unsigned long long min_key(unsigned long long a, unsigned long long b)
 {
-    constexpr int W = 256 + 2 * kPlocRadius;
-    __shared__ float4 slo[W], shi[W];
-    const int base = blockIdx.x * 256;
-    for (int t = threadIdx.x; t < W; t += 256) {
-        const int g = base - kPlocRadius + t;
-        if (g >= 0 && g < m) {
-            slo[t] = clo[g];
-            shi[t] = chi[g];
-        }
-    }
-    __syncthreads();
-    const int i = base + threadIdx.x;
-    if (i >= m) return;
-    const int li = threadIdx.x + kPlocRadius;
-    const float4 a = slo[li], b = shi[li];
-    float best = __builtin_huge_valf();
-    int bj = -1, bk = 0;
-    const int o0 = max(-kPlocRadius, -i), o1 = min(kPlocRadius, m - 1 - i);
-    for (int o = o0; o <= o1; ++o)
-        if (o != 0) ploc_consider(a, b, slo[li + o], shi[li + o], i, o, best, bj, bk);
-    nn[i] = bj;
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(__longlong_as_double((long long)a)), "v"(__longlong_as_double((long long)b)));
+    return (unsigned long long)__double_as_longlong(r);
+}
+// The candidate of a key.
+__device__ __forceinline__ int ploc_neighbour(unsigned long long key, int i)
+{
+    const int k = (int)(uint32_t)key;
+    return (k & 1) ? i + (k >> 2) : i - (k >> 2);
 }
 
-// The last passes (m <= kPlocFull clusters, the top of the tree): exact
-// nearest neighbour over all clusters, one workgroup.
+// Where a pass stands: `m` clusters in list `cur`.  Pass p reads state p and
+// writes state p + 1, so passes are queued without waiting for their counts:
+// a launch covers the clusters the host last knew of, and blocks past the
+// current count return.
+struct PlocState {
+    int m, cur;
+    int depth;  // of the whole tree, once m is 1
+};
+struct PlocBufs {
+    float4 *lo[2], *hi[2];  // cluster boxes; lo.w: inner nodes on the longest path down
+    int* id[2];             // inner node, or ~leaf
+    int* nn;
+    unsigned long long* counts;
+    PlocState* state;
+    BNode* nodes;
+    int *iparent, *lparent;
+};
+
+// Clusters of a block of the windowed search.  Its 256 threads also find the
+// neighbours of the kPlocRadius clusters on each side, which decide whether
+// its own are mutual, so that the flags need no launch between.  Blocks of
+// 1024 waste less on that (6% against a third) but leave CUs idle: the search
+// of 8 passes from 0.5M clusters took 125 us in them, 115 in blocks of 256;
+// of the 8 from 55k clusters 88 against 68.
+constexpr int kPlocThreads = 256;
+constexpr int kPlocOwn = kPlocThreads - 2 * kPlocRadius;
+// Blocks whose counts each block of the second half adds up by itself; above,
+// a launch between does it once (the build over 2M triangles, 10,300 blocks:
+// 1.95 ms against 1.89; the adding grows with the square of the count).
+constexpr int kPlocSums = 8192;
+// The passes at up to kPlocFull clusters (the top of the tree) search all
+// clusters; from kPlocTop down all of them run in one launch of one block.
 constexpr int kPlocFull = 1024;
-__global__ __launch_bounds__(kPlocFull) void k_ploc_nn_full(const float4* __restrict__ clo,
-                                                            const float4* __restrict__ chi,
-                                                            int m, int* __restrict__ nn)
+constexpr int kPlocTop = 256;
+// From here down one wave does it all (its share of the launch below: 10 us
+// less than with every wave to the end; at 64 the same).
+constexpr int kPlocWave = 32;
+// Windowed passes queued before the host looks at the count.
+constexpr int kPlocQueue = 8;
+
+__device__ __forceinline__ int lanes_below(unsigned long long mask)
 {
-    __shared__ float4 slo[kPlocFull], shi[kPlocFull];
-    const int i = threadIdx.x;
-    if (i < m) {
-        slo[i] = clo[i];
-        shi[i] = chi[i];
-    }
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+}
+
+// Of the block: its clusters that survive the pass (unpaired, or the lower of
+// a mutual pair) before this thread's, in the low word, and its pairs before
+// this thread's in the high word; `total` the block's sums.
+__device__ __forceinline__ unsigned long long ploc_rank(bool survives, bool pair,
+                                                        unsigned long long* waves,
+                                                        unsigned long long& total)
+{
+    const unsigned long long ms = __ballot(survives), mp = __ballot(pair);
+    const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 0)
+        waves[w] = ((unsigned long long)__popcll(mp) << 32) | (unsigned long long)__popcll(ms);
     __syncthreads();
-    if (i >= m) return;
-    const float4 a = slo[i], b = shi[i];
-    float best = __builtin_huge_valf();
-    int bj = -1, bk = 0;
-    for (int j = 0; j < m; ++j)
-        if (j != i) ploc_consider(a, b, slo[j], shi[j], i, j - i, best, bj, bk);
-    nn[i] = bj;
-}
-
-// Per cluster: low word 1 if it survives the pass (unpaired, or the lower
-// of a mutual pair), high word 1 if it is the lower of a mutual pair.
-__global__ void k_ploc_flags(const int* __restrict__ nn, int m,
-                             unsigned long long* __restrict__ flag)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const int j = nn[i];
-    const bool mutual = nn[j] == i;
-    unsigned long long f = 0;
-    if (!mutual) f = 1ull;
-    else if (i < j) f = (1ull << 32) | 1ull;
-    flag[i] = f;
-}
-
-// Compaction and merge.  scan = inclusive sum of the flags; with M merges
-// in a pass over m clusters, the pass's nodes are [m - 1 - M, m - 1).
-__global__ void k_ploc_merge(const int* __restrict__ nn, int m,
-                             const unsigned long long* __restrict__ scan,
-                             const float4* __restrict__ clo, const float4* __restrict__ chi,
-                             const int* __restrict__ cid, float4* __restrict__ olo,
-                             float4* __restrict__ ohi, int* __restrict__ ocid,
-                             BNode* __restrict__ nodes, int* __restrict__ iparent,
-                             int* __restrict__ lparent)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const int j = nn[i];
-    const bool mutual = nn[j] == i;
-    if (mutual && j < i) return;  // absorbed by its partner
-    const unsigned long long f = mutual ? (1ull << 32) | 1ull : 1ull;
-    const unsigned long long ex = scan[i] - f;
-    const int pos = (int)(uint32_t)ex;
-    if (!mutual) {
-        olo[pos] = clo[i];
-        ohi[pos] = chi[i];
-        ocid[pos] = cid[i];
-        return;
+    unsigned long long before = 0;
+    total = 0;
+    for (int k = 0; k < nw; ++k) {
+        const unsigned long long v = waves[k];
+        if (k < w) before += v;
+        total += v;
     }
-    const int merges = (int)(scan[m - 1] >> 32);
-    const int id = m - 1 - merges + (int)(ex >> 32);
-    const float4 l0 = clo[i], h0 = chi[i], l1 = clo[j], h1 = chi[j];
-    const int c0 = cid[i], c1 = cid[j];
+    return before + (((unsigned long long)lanes_below(mp) << 32) | (unsigned long long)lanes_below(ms));
+}
+
+// The inner node `id` of a mutual pair, and its cluster.
+__device__ __forceinline__ void ploc_pair(const PlocBufs& B, int id, float4& l, float4& h, int c0,
+                                          const float4& l1, const float4& h1, int c1)
+{
     BNode n;
-    n.a = make_float4(l0.x, l0.y, l0.z, h0.x);
-    n.b = make_float4(h0.y, h0.z, l1.x, l1.y);
+    n.a = make_float4(l.x, l.y, l.z, h.x);
+    n.b = make_float4(h.y, h.z, l1.x, l1.y);
     n.c = make_float4(l1.z, h1.x, h1.y, h1.z);
     n.d = make_int4(c0, c1, 0, 0);
-    nodes[id] = n;
-    if (c0 >= 0) iparent[c0] = 2 * id + 0;
-    else lparent[~c0] = 2 * id + 0;
-    if (c1 >= 0) iparent[c1] = 2 * id + 1;
-    else lparent[~c1] = 2 * id + 1;
-    olo[pos] = make_float4(fminf(l0.x, l1.x), fminf(l0.y, l1.y), fminf(l0.z, l1.z), 0.0f);
-    ohi[pos] = make_float4(fmaxf(h0.x, h1.x), fmaxf(h0.y, h1.y), fmaxf(h0.z, h1.z), 0.0f);
-    ocid[pos] = id;
+    B.nodes[id] = n;
+    if (c0 >= 0) B.iparent[c0] = 2 * id + 0;
+    else B.lparent[~c0] = 2 * id + 0;
+    if (c1 >= 0) B.iparent[c1] = 2 * id + 1;
+    else B.lparent[~c1] = 2 * id + 1;
+    l = make_float4(fminf(l.x, l1.x), fminf(l.y, l1.y), fminf(l.z, l1.z), fmaxf(l.w, l1.w) + 1.0f);
+    h = make_float4(fmaxf(h.x, h1.x), fmaxf(h.y, h1.y), fmaxf(h.z, h1.z), 0.0f);
+}
+
+// Windowed pass, first half: every cluster's partner (-1: none) within
+// kPlocRadius positions and each block's counts.  The block's window of
+// boxes is staged in LDS as (lower, upper) per axis, three 8-byte reads per
+// candidate; the reads and the vector ALUs take about as long.
+__global__ __launch_bounds__(kPlocThreads) void k_ploc_find(PlocBufs B, int in)
+{
+    constexpr int T = kPlocThreads, W = T + 2 * kPlocRadius;
+    __shared__ float2 sx[W], sy[W], sz[W];
+    __shared__ int snn[T];
+    __shared__ unsigned long long waves[T / 64];
+    const int m = B.state[in].m, cur = B.state[in].cur;
+    const int base = blockIdx.x * kPlocOwn;
+    if (m <= kPlocFull || base >= m) return;
+    const int t = threadIdx.x;
+    const float inf = __builtin_huge_valf();
+    for (int k = t; k < W; k += T) {
+        const int g = base - 2 * kPlocRadius + k;
+        // no cluster there: a box whose unions have infinite area
+        float4 l = make_float4(-inf, -inf, -inf, 0.0f), h = make_float4(inf, inf, inf, 0.0f);
+        if (g >= 0 && g < m) {
+            l = B.lo[cur][g];
+            h = B.hi[cur][g];
+        }
+        sx[k] = make_float2(l.x, h.x);
+        sy[k] = make_float2(l.y, h.y);
+        sz[k] = make_float2(l.z, h.z);
+    }
+    __syncthreads();
+    const int i = base - kPlocRadius + t;
+    int bj = -1;
+    if (i >= 0 && i < m) {
+        const int li = t + kPlocRadius;
+        const float2 ax = sx[li], ay = sy[li], az = sz[li];
+        // candidates in the order of their tie keys, two distances at a time:
+        // the left one first, but the right one at odd distances from an even
+        // position; a later one has to be less
+        const bool right_first = (i & 1) == 0;
+        float best = inf;
+        int bo = 0;
+#pragma unroll 4
+        for (int d = 1; d <= kPlocRadius; d += 2) {
+            const float l1 = ploc_area(ax, ay, az, sx[li - d], sy[li - d], sz[li - d]);
+            const float r1 = ploc_area(ax, ay, az, sx[li + d], sy[li + d], sz[li + d]);
+            const float l2 = ploc_area(ax, ay, az, sx[li - d - 1], sy[li - d - 1], sz[li - d - 1]);
+            const float r2 = ploc_area(ax, ay, az, sx[li + d + 1], sy[li + d + 1], sz[li + d + 1]);
+            const bool take_r1 = r1 < l1 || (right_first && r1 == l1);
+            const float v1 = take_r1 ? r1 : l1;
+            if (v1 < best) {
+                best = v1;
+                bo = take_r1 ? d : -d;
+            }
+            const bool take_r2 = r2 < l2;
+            const float v2 = take_r2 ? r2 : l2;
+            if (v2 < best) {
+                best = v2;
+                bo = take_r2 ? d + 1 : -d - 1;
+            }
+        }
+        bj = i + bo;
+        if (bo == 0) {  // no finite area: the clusters that are there, one by one
+            unsigned long long key = kNoKey;
+            for (int o = max(-kPlocRadius, -i); o <= min(kPlocRadius, m - 1 - i); ++o)
+                if (o != 0)
+                    key = min_key(key, ploc_key(ploc_area(ax, ay, az, sx[li + o], sy[li + o],
+                                                          sz[li + o]), i, o));
+            bj = ploc_neighbour(key, i);
+        }
+    }
+    snn[t] = bj;
+    __syncthreads();
+    const bool own = t >= kPlocRadius && t < kPlocRadius + kPlocOwn && i < m;
+    // an own cluster's neighbour is among the block's threads
+    const bool mutual = own && snn[t + (bj - i)] == i;
+    unsigned long long total;
+    ploc_rank(own && !(mutual && bj < i), mutual && i < bj, waves, total);
+    if (own) B.nn[i] = mutual ? bj : -1;
+    if (t == 0) B.counts[blockIdx.x] = total;
+}
+
+// The blocks' counts made exclusive sums, the total behind them.  One block.
+__global__ __launch_bounds__(1024) void k_ploc_sums(PlocBufs B, int in)
+{
+    __shared__ unsigned long long part[1024];
+    const int m = B.state[in].m, t = threadIdx.x;
+    if (m <= kPlocFull) return;
+    const int nb = (m + kPlocOwn - 1) / kPlocOwn, per = (nb + 1023) / 1024;
+    const int k0 = min(nb, t * per), k1 = min(nb, k0 + per);
+    unsigned long long sum = 0;
+    for (int k = k0; k < k1; ++k) sum += B.counts[k];
+    part[t] = sum;
+    __syncthreads();
+    for (int d = 1; d < 1024; d <<= 1) {
+        const unsigned long long v = t >= d ? part[t - d] : 0;
+        __syncthreads();
+        part[t] += v;
+        __syncthreads();
+    }
+    unsigned long long run = part[t] - sum;
+    for (int k = k0; k < k1; ++k) {
+        const unsigned long long v = B.counts[k];
+        B.counts[k] = run;
+        run += v;
+    }
+    if (t == 1023) B.counts[nb] = run;
+}
+
+// Windowed pass, second half: compaction and merge.  With M merges in a pass
+// over m clusters, the pass's nodes are [m - 1 - M, m - 1).
+template <bool SUMMED>
+__global__ __launch_bounds__(kPlocOwn) void k_ploc_join(PlocBufs B, int in, int out)
+{
+    constexpr int T = kPlocOwn;
+    __shared__ unsigned long long waves[T / 64], sums[2][T / 64];
+    const int m = B.state[in].m, cur = B.state[in].cur;
+    const int t = threadIdx.x, base = blockIdx.x * T;
+    if (m <= kPlocFull) {
+        if (blockIdx.x == 0 && t == 0) B.state[out] = B.state[in];
+        return;
+    }
+    if (base >= m) return;
+    // the counts of the blocks before this one, and of all
+    const int nb = (m + kPlocOwn - 1) / kPlocOwn;
+    unsigned long long before = 0, all = 0;
+    if (!SUMMED) {
+        for (int k = t; k < nb; k += T) {
+            const unsigned long long v = B.counts[k];
+            all += v;
+            if (k < (int)blockIdx.x) before += v;
+        }
+    } else if (t == 0) {
+        before = B.counts[blockIdx.x];
+        all = B.counts[nb];
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        before += __shfl_xor(before, d);
+        all += __shfl_xor(all, d);
+    }
+    if ((t & 63) == 0) {
+        sums[0][t >> 6] = before;
+        sums[1][t >> 6] = all;
+    }
+    const int i = base + t;
+    const bool have = i < m;
+    const int j = have ? B.nn[i] : -1;
+    const bool survives = have && (j < 0 || i < j), pair = survives && j >= 0;
+    unsigned long long total;
+    unsigned long long ex = ploc_rank(survives, pair, waves, total);
+    all = 0;
+    for (int k = 0; k < T / 64; ++k) {
+        ex += sums[0][k];
+        all += sums[1][k];
+    }
+    if (blockIdx.x == 0 && t == 0) B.state[out] = PlocState{(int)(uint32_t)all, cur ^ 1, 0};
+    if (!survives) return;
+    float4 l = B.lo[cur][i], h = B.hi[cur][i];
+    int id = B.id[cur][i];
+    if (pair) {
+        const int node = m - 1 - (int)(all >> 32) + (int)(ex >> 32);
+        ploc_pair(B, node, l, h, id, B.lo[cur][j], B.hi[cur][j], B.id[cur][j]);
+        id = node;
+    }
+    const int pos = (int)(uint32_t)ex;
+    B.lo[cur ^ 1][pos] = l;
+    B.hi[cur ^ 1][pos] = h;
+    B.id[cur ^ 1][pos] = id;
+}
+
+// Key of the least candidate of cluster i among j0, j0 + dj, ... below j1;
+// kNoKey when there is none.
+__device__ __forceinline__ unsigned long long ploc_least(const float4* slo, const float4* shi, int i,
+                                                         int j0, int j1, int dj)
+{
+    const float4 a = slo[i], b = shi[i];
+    const float2 ax = make_float2(a.x, b.x), ay = make_float2(a.y, b.y), az = make_float2(a.z, b.z);
+    unsigned long long best = kNoKey;
+    // four candidates in flight, without branches: a lone wave waits for
+    // every read and every result
+    for (; j0 < j1; j0 += 4 * dj) {
+        float4 l[4], h[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = min(j0 + u * dj, kPlocFull - 1);
+            l[u] = slo[j];
+            h[u] = shi[j];
+        }
+        unsigned long long k[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = j0 + u * dj;
+            k[u] = ploc_key(ploc_area(ax, ay, az, make_float2(l[u].x, h[u].x),
+                                      make_float2(l[u].y, h[u].y), make_float2(l[u].z, h[u].z)),
+                            i, j - i);
+            k[u] = j < j1 && j != i ? k[u] : kNoKey;
+        }
+        best = min_key(best, min_key(min_key(k[0], k[1]), min_key(k[2], k[3])));
+    }
+    return best;
+}
+
+// First half of a pass over kPlocTop < m <= kPlocFull clusters: each block
+// takes 16 clusters, each of its 64 sixteenths of a wave one part of the
+// candidates.  One thread per cluster in a single block is bound by that
+// CU's vector ALUs (46.7 us a pass over the 37 passes of a 0.5M-triangle
+// terrain; 5.4 a pass here, 3.8 for its second half).
+__global__ __launch_bounds__(1024) void k_ploc_find_all(PlocBufs B, int in)
+{
+    __shared__ float4 slo[kPlocFull], shi[kPlocFull];
+    __shared__ unsigned long long key[16];
+    const int m = B.state[in].m, cur = B.state[in].cur;
+    const int t = threadIdx.x;
+    if (m <= kPlocTop || m > kPlocFull || (int)blockIdx.x * 16 >= m) return;
+    if (t < m) {
+        slo[t] = B.lo[cur][t];
+        shi[t] = B.hi[cur][t];
+    }
+    if (t < 16) key[t] = kNoKey;
+    __syncthreads();
+    const int i = blockIdx.x * 16 + (t & 15);
+    if (i < m) atomicMin(&key[t & 15], ploc_least(slo, shi, i, t >> 4, m, 64));
+    __syncthreads();
+    if (t < 16 && i < m) B.nn[i] = ploc_neighbour(key[t], i);
+}
+
+// One block over the last clusters.  LAST: all remaining passes, the clusters
+// in LDS throughout; each wave a share of the candidates of 64 clusters, and
+// from kPlocWave clusters down one wave does it all without barriers, its lanes
+// shared out over clusters and candidates.  Otherwise the second half of one
+// pass after k_ploc_find_all.  The loops end: a pass over two clusters or
+// more merges at least the least pair of all (its candidates are totally
+// ordered), and one that did not would stop them.
+template <bool LAST>
+__global__ __launch_bounds__(1024) void k_ploc_top(PlocBufs B, int in, int out)
+{
+    __shared__ float4 slo[kPlocFull], shi[kPlocFull];
+    __shared__ int sid[kPlocFull], snn[kPlocFull];
+    __shared__ unsigned long long key[kPlocFull];
+    __shared__ unsigned long long waves[16];
+    int m = B.state[in].m;
+    const int cur = B.state[in].cur, t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (m > kPlocFull || (!LAST && m <= kPlocTop)) {
+        if (t == 0) B.state[out] = B.state[in];
+        return;
+    }
+    if (t < m) {
+        slo[t] = B.lo[cur][t];
+        shi[t] = B.hi[cur][t];
+        sid[t] = B.id[cur][t];
+    }
+    __syncthreads();
+    bool stuck = false;
+    while (m > (LAST ? kPlocWave : 1) && !stuck) {
+        int j = -1;
+        if (LAST) {
+            key[t] = kNoKey;
+            __syncthreads();
+            const int groups = (m + 63) >> 6, parts = 16 / groups;
+            const int g = w % groups, p = w / groups, i = g * 64 + lane;
+            if (p < parts && i < m) atomicMin(&key[i], ploc_least(slo, shi, i, p, m, parts));
+            __syncthreads();
+            if (t < m) j = ploc_neighbour(key[t], t);
+        } else if (t < m) {
+            j = B.nn[t];
+        }
+        snn[t] = j;
+        __syncthreads();
+        const bool mutual = t < m && snn[j] == t;
+        const bool survives = t < m && !(mutual && j < t), pair = mutual && t < j;
+        unsigned long long total;
+        const unsigned long long ex = ploc_rank(survives, pair, waves, total);
+        float4 l, h;
+        int id = 0;
+        if (survives) {
+            l = slo[t];
+            h = shi[t];
+            id = sid[t];
+            if (pair) {
+                const int node = m - 1 - (int)(total >> 32) + (int)(ex >> 32);
+                ploc_pair(B, node, l, h, id, slo[j], shi[j], sid[j]);
+                id = node;
+            }
+        }
+        __syncthreads();
+        const int pos = (int)(uint32_t)ex;
+        if (survives) {
+            slo[pos] = l;
+            shi[pos] = h;
+            sid[pos] = id;
+        }
+        __syncthreads();
+        const int m2 = (int)(uint32_t)total;
+        stuck = m2 >= m;
+        m = m2;
+        if (!LAST) break;
+    }
+    if (!LAST) {
+        if (t < m) {
+            B.lo[cur ^ 1][t] = slo[t];
+            B.hi[cur ^ 1][t] = shi[t];
+            B.id[cur ^ 1][t] = sid[t];
+        }
+        if (t == 0) B.state[out] = PlocState{m, cur ^ 1, 0};
+        return;
+    }
+    if (w != 0) return;
+    while (m > 1 && !stuck) {
+        const int span = 1 << (32 - __builtin_clz(m - 1));  // lanes per part: m or more
+        const int i = lane & (span - 1);
+        unsigned long long k = kNoKey;
+        if (i < m) k = ploc_least(slo, shi, i, lane / span, m, 64 / span);
+        for (int d = span; d < 64; d <<= 1) k = min_key(k, __shfl_xor(k, d));
+        const int j = lane < m ? ploc_neighbour(k, lane) : lane;
+        const bool mutual = lane < m && __shfl(j, j) == lane;
+        const bool survives = lane < m && !(mutual && j < lane), pair = mutual && lane < j;
+        const unsigned long long ms = __ballot(survives), mp = __ballot(pair);
+        float4 l = slo[lane], h = shi[lane];
+        int id = sid[lane];
+        if (pair) {
+            const int node = m - 1 - (int)__popcll(mp) + lanes_below(mp);
+            ploc_pair(B, node, l, h, id, slo[j], shi[j], sid[j]);
+            id = node;
+        }
+        // one wave: its LDS operations complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const int pos = lanes_below(ms);
+        if (survives) {
+            slo[pos] = l;
+            shi[pos] = h;
+            sid[pos] = id;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        stuck = mp == 0;
+        m = (int)__popcll(ms);
+    }
+    if (t == 0) {
+        B.state[out] = PlocState{m, cur ^ 1, (int)slo[0].w};
+        B.iparent[0] = -1;  // node 0 is the root
+    }
 }
 
 // One triangle: a root whose two children are the same leaf; testing it
@@ -354,22 +701,6 @@ __global__ void k_single(const float4* __restrict__ clo, const float4* __restric
     nodes[0] = n;
     iparent[0] = -1;
     lparent[0] = 0;
-}
-
-// Depth = inner nodes on the longest root-to-leaf path.
-__global__ void k_depth(const int* __restrict__ iparent, const int* __restrict__ lparent, int n,
-                        unsigned int* __restrict__ depth)
-{
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    int p = lparent[j] >> 1;
-    unsigned int d = 1;
-    while (p != 0) {
-        p = iparent[p] >> 1;
-        ++d;
-        if (d > 4096) break;  // malformed tree guard
-    }
-    atomicMax(depth, d);
 }
 
 // BVH2 -> BVH4: every even-depth BVH2 node becomes a BVH4 node whose
@@ -620,7 +951,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     DevBuf tmp = dev_alloc(ctx, tmp_bytes > 0 ? tmp_bytes : 16);
     VLB_HIP(rocprim::radix_sort_pairs(tmp.p, tmp_bytes, keys.as<uint32_t>(), keys2.as<uint32_t>(),
                                       vals.as<uint32_t>(), s.leaf_prims.as<uint32_t>(), (size_t)n, 0, 30, st));
-    // hierarchy (PLOC), one host round trip per pass for the cluster count
+    // hierarchy (PLOC)
     const int nin = n > 1 ? n - 1 : 1;
     s.nodes = dev_alloc(ctx, (size_t)nin * sizeof(BNode));
     s.tris = dev_alloc(ctx, (size_t)n * kTriWords * sizeof(float));
@@ -635,55 +966,57 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     k_leaves<<<nblk(n), 256, 0, st>>>(s.leaf_prims.as<uint32_t>(), n, lo.as<float4>(), hi.as<float4>(),
                                       clo[0].as<float4>(), chi[0].as<float4>(), cid[0].as<int>());
     VLB_HIP(hipGetLastError());
-    DevBuf dep = dev_alloc(ctx, sizeof(unsigned int));
-    VLB_HIP(hipMemsetAsync(dep.p, 0, sizeof(unsigned int), st));
+    DevBuf nn, counts, state;
+    PlocState left{1, 0, 1};
     if (n == 1) {
         k_single<<<1, 1, 0, st>>>(clo[0].as<float4>(), chi[0].as<float4>(), s.nodes.as<BNode>(),
                                   iparent.as<int>(), lparent.as<int>());
-        unsigned int one = 1;
-        VLB_HIP(hipMemcpyAsync(dep.p, &one, sizeof one, hipMemcpyHostToDevice, st));
     } else {
-        DevBuf nn = dev_alloc(ctx, (size_t)n * sizeof(int));
-        DevBuf flag = dev_alloc(ctx, (size_t)n * sizeof(unsigned long long));
-        DevBuf scan = dev_alloc(ctx, (size_t)n * sizeof(unsigned long long));
-        size_t ps_bytes = 0;
-        VLB_HIP(rocprim::inclusive_scan(nullptr, ps_bytes, flag.as<unsigned long long>(),
-                                        scan.as<unsigned long long>(), (size_t)n,
-                                        rocprim::plus<unsigned long long>(), st));
-        DevBuf ps_tmp = dev_alloc(ctx, ps_bytes > 0 ? ps_bytes : 16);
-        int m = n, cur = 0;
-        // every pass merges at least one pair, so at most n - 1 passes
-        for (int pass = 0; m > 1; ++pass) {
-            VLB_REQUIRE(pass < n, VLB_ERR_DEVICE, "PLOC build made no progress");
-            if (m <= kPlocFull)
-                k_ploc_nn_full<<<1, kPlocFull, 0, st>>>(clo[cur].as<float4>(), chi[cur].as<float4>(),
-                                                        m, nn.as<int>());
-            else
-                k_ploc_nn<<<nblk(m), 256, 0, st>>>(clo[cur].as<float4>(), chi[cur].as<float4>(), m,
-                                                   nn.as<int>());
-            k_ploc_flags<<<nblk(m), 256, 0, st>>>(nn.as<int>(), m, flag.as<unsigned long long>());
-            VLB_HIP(rocprim::inclusive_scan(ps_tmp.p, ps_bytes, flag.as<unsigned long long>(),
-                                            scan.as<unsigned long long>(), (size_t)m,
-                                            rocprim::plus<unsigned long long>(), st));
-            k_ploc_merge<<<nblk(m), 256, 0, st>>>(
-                nn.as<int>(), m, scan.as<unsigned long long>(), clo[cur].as<float4>(),
-                chi[cur].as<float4>(), cid[cur].as<int>(), clo[cur ^ 1].as<float4>(),
-                chi[cur ^ 1].as<float4>(), cid[cur ^ 1].as<int>(), s.nodes.as<BNode>(),
-                iparent.as<int>(), lparent.as<int>());
-            VLB_HIP(hipGetLastError());
-            unsigned long long tot = 0;
-            VLB_HIP(hipMemcpyAsync(&tot, scan.as<unsigned long long>() + (m - 1), sizeof tot,
-                                   hipMemcpyDeviceToHost, st));
-            VLB_HIP(hipStreamSynchronize(st));
-            const int m2 = (int)(uint32_t)tot;
-            VLB_REQUIRE(m2 >= 1 && m2 < m, VLB_ERR_DEVICE, "PLOC build made no progress");
-            m = m2;
-            cur ^= 1;
+        nn = dev_alloc(ctx, (size_t)n * sizeof(int));
+        counts = dev_alloc(ctx, (size_t)(n / kPlocOwn + 2) * sizeof(unsigned long long));
+        state = dev_alloc(ctx, (kPlocQueue + 1) * sizeof(PlocState));
+        PlocBufs B;
+        for (int k = 0; k < 2; ++k) {
+            B.lo[k] = clo[k].as<float4>();
+            B.hi[k] = chi[k].as<float4>();
+            B.id[k] = cid[k].as<int>();
         }
-        const int root_parent = -1;
-        VLB_HIP(hipMemcpyAsync(iparent.p, &root_parent, sizeof root_parent, hipMemcpyHostToDevice, st));
-        k_depth<<<nblk(n), 256, 0, st>>>(iparent.as<int>(), lparent.as<int>(), n,
-                                         dep.as<unsigned int>());
+        B.nn = nn.as<int>();
+        B.counts = counts.as<unsigned long long>();
+        B.state = state.as<PlocState>();
+        B.nodes = s.nodes.as<BNode>();
+        B.iparent = iparent.as<int>();
+        B.lparent = lparent.as<int>();
+        int in = 0;
+        left = PlocState{n, 0, 0};
+        VLB_HIP(hipMemcpyAsync(&B.state[0], &left, sizeof left, hipMemcpyHostToDevice, st));
+        while (left.m > kPlocFull) {
+            const int before = left.m;
+            const int nb = (before + kPlocOwn - 1) / kPlocOwn;
+            for (int p = 0; p < kPlocQueue; ++p, in = p) {
+                k_ploc_find<<<nb, kPlocThreads, 0, st>>>(B, in);
+                if (nb > kPlocSums) {
+                    k_ploc_sums<<<1, 1024, 0, st>>>(B, in);
+                    k_ploc_join<true><<<nb, kPlocOwn, 0, st>>>(B, in, p + 1);
+                } else {
+                    k_ploc_join<false><<<nb, kPlocOwn, 0, st>>>(B, in, p + 1);
+                }
+            }
+            VLB_HIP(hipGetLastError());
+            VLB_HIP(hipMemcpyAsync(&left, &B.state[kPlocQueue], sizeof left, hipMemcpyDeviceToHost, st));
+            VLB_HIP(hipStreamSynchronize(st));
+            // a pass over several clusters merges at least one pair
+            VLB_REQUIRE(left.m >= 1 && left.m < before, VLB_ERR_DEVICE, "PLOC build made no progress");
+        }
+        if (left.m > kPlocTop)
+            for (int p = 0; p < kPlocQueue; ++p, in = p) {
+                k_ploc_find_all<<<(left.m + 15) / 16, 1024, 0, st>>>(B, in);
+                k_ploc_top<false><<<1, 1024, 0, st>>>(B, in, p + 1);
+            }
+        const int out = in == 0 ? 1 : 0;
+        k_ploc_top<true><<<1, 1024, 0, st>>>(B, in, out);
+        VLB_HIP(hipGetLastError());
+        VLB_HIP(hipMemcpyAsync(&left, &B.state[out], sizeof left, hipMemcpyDeviceToHost, st));
     }
     VLB_HIP(hipGetLastError());
     // BVH4: even-depth BVH2 nodes; an exclusive scan of their child counts
@@ -710,6 +1043,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
                            hipMemcpyDeviceToHost, st));
     VLB_HIP(hipMemcpyAsync(hb, bnd.p, 13 * sizeof(float), hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
+    VLB_REQUIRE(left.m == 1, VLB_ERR_DEVICE, "PLOC build made no progress");
     const int n4 = 1 + (int)(uint32_t)(last[0] + last[1]);
     // node unit: the power of two that brings the largest coordinate to
     // [2^13, 2^14) units, so that offsets stay within FP16's range
@@ -728,8 +1062,6 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
                                           s.nodes4.as<Node4>(), s.tris.as<float4>());
     VLB_HIP(hipGetLastError());
     VLB_HIP(hipEventRecord(e1, st));
-    unsigned int depth = 0;
-    VLB_HIP(hipMemcpyAsync(&depth, dep.p, sizeof depth, hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
     float ms = 0.0f;
     VLB_HIP(hipEventElapsedTime(&ms, e0, e1));
@@ -738,7 +1070,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     s.build_ms = ms;
     s.nnodes = nin;
     s.nnodes4 = n4;
-    s.depth = depth;
+    s.depth = (uint32_t)left.depth;
     for (int a = 0; a < 3; ++a) {
         s.bmin[a] = hb[6 + a];
         s.bmax[a] = hb[9 + a];
