@@ -269,3 +269,28 @@ def test_exported_tree_of_many_blocks_is_whole(ctx):
     assert np.array_equal(hi[inner], np.maximum(nodes[c, 3:6], nodes[c, 9:12]))
     prim = leaf[~kids[~inner]]
     assert np.array_equal(lo[~inner], v.min(1)[prim]) and np.array_equal(hi[~inner], v.max(1)[prim])
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 300_001])
+def test_first_bad_index_or_coordinate_is_named(ctx, n):
+    """Geometry checked on the device: the first bad index is reported, before
+    any bad coordinate; coordinates of unused vertices count; 2^100 passes."""
+    rng = np.random.default_rng(n)
+    v = rng.uniform(-1, 1, (3 * n + 2, 3)).astype(np.float32)
+    idx = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    good = v.copy()
+    good[-1] = 2.0 ** 100
+    ctx.release_scene(ctx.upload_scene(good, idx))
+    for bad in (np.nan, np.inf, np.float32(1.5) * np.float32(2.0 ** 100)):
+        w = v.copy()
+        w[-1, 1] = bad
+        w[-1, 2] = np.nan
+        with pytest.raises(vlb.VlbError, match=f"coordinate .* at {w.size - 2}$"):
+            ctx.upload_scene(w, idx)
+    w = v.copy()
+    w[0, 0] = np.nan
+    j = idx.copy()
+    j[n // 2:, 1] = len(v)
+    with pytest.raises(vlb.VlbError, match=f"index out of range at {3 * (n // 2) + 1}$"):
+        ctx.upload_scene(w, j)
+    assert ctx.scene_info(ctx.upload_scene(v, idx))["num_tris"] == n

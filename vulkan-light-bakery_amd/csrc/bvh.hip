@@ -16,6 +16,24 @@
 namespace vlb {
 namespace {
 
+// First index out of range and first vertex coordinate that is not finite or
+// beyond 2^100 (bad[0], bad[1]; 0xffffffffffffffff: none).  On the host these
+// loops took 0.45 of the 2.95 ms of opening a 0.5M-triangle terrain.
+__global__ void k_check(const uint32_t* __restrict__ idx, unsigned long long nidx, uint32_t nverts,
+                        const float* __restrict__ xyz, unsigned long long ncoords,
+                        unsigned long long* __restrict__ bad)
+{
+    const unsigned long long step = (unsigned long long)gridDim.x * blockDim.x;
+    const unsigned long long t = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+    unsigned long long bi = ~0ull, bc = ~0ull;
+    for (unsigned long long i = t; i < nidx; i += step)
+        if (idx[i] >= nverts) bi = i < bi ? i : bi;
+    for (unsigned long long i = t; i < ncoords; i += step)
+        if (!(fabsf(xyz[i]) <= 0x1p100f)) bc = i < bc ? i : bc;
+    if (bi != ~0ull) atomicMin(&bad[0], bi);
+    if (bc != ~0ull) atomicMin(&bad[1], bc);
+}
+
 // Gather triangles, per-prim boxes and centroids, shading records.
 __global__ void k_gather(const float* __restrict__ xyz, const uint32_t* __restrict__ idx,
                          const float* __restrict__ normals, const float* __restrict__ albedo,
@@ -911,6 +929,20 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     DevBuf d_nrm, d_alb;
     VLB_HIP(hipMemcpyAsync(d_xyz.p, xyz, d_xyz.bytes, hipMemcpyHostToDevice, st));
     VLB_HIP(hipMemcpyAsync(d_idx.p, idx, d_idx.bytes, hipMemcpyHostToDevice, st));
+    unsigned long long bad[2] = {~0ull, ~0ull};
+    DevBuf d_bad = dev_alloc(ctx, sizeof bad);
+    VLB_HIP(hipMemcpyAsync(d_bad.p, bad, sizeof bad, hipMemcpyHostToDevice, st));
+    k_check<<<std::min(2048, nblk(n)), 256, 0, st>>>(d_idx.as<uint32_t>(), (unsigned long long)n * 3,
+                                                    nverts, d_xyz.as<float>(),
+                                                    (unsigned long long)nverts * 3,
+                                                    d_bad.as<unsigned long long>());
+    VLB_HIP(hipGetLastError());
+    VLB_HIP(hipMemcpyAsync(bad, d_bad.p, sizeof bad, hipMemcpyDeviceToHost, st));
+    VLB_HIP(hipStreamSynchronize(st));
+    VLB_REQUIRE(bad[0] == ~0ull, VLB_ERR_INVALID, "index out of range at " + std::to_string(bad[0]));
+    // the BVH4 node grids need finite boxes of bounded magnitude
+    VLB_REQUIRE(bad[1] == ~0ull, VLB_ERR_INVALID,
+                "vertex coordinate not finite or beyond 2^100 at " + std::to_string(bad[1]));
     if (normals) {
         d_nrm = dev_alloc(ctx, (size_t)nverts * 3 * sizeof(float));
         VLB_HIP(hipMemcpyAsync(d_nrm.p, normals, d_nrm.bytes, hipMemcpyHostToDevice, st));
