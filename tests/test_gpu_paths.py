@@ -294,3 +294,17 @@ def test_first_bad_index_or_coordinate_is_named(ctx, n):
     with pytest.raises(vlb.VlbError, match=f"index out of range at {3 * (n // 2) + 1}$"):
         ctx.upload_scene(w, j)
     assert ctx.scene_info(ctx.upload_scene(v, idx))["num_tris"] == n
+
+
+@pytest.mark.parametrize("P,R", [(1, 1), (1, 33), (16, 32), (17, 95), (64, 1024), (500, 2049), (1500, 4096)])
+def test_work_fetch_covers_every_ray(ctx, room, P, R):
+    """Launches from one trace tile to more rounds than waves, through the
+    fused kernel (small launches with fewer workgroups) and the wavefront
+    kernels (work taken by their own counters): the same bits."""
+    s, sid, o = room
+    probes = np.random.default_rng(P + R).uniform([1, 0.5, 1], [9, 3.5, 9], (P, 3)).astype(np.float32)
+    lights = [(vlb.LIGHT_DIRECTIONAL, (0.3, -1.0, 0.2), (3.0, 2.0, 1.0))]
+    got = [ctx.bake(sid, vlb.Params(probes=probes, rays=R, lights=lights, trace_variant=v))
+           for v in (0, 4, 12, 36, 13)]
+    for g in got[1:]:
+        assert np.array_equal(_bits(g), _bits(got[0]))

@@ -23,9 +23,9 @@
 // k_trace walks its rays XCD by XCD: workgroup b runs on XCD b % 8
 // (round-robin dispatch), and XCD x owns the x-th contiguous eighth of the
 // rays, so neighbouring probes and directions share that XCD's L2.  Work is
-// taken 256 rays at a time from the XCD's counter, then from the other
-// XCDs' once it is drained, so the launch ends when the work does rather
-// than when its unluckiest workgroup does.
+// taken 64 rays at a time from the XCD's counters, then from the other XCDs'
+// once they are drained, so the launch ends when the work does rather than
+// when its unluckiest workgroup does.
 #include "project_common.hpp"
 
 namespace vlb {
@@ -39,9 +39,9 @@ __global__ void k_zero_ctr8(unsigned long long* c)
 
 // ----------------------------------------------------------- trace + shade
 // One ray per lane, persistent, over "trace tiles" (16 probes x 32 rays =
-// 512 rays) taken half a tile per workgroup and fetch.  Thread t of a tile traces for probe 16*pg + (l & 15)
-// the ray 32*ch + 8*(l >> 4) + e, with l = t >> 3 and e = t & 7, and stores
-// its radiance at rad[((tile*3 + c)*64 + l)*8 + e]: the 16x16 MFMA A-operand
+// 512 rays), 64 rays per wave and fetch.  Thread t of a tile traces for probe
+// 16*pg + (l & 15) the ray 32*ch + 8*(l >> 4) + e, with l = t >> 3 and
+// e = t & 7, and stores its radiance at rad[((tile*3 + c)*64 + l)*8 + e]: the 16x16 MFMA A-operand
 // order of the projection kernel, written fully coalesced.  The lane map
 // (tile_map, a.map) sets how many neighbouring probes x directions (probes
 // Morton sorted, directions on a Hilbert curve) one wave covers.
@@ -58,41 +58,11 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_trace(BakeArgs a)
     Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
     TraceCount cnt;
     uint32_t nshadow = 0;
-    // 32 64-aligned ranges, range 4x + w owned by wave w of the workgroups on
-    // XCD x (= blockIdx % 8); a wave takes 64 rays per fetch from its own
-    // range, then from its XCD's other ranges, then from the other XCDs'
-    // (nitems is a multiple of 512, so a fetched chunk is whole)
-    const size_t nitems = (size_t)a.ntrace * 512;
-    const size_t per_rng = ((nitems + 31) / 32 + 63) / 64 * 64;
-    const int own = (blockIdx.x & 7) * 4 + (tid >> 6);
-    int victim = 0;  // ranges tried (wave-uniform)
+    __shared__ unsigned used;
+    const WorkRanges work(a.wctr, (size_t)a.ntrace * 512, &used);
+    const int own = WorkRanges::own();
     for (;;) {
-        unsigned long long b = ~0ull;
-        if (lane == 0) {
-            while (victim < 32) {
-                const int v = (own & ~3) + ((own + victim) & 3) + 4 * (victim >> 2);
-                const int vv = v & 31;
-                const size_t vbeg = (size_t)vv * per_rng;
-                const size_t vend = min(nitems, vbeg + per_rng);
-                if (vbeg < vend) {
-                    const unsigned long long base = atomicAdd(&a.wctr[vv * kCtrStride], 64ull);
-                    if (vbeg + base < vend) {
-                        b = vbeg + base;
-                        break;
-                    }
-                }
-                ++victim;
-            }
-        }
-        // every lane is active here, so the first active lane is lane 0: the
-        // fetch position and range count become scalars.  Broadcast with
-        // __shfl they stayed per-lane values: 34 instead of 26 spilled VGPRs
-        // at 8 waves/SIMD and a trace stage 0.5-2% longer on the
-        // 11k-triangle room bake, 2048 probes x 4096 rays.  (The
-        // multi-job kernel measured the same either way and keeps __shfl.)
-        b = ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(b >> 32)) << 32) |
-            (unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)b);
-        victim = __builtin_amdgcn_readfirstlane(victim);
+        const unsigned long long b = work.take(own);
         if (b == ~0ull) break;
         const size_t it = (size_t)b + lane;
         int tile, l, e;
@@ -237,6 +207,10 @@ void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far,
 {
     VLB_REQUIRE(grid % 8 == 0, VLB_ERR_INVALID, "trace grid must be a multiple of 8");
     k_zero_ctr8<<<1, 64, 0, st>>>(a.wctr);
+    // a small launch: no more workgroups than take one set of rays per wave (64
+    // probes x 1024 rays, one-shot: 230 us with a full grid asking for work,
+    // 190 with these 256 workgroups)
+    grid = std::min(grid, std::max(8, (a.ntrace * 2 + 7) / 8 * 8));
     // recording (hit ids are the same in any shadow order) and multi-bounce
     // plans keep slot-order shadows.  The multi-bounce kernel takes the
     // variant's occupancy bound like the direct one: it is bound by the latency
