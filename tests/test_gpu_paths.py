@@ -296,7 +296,7 @@ def test_first_bad_index_or_coordinate_is_named(ctx, n):
     assert ctx.scene_info(ctx.upload_scene(v, idx))["num_tris"] == n
 
 
-@pytest.mark.parametrize("P,R", [(1, 1), (1, 33), (16, 32), (17, 95), (64, 1024), (500, 2049), (1500, 4096)])
+@pytest.mark.parametrize("P,R", [(1, 1), (1, 33), (16, 32), (17, 95), (64, 1024), (64, 1056), (256, 1024), (257, 1024), (500, 2049), (1500, 4096)])
 def test_work_fetch_covers_every_ray(ctx, room, P, R):
     """Launches from one trace tile to more rounds than waves, through the
     fused kernel (small launches with fewer workgroups) and the wavefront

@@ -177,7 +177,8 @@ void apply_variant(Context& ctx, Plan& pl, uint32_t v)
 void launch_trace_stage(Plan& pl, bool record, bool count, hipStream_t st)
 {
     if (pl.wave) launch_wave(pl.args, record, count, pl.wgrid, st);
-    else launch_trace(pl.args, record, count, record || count ? 0 : pl.occ, pl.far, pl.grid, st);
+    else launch_trace(pl.args, record, count, record || count ? 0 : pl.occ, pl.far, pl.grid,
+                     pl.ctx->num_cus, st);
 }
 
 

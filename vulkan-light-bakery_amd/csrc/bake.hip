@@ -101,6 +101,39 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_trace(BakeArgs a)
     }
 }
 
+// Small launches, one fetch per wave at most: wave w takes the rays from
+// w * n on, n = 64 or fewer, so that the chip has waves to run while each
+// waits for its loads, and a wave's longest ray is the longest of fewer.  No
+// counters, and the registers of an unbounded kernel.
+__global__ __launch_bounds__(256) void k_trace_small(BakeArgs a, int n)
+{
+    __shared__ uint32_t lds[stack_words(kLdsDepth)];
+    const int tid = threadIdx.x, lane = tid & 63;
+    Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
+    TraceCount cnt;
+    uint32_t nshadow = 0;
+    const size_t it = ((size_t)blockIdx.x * 4 + (tid >> 6)) * n + lane;
+    if (lane >= n || it >= (size_t)a.ntrace * 512) return;
+    int tile, l, e;
+    tile_map(a.map, it, tile, l, e);
+    const int pg = tile / a.nchunk;
+    const int ch = tile - pg * a.nchunk;
+    const int probe = pg * 16 + (l & 15);
+    const float4 dd = a.dirs[ch * 32 + 8 * (l >> 4) + e];
+    float3 L = make_float3(0.f, 0.f, 0.f);
+    if (probe < a.P && dd.w != 0.0f) {
+        const float4 pp = a.probes[probe];
+        int hp = -1;
+        L = shade_ray<false, false, false, false>(a.sc, a.sp, make_float3(pp.x, pp.y, pp.z),
+                                                  make_float3(dd.x, dd.y, dd.z), a.tmin, a.tmax, st,
+                                                  cnt, nshadow, hp);
+    }
+    float* out = a.rad + (size_t)tile * 1536 + l * 8 + e;
+    out[0] = L.x;
+    out[512] = L.y;
+    out[1024] = L.z;
+}
+
 // ------------------------------------------------------------- projection
 // Tile = (probe group pg, slice sl): chunks sl*nch .. sl*nch + nch - 1 of the
 // group's trace tiles (consecutive in `rad`), partials of slice sl.
@@ -202,14 +235,35 @@ int trace_grid_size(Context& ctx, int occ, bool far)
     return (g + 7) & ~7;
 }
 
-void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid,
+// Rays per wave of k_trace_small for this many rays, or 0: k_trace.  Up to 4
+// waves/SIMD either way: 16 rays per wave while that makes no more waves, then
+// 64.  A bake without tables (trace, projection, merge, launches), k_trace
+// against k_trace_small: 65,536 rays in the 11k-triangle room 106 us against
+// 93 with 16 rays per wave, 98 with 32, 101 with 64; 262,144 rays 134 against
+// 121; in the 0.5M-triangle terrain 137 against 119, and 181 either way.
+// Beyond that both have the waves they can hold.
+static int small_launch(const BakeArgs& a, int num_cus)
+{
+    const long long rays = (long long)a.ntrace * 512, waves = 16ll * num_cus;
+    const int n = rays <= 16 * waves ? 16 : rays <= 64 * waves ? 64 : 0;
+    return n && (rays / n + 3) / 4 <= (long long)(a.spill_stride / 256) ? n : 0;
+}
+
+void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid, int num_cus,
                   hipStream_t st)
 {
     VLB_REQUIRE(grid % 8 == 0, VLB_ERR_INVALID, "trace grid must be a multiple of 8");
+    const bool wide = a.sc.ntris >= kNarrowTris;  // else record64's short form
+    const int per = small_launch(a, num_cus);
+    if (per && !record && !count && !far && !wide && !a.sp.ind.coeffs) {
+        k_trace_small<<<(a.ntrace * 512 / per + 3) / 4, 256, 0, st>>>(a, per);
+        VLB_HIP(hipGetLastError());
+        return;
+    }
     k_zero_ctr8<<<1, 64, 0, st>>>(a.wctr);
-    // a small launch: no more workgroups than take one set of rays per wave (64
-    // probes x 1024 rays, one-shot: 230 us with a full grid asking for work,
-    // 190 with these 256 workgroups)
+    // no more workgroups than take one set of rays per wave (64 probes x 1024
+    // rays in this kernel, one-shot: 230 us with a full grid asking for work,
+    // 190 with 256 workgroups)
     grid = std::min(grid, std::max(8, (a.ntrace * 2 + 7) / 8 * 8));
     // recording (hit ids are the same in any shadow order) and multi-bounce
     // plans keep slot-order shadows.  The multi-bounce kernel takes the
@@ -217,7 +271,6 @@ void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far,
     // and issue of its eight corner rays per hit, so 8 waves/SIMD with spills
     // outside the loops beat 3 without (2048 probes x 4096 rays of the
     // 11k-triangle room: 2.9 ms per bounce at 64 VGPRs against 4.1 at 144).
-    const bool wide = a.sc.ntris >= kNarrowTris;  // else record64's short form
     if (a.sp.ind.coeffs) {
         if (record) k_trace<true, false, 0, true><<<grid, 256, 0, st>>>(a);
         else if (count) k_trace<false, true, 0, true><<<grid, 256, 0, st>>>(a);

@@ -486,7 +486,7 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
 // bake.hip
 int  trace_grid_size(Context& ctx, int occ, bool far);
 void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid,
-                  hipStream_t stream);
+                  int num_cus, hipStream_t stream);
 void launch_project(const BakeArgs& a, int precision, int grid, hipStream_t stream);
 void launch_copy_f32(float* dst, const float* src, size_t n, hipStream_t stream);
 // wave.hip
