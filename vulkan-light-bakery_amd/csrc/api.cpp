@@ -1120,7 +1120,7 @@ vlb_status vlb_probe_lookup(vlb_ctx* h, uint32_t scene, const vlb_probe_grid_des
         VLB_HIP(hipMemcpyAsync(d_c.p, coeffs, d_c.bytes, hipMemcpyHostToDevice, c->stream));
         VLB_HIP(hipMemcpyAsync(d_p.p, points, d_p.bytes, hipMemcpyHostToDevice, c->stream));
         VLB_HIP(hipMemcpyAsync(d_n.p, normals, d_n.bytes, hipMemcpyHostToDevice, c->stream));
-        const int grid = lookup_grid_size(*c);
+        const int grid = lookup_grid_size(*c, s, n);
         const uint32_t stride = (uint32_t)grid * 256u;
         DevBuf spill = dev_alloc(*c, scene_spill_bytes(s, stride));
         LookupArgs a;

@@ -506,7 +506,7 @@ void launch_multi_trace(const MultiArgs& a, bool count, int grid, int shade_grid
 void launch_multi_project(const MultiArgs& a, int precision, int grid, hipStream_t st);
 void launch_multi_merge(const MultiArgs& a, int grid, hipStream_t st);
 // lookup.hip
-int  lookup_grid_size(Context& ctx);
+int  lookup_grid_size(Context& ctx, const Scene& sc, uint32_t n);
 void launch_lookup(const LookupArgs& a, int grid, hipStream_t st);
 // sh_image.hip
 void launch_skybox_table(int N, const float* wtab, float4* tab, hipStream_t st);
