@@ -219,7 +219,9 @@ typedef struct vlb_bake_stats {
 int32_t     vlb_abi_version(void);
 /* Replaces Application::Application (src/application.cpp:540-556): device
  * selection, queues and pools become one HIP device + one stream.
- * hbm_budget_bytes == 0 means "all free memory". */
+ * hbm_budget_bytes == 0 means "all free memory".  The context keeps freed
+ * device blocks for its next calls (at most 1/32 of the device's memory, never
+ * against a request that would not fit beside them). */
 vlb_status  vlb_ctx_create(int32_t device, uint64_t hbm_budget_bytes, vlb_ctx** out);
 /* Frees the context's scenes and device buffers.  VLB_ERR_INVALID (and
  * nothing freed) while plans, batches or servers made from it are alive:

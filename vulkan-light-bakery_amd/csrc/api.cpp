@@ -233,8 +233,8 @@ void build_plan(Context& ctx, Scene& sc, const vlb_bake_params& p, Plan& pl)
     pl.out = dev_alloc(ctx, (size_t)P * K * 3 * sizeof(float));
     pl.out64 = dev_alloc(ctx, (size_t)P * K * 3 * sizeof(double));
     pl.counters = dev_alloc(ctx, 4 * sizeof(unsigned long long));
-    // work counters of every variant: 8 per-XCD counters 128 B apart (fused),
-    // or 16 packed ones (wavefront)
+    // work counters of every variant, each on a line of its own: 32 (fused) or
+    // 16 (wavefront)
     pl.wctr = dev_alloc(ctx, 32 * kCtrStride * sizeof(unsigned long long));
 
     // ---- kernel arguments
