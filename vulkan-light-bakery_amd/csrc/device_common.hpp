@@ -164,6 +164,20 @@ struct WorkRanges {
 };
 
 // ---------------------------------------------------------------- helpers
+// The running kernel's first argument (constant memory).  Called inside a
+// persistent kernel's loop, it makes the compiler read the arguments again
+// for each set of rays, where they are used; named directly they are loaded
+// once before the loop and held in scalar registers, more than 8 waves/SIMD
+// leave, which spill into vector registers, which spill into scratch.
+template <class T>
+__device__ __forceinline__ const T& kernel_args()
+{
+    typedef const T __attribute__((address_space(4)))* P;
+    P p = (P)__builtin_amdgcn_kernarg_segment_ptr();
+    __asm__ __volatile__("" : "+s"(p));
+    return *(const T*)p;
+}
+
 __device__ __forceinline__ float dot3(const float3& a, const float3& b)
 {
     return a.x * b.x + a.y * b.y + a.z * b.z;
