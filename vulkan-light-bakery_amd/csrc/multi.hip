@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void k_rays_jobs(MultiArgs a, const JobDesc* _
 // hence one segment and one job).  Same values as the wavefront passes, bit
 // for bit.
 template <bool COUNT, int OCC, bool FAR = false, bool WIDE = COUNT>
-__global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs a,
+__global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs args,
                                                                        const JobDesc* __restrict__ jobs,
                                                                        const Segment* __restrict__ seg,
                                                                        const WorkHeader* __restrict__ hdr)
@@ -270,38 +270,18 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs
     __shared__ uint32_t lds[stack_words(kLdsDepth)];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    Stack st = make_stack(lds, kLdsDepth, a.spill + (size_t)blockIdx.x * 256 + tid, a.spill_stride);
+    Stack st = make_stack(lds, kLdsDepth, args.spill + (size_t)blockIdx.x * 256 + tid, args.spill_stride);
     TraceCount cnt;
     uint32_t nshadow = 0;
     const int nseg = hdr->nseg;
-    const size_t nitems = (size_t)hdr->ntrace * 512;
-    // 32 64-aligned ranges, range 4x + w owned by wave w of the workgroups on
-    // XCD x; a wave takes 64 items per fetch from its own range, then from
-    // its XCD's other ranges, then from the other XCDs' (nitems is a multiple
-    // of 512, so a fetched chunk is whole and lies in one pair of tiles)
-    const size_t per_rng = ((nitems + 31) / 32 + 63) / 64 * 64;
-    const int own = (blockIdx.x & 7) * 4 + (tid >> 6);
-    int victim = 0;  // ranges tried (wave-uniform)
+    // what a wave takes lies in one pair of tiles
+    __shared__ unsigned used;
+    const WorkRanges work(args.wctr, (size_t)hdr->ntrace * 512, &used);
+    const int own = WorkRanges::own();
     for (;;) {
-        unsigned long long b = ~0ull;
-        if (lane == 0) {
-            while (victim < 32) {
-                const int v = ((own & ~3) + ((own + victim) & 3) + 4 * (victim >> 2)) & 31;
-                const size_t vbeg = (size_t)v * per_rng;
-                const size_t vend = min(nitems, vbeg + per_rng);
-                if (vbeg < vend) {
-                    const unsigned long long base = atomicAdd(&a.wctr[v * kCtrStride], 64ull);
-                    if (vbeg + base < vend) {
-                        b = vbeg + base;
-                        break;
-                    }
-                }
-                ++victim;
-            }
-        }
-        b = ((unsigned long long)__shfl((unsigned)(b >> 32), 0) << 32) | (unsigned long long)__shfl((unsigned)b, 0);
-        victim = __shfl(victim, 0);
+        const unsigned long long b = work.take(own);
         if (b == ~0ull) break;
+        const MultiArgs& a = kernel_args<MultiArgs>();
         const size_t it = (size_t)b + lane;
         int tile, l, e;
         tile_map(a.map, it, tile, l, e);
@@ -324,9 +304,9 @@ __global__ __launch_bounds__(256, OCC > 0 ? OCC : 1) void k_fused_jobs(MultiArgs
         out[1024] = L.z;
     }
     if (COUNT) {
-        atomicAdd(&a.counters[0], (unsigned long long)cnt.nodes);
-        atomicAdd(&a.counters[1], (unsigned long long)cnt.tris);
-        atomicAdd(&a.counters[2], (unsigned long long)nshadow);
+        atomicAdd(&args.counters[0], (unsigned long long)cnt.nodes);
+        atomicAdd(&args.counters[1], (unsigned long long)cnt.tris);
+        atomicAdd(&args.counters[2], (unsigned long long)nshadow);
     }
 }
 
