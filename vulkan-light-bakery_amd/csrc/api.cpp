@@ -32,9 +32,14 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
     size_t step = 4096;
     while (step * 16 < bytes && step < (2u << 20)) step *= 2;
     b.cap = (bytes + step - 1) / step * step;
-    if (pooled) b.p = ctx.pool.take(bytes, b.cap);
+    // a block holds more than the bytes asked for only while all of them stay
+    // within the budget; a request is refused by the bytes asked for alone
+    const size_t room = ctx.budget ? (size_t)(ctx.budget - std::min(ctx.budget, now + ctx.slack.load()))
+                                   : ~(size_t)0;
+    if (pooled) b.p = ctx.pool.take(bytes, room, b.cap);
     if (!b.p) {
-        if (ctx.budget && now + ctx.pool.kept() + b.cap > ctx.budget) ctx.pool.trim();
+        if (b.cap > room || ctx.pool.kept() > room - b.cap) ctx.pool.trim();
+        if (b.cap > room) b.cap = bytes;
         hipError_t e = hipMalloc(&b.p, b.cap);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -50,8 +55,10 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
     }
     b.bytes = bytes;
     b.acct = &ctx.in_use;
+    b.slack = &ctx.slack;
     b.pool = pooled ? &ctx.pool : nullptr;
     ctx.in_use.fetch_add(bytes);
+    ctx.slack.fetch_add(b.cap - bytes);
     return b;
 }
 

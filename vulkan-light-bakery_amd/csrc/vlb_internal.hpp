@@ -55,12 +55,15 @@ class DevPool {
 public:
     ~DevPool() { trim(); }
     void set_limit(size_t bytes) { limit_ = bytes; }
-    // The smallest kept block of at least `bytes` and little more, or null.
-    void* take(size_t bytes, size_t& cap)
+    // The smallest kept block of at least `bytes` and little more, at most
+    // `room`, or null.
+    void* take(size_t bytes, size_t room, size_t& cap)
     {
         std::lock_guard<std::mutex> lk(mu_);
         auto it = free_.lower_bound(bytes);
-        if (it == free_.end() || it->first > bytes + bytes / 4 + (64u << 10)) return nullptr;
+        if (it == free_.end() || it->first > bytes + bytes / 4 + (64u << 10) ||
+            it->first > room)
+            return nullptr;
         void* p = it->second;
         cap = it->first;
         kept_ -= cap;
@@ -113,6 +116,7 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0, cap = 0;
     std::atomic<uint64_t>* acct = nullptr;
+    std::atomic<uint64_t>* slack = nullptr;  // counts cap - bytes
     DevPool* pool = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
@@ -133,6 +137,7 @@ struct DevBuf {
         std::swap(bytes, o.bytes);
         std::swap(cap, o.cap);
         std::swap(acct, o.acct);
+        std::swap(slack, o.slack);
         std::swap(pool, o.pool);
     }
     void release()
@@ -141,10 +146,11 @@ struct DevBuf {
             if (pool && std::uncaught_exceptions() == 0) pool->put(p, cap);
             else (void)hipFree(p);
             if (acct) acct->fetch_sub(bytes);
+            if (slack) slack->fetch_sub(cap - bytes);
         }
         p = nullptr;
         bytes = cap = 0;
-        acct = nullptr;
+        acct = slack = nullptr;
         pool = nullptr;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
@@ -193,6 +199,7 @@ struct Context {
     hipStream_t stream = nullptr;
     uint64_t budget = 0;                  // bytes
     std::atomic<uint64_t> in_use{0};      // bytes allocated through dev_alloc
+    std::atomic<uint64_t> slack{0};       // what their blocks hold beyond that
     DevPool pool;                         // before every member that holds blocks
     // message of the last failure on this context, from any thread (the
     // serving entry points may fail concurrently): written and copied out
