@@ -1,0 +1,51 @@
+"""GPU tests of what the library refuses and what it may hold: scene depth,
+bad geometry, device memory budgets and kept device blocks."""
+import numpy as np
+import pytest
+
+import orc
+import vlb
+
+pytestmark = pytest.mark.gpu
+
+
+def _concentric(n):
+    """n triangles of growing size around one centre, all of one Morton code:
+    each one's least union is with its next smaller neighbour, so one pair
+    merges per clustering pass and the tree is a chain of depth n - 1."""
+    s = 1.0 + np.arange(n) * 1e-3
+    z = np.zeros(n)
+    v = np.stack([np.stack([-s, -s, z], 1), np.stack([s, -s, z], 1), np.stack([z, s, z], 1)], 1)
+    return v.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+
+
+@pytest.mark.parametrize("n", [4096, 4097, 4098, 4099, 10_000])
+def test_trees_beyond_the_depth_limit_are_refused(ctx, n):
+    """Depth 4096 is the limit: at it a scene answers as the oracle does,
+    beyond it the upload is refused, also where the tree is several times as
+    deep, and the context goes on."""
+    xyz, idx = _concentric(n)
+    if n - 1 > 4096:
+        with pytest.raises(vlb.VlbError) as e:
+            ctx.upload_scene(xyz, idx)
+        assert e.value.status == vlb.ERR_INVALID
+        small, sidx = _concentric(100)
+        sid = ctx.upload_scene(small, sidx)
+        assert ctx.scene_info(sid)["depth"] == 99
+        ctx.release_scene(sid)
+        return
+    sid = ctx.upload_scene(xyz, idx)
+    assert ctx.scene_info(sid)["depth"] == n - 1
+    rng = np.random.default_rng(n)
+    m = 1000
+    org = np.zeros((m, 3), np.float32)
+    org[:, :2] = rng.uniform(-5, 5, (m, 2))
+    org[:, 2] = rng.choice([-1.0, 1.0], m)
+    d = np.zeros((m, 3), np.float32)
+    d[:, :2] = rng.uniform(-0.3, 0.3, (m, 2))
+    d[:, 2] = -org[:, 2]
+    got = ctx.trace_closest(sid, org, d, 0.0, 10.0)
+    ref = orc.Scene(xyz, idx, bvh=False).trace_closest(org, d, 0.0, 10.0, brute=True)
+    assert (ref[0] >= 0).any() and (ref[0] < 0).any()
+    assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
+    ctx.release_scene(sid)

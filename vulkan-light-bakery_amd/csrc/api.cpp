@@ -525,7 +525,6 @@ vlb_status vlb_scene_upload(vlb_ctx* h, const float* xyz, uint32_t nverts, const
         VLB_HIP(hipSetDevice(c->device));
         auto s = std::make_unique<Scene>();
         build_scene_bvh(*c, *s, xyz, nverts, idx, ntris, normals, albedo);
-        VLB_REQUIRE(s->depth <= 4096, VLB_ERR_INVALID, "BVH build produced a malformed tree");
         s->id = c->next_scene++;
         *out_scene = s->id;
         c->scenes[s->id] = std::move(s);

@@ -721,6 +721,9 @@ __global__ void k_single(const float4* __restrict__ clo, const float4* __restric
     lparent[0] = 0;
 }
 
+// Deepest tree (inner-node levels) a scene may have.
+constexpr int kMaxDepth = 4096;
+
 // BVH2 -> BVH4: every even-depth BVH2 node becomes a BVH4 node whose
 // children are its grandchildren through inner children, or the child itself
 // when that is a leaf (2 to 4 entries).  Per BVH2 node: its BVH4 node's inner
@@ -731,7 +734,7 @@ __global__ void k_count4(const BNode* __restrict__ n2, const int* __restrict__ i
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nin) return;
     int d = 0, p = i;
-    while (p != 0 && d < 8192) {
+    while (p != 0 && d <= kMaxDepth) {  // a deeper tree is refused before its counts are used
         p = iparent[p] >> 1;
         ++d;
     }
@@ -1076,6 +1079,12 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
     VLB_HIP(hipMemcpyAsync(hb, bnd.p, 13 * sizeof(float), hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
     VLB_REQUIRE(left.m == 1, VLB_ERR_DEVICE, "PLOC build made no progress");
+    // before anything is numbered: k_count4 tells even from odd depths only
+    // down to kMaxDepth, so a deeper tree's counts place leaves and nodes past
+    // their arrays (10,000 concentric triangles make a tree of depth 9,999)
+    VLB_REQUIRE(left.depth <= kMaxDepth, VLB_ERR_INVALID, "BVH build produced a malformed tree");
+    VLB_REQUIRE((int)((last[0] + last[1]) >> 32) == (n == 1 ? 2 : n), VLB_ERR_DEVICE,
+                "BVH build lost a leaf");
     const int n4 = 1 + (int)(uint32_t)(last[0] + last[1]);
     // node unit: the power of two that brings the largest coordinate to
     // [2^13, 2^14) units, so that offsets stay within FP16's range
