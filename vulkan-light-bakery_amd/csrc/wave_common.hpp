@@ -137,7 +137,7 @@ __device__ __forceinline__ void trav_init(TravState& T, const SceneView& sc, con
                                           const float3& d, float tmin, float tmax)
 {
     T.w = wt_setup(o, d);
-    T.s = slab_setup(o, d, wt_thin(T.w), sc.maxabs, sc.unit);
+    T.s = slab_setup(o, d, T.w, sc.maxabs, sc.unit);
     T.tmin = tmin;
     T.unit = sc.unit;
     T.tb = tmax;
