@@ -1,5 +1,7 @@
 """GPU tests of what the library refuses and what it may hold: scene depth,
 bad geometry, device memory budgets and kept device blocks."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -49,3 +51,53 @@ def test_trees_beyond_the_depth_limit_are_refused(ctx, n):
     assert (ref[0] >= 0).any() and (ref[0] < 0).any()
     assert np.array_equal(got[0], ref[0]) and np.array_equal(got[1], ref[1])
     ctx.release_scene(sid)
+
+
+def _free_bytes():
+    """Free memory of the device, as the driver sees it."""
+    free, total = C.c_size_t(), C.c_size_t()
+    assert vlb.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def _plans(c, sid, n, rays):
+    """n plans that hold 12 * 1024 * rays bytes of radiance each."""
+    probes = np.random.default_rng(1).uniform(-1, 1, (1024, 3)).astype(np.float32)
+    p = vlb.Params(probes=probes, rays=rays)
+    return [c.plan(sid, p) for _ in range(n)]
+
+
+def _fill(c):
+    """16 MiB blocks until the budget refuses one."""
+    fill = []
+    with pytest.raises(vlb.VlbError) as e:
+        while True:
+            fill.append(c.alloc(16 << 20))
+    assert e.value.status == vlb.ERR_BUDGET
+    return fill
+
+
+def test_reused_blocks_stay_within_the_budget():
+    """Blocks kept from larger buffers: a context filled to its budget through
+    them is given as much as one that kept none, and holds no more of the
+    device than the budget (and what hipMalloc rounds up to: at most 2 MiB for
+    each buffer of a mebibyte or more)."""
+    budget, room = 1200 << 20, []
+    for kept in (False, True):
+        with vlb.Context(hbm_budget=budget) as c:
+            sid = c.upload_scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32))
+            small = _plans(c, sid, 1, 64)
+            small[0].execute()
+            small[0].download()
+            before = _free_bytes()
+            for pl in _plans(c, sid, 8 if kept else 0, 8192):  # 8 x 96 MiB
+                pl.destroy()
+            plans = _plans(c, sid, 8, 6720)                    # 8 x 79 MiB
+            fill = _fill(c)
+            assert before - _free_bytes() <= budget + (48 << 20)
+            room.append(len(fill))
+            for d in fill:
+                c.free(d)
+            for pl in plans + small:
+                pl.destroy()
+    assert room[0] == room[1] > 0

@@ -27,19 +27,11 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
                                         std::to_string(now) + " of " + std::to_string(ctx.budget) +
                                         " in use)"};
     DevBuf b;
-    // capacities in steps of 1/16 (4 KiB at least, 2 MiB from 64 MiB on), so
-    // that blocks fit the next call of about the same size
-    size_t step = 4096;
-    while (step * 16 < bytes && step < (2u << 20)) step *= 2;
-    b.cap = (bytes + step - 1) / step * step;
-    // a block holds more than the bytes asked for only while all of them stay
-    // within the budget; a request is refused by the bytes asked for alone
-    const size_t room = ctx.budget ? (size_t)(ctx.budget - std::min(ctx.budget, now + ctx.slack.load()))
-                                   : ~(size_t)0;
-    if (pooled) b.p = ctx.pool.take(bytes, room, b.cap);
+    b.cap = dev_capacity(bytes);
+    if (pooled) b.p = ctx.pool.take(b.cap);
     if (!b.p) {
-        if (b.cap > room || ctx.pool.kept() > room - b.cap) ctx.pool.trim();
-        if (b.cap > room) b.cap = bytes;
+        // kept blocks make room: what is held stays within the budget
+        if (ctx.budget && ctx.pool.kept() > ctx.budget - now - bytes) ctx.pool.trim();
         hipError_t e = hipMalloc(&b.p, b.cap);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -55,10 +47,8 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
     }
     b.bytes = bytes;
     b.acct = &ctx.in_use;
-    b.slack = &ctx.slack;
     b.pool = pooled ? &ctx.pool : nullptr;
     ctx.in_use.fetch_add(bytes);
-    ctx.slack.fetch_add(b.cap - bytes);
     return b;
 }
 

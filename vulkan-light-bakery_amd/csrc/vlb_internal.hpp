@@ -44,6 +44,11 @@ struct Error {
 // Bounded (kPoolShare of the device's memory), emptied when an allocation
 // would not fit the context's budget or the device, and with the context.
 //
+// A block is taken only for requests of its own capacity (dev_capacity), so a
+// context never holds more of the device for its buffers than the same calls
+// to hipMalloc would.  (Larger blocks taken for smaller requests, up to a
+// quarter, held a tenth more than the budget once it filled up.)
+//
 // A block may come back while kernels on the context's stream still use it;
 // later work on that stream is ordered behind them.  Work on any other stream
 // (the server's, the user's) first waits for the context's stream
@@ -55,17 +60,13 @@ class DevPool {
 public:
     ~DevPool() { trim(); }
     void set_limit(size_t bytes) { limit_ = bytes; }
-    // The smallest kept block of at least `bytes` and little more, at most
-    // `room`, or null.
-    void* take(size_t bytes, size_t room, size_t& cap)
+    // A kept block of this capacity, or null.
+    void* take(size_t cap)
     {
         std::lock_guard<std::mutex> lk(mu_);
-        auto it = free_.lower_bound(bytes);
-        if (it == free_.end() || it->first > bytes + bytes / 4 + (64u << 10) ||
-            it->first > room)
-            return nullptr;
+        auto it = free_.find(cap);
+        if (it == free_.end()) return nullptr;
         void* p = it->second;
-        cap = it->first;
         kept_ -= cap;
         free_.erase(it);
         return p;
@@ -109,6 +110,16 @@ private:
 };
 constexpr size_t kPoolShare = 32;  // of the device's memory: 9 of 288 GB
 
+// What hipMalloc takes of the device for `bytes` anyway (measured: 4 KiB
+// pieces of a shared chunk below 64 KiB, 64 KiB steps to 1 MiB, 2 MiB steps
+// beyond): the capacity of a block, so that one serves all requests that cost
+// the device the same.
+inline size_t dev_capacity(size_t bytes)
+{
+    const size_t step = bytes < (64u << 10) ? 4096 : bytes <= (1u << 20) ? 64u << 10 : 2u << 20;
+    return (bytes + step - 1) / step * step;
+}
+
 // Device allocation owned by RAII; `acct` is the owning context's byte
 // counter (HBM budget admission), `pool` where the block goes back (null:
 // freed).
@@ -116,7 +127,6 @@ struct DevBuf {
     void* p = nullptr;
     size_t bytes = 0, cap = 0;
     std::atomic<uint64_t>* acct = nullptr;
-    std::atomic<uint64_t>* slack = nullptr;  // counts cap - bytes
     DevPool* pool = nullptr;
     DevBuf() = default;
     DevBuf(const DevBuf&) = delete;
@@ -137,7 +147,6 @@ struct DevBuf {
         std::swap(bytes, o.bytes);
         std::swap(cap, o.cap);
         std::swap(acct, o.acct);
-        std::swap(slack, o.slack);
         std::swap(pool, o.pool);
     }
     void release()
@@ -146,11 +155,10 @@ struct DevBuf {
             if (pool && std::uncaught_exceptions() == 0) pool->put(p, cap);
             else (void)hipFree(p);
             if (acct) acct->fetch_sub(bytes);
-            if (slack) slack->fetch_sub(cap - bytes);
         }
         p = nullptr;
         bytes = cap = 0;
-        acct = slack = nullptr;
+        acct = nullptr;
         pool = nullptr;
     }
     template <class T> T* as() const { return static_cast<T*>(p); }
@@ -199,7 +207,6 @@ struct Context {
     hipStream_t stream = nullptr;
     uint64_t budget = 0;                  // bytes
     std::atomic<uint64_t> in_use{0};      // bytes allocated through dev_alloc
-    std::atomic<uint64_t> slack{0};       // what their blocks hold beyond that
     DevPool pool;                         // before every member that holds blocks
     // message of the last failure on this context, from any thread (the
     // serving entry points may fail concurrently): written and copied out
