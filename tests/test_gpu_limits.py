@@ -101,3 +101,21 @@ def test_reused_blocks_stay_within_the_budget():
             for pl in plans + small:
                 pl.destroy()
     assert room[0] == room[1] > 0
+
+
+def test_oldest_kept_blocks_go_first():
+    """More freed than a context keeps (1/32 of the device): the blocks freed
+    last stay, not only the one that went over."""
+    total = C.c_size_t()
+    assert vlb.lib.hipMemGetInfo(C.byref(C.c_size_t()), C.byref(total)) == 0
+    limit = total.value // 32
+    with vlb.Context() as c:
+        sid = c.upload_scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32))
+        size = []
+        for share in (0.55, 0.25, 0.35):
+            rays = int(share * limit) // (12 * 1024 * 64) * 64
+            size.append(12 * 1024 * rays)
+            _plans(c, sid, 1, rays)[0].destroy()
+        held = _free_bytes()
+    kept = _free_bytes() - held
+    assert size[1] + size[2] <= kept <= limit + (64 << 20)

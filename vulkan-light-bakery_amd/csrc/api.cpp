@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <list>
 #include <numeric>
 #include <vector>
 
@@ -16,6 +17,60 @@
 using namespace vlb;
 
 namespace vlb {
+
+void* DevPool::take(size_t cap)
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    auto it = size_.upper_bound(cap);  // behind the blocks of this capacity
+    if (it == size_.begin() || (--it)->first != cap) return nullptr;
+    void* p = it->second->p;
+    age_.erase(it->second);
+    size_.erase(it);
+    kept_ -= cap;
+    return p;
+}
+void DevPool::drop_oldest(size_t keep, std::list<Block>& out)
+{
+    while (kept_ > keep) {
+        const auto first = age_.begin();
+        auto range = size_.equal_range(first->cap);
+        while (range.first->second != first) ++range.first;
+        size_.erase(range.first);
+        kept_ -= first->cap;
+        out.splice(out.end(), age_, first);
+    }
+}
+void DevPool::put(void* p, size_t cap) noexcept
+{
+    std::list<Block> out;
+    bool kept = false;
+    if (cap <= limit_) {
+        std::lock_guard<std::mutex> lk(mu_);
+        drop_oldest(limit_ - cap, out);
+        try {
+            age_.push_back({p, cap});
+            try {
+                size_.emplace(cap, std::prev(age_.end()));
+                kept_ += cap;
+                kept = true;
+            } catch (...) {
+                age_.pop_back();
+            }
+        } catch (...) {  // no host memory for the entry
+        }
+    }
+    if (!kept) (void)hipFree(p);
+    for (const Block& b : out) (void)hipFree(b.p);
+}
+void DevPool::shrink(size_t keep)
+{
+    std::list<Block> out;
+    {
+        std::lock_guard<std::mutex> lk(mu_);
+        drop_oldest(keep, out);
+    }
+    for (const Block& b : out) (void)hipFree(b.p);
+}
 
 DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
 {
@@ -31,11 +86,11 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
     if (pooled) b.p = ctx.pool.take(b.cap);
     if (!b.p) {
         // kept blocks make room: what is held stays within the budget
-        if (ctx.budget && ctx.pool.kept() > ctx.budget - now - bytes) ctx.pool.trim();
+        if (ctx.budget) ctx.pool.shrink((size_t)(ctx.budget - now - bytes));
         hipError_t e = hipMalloc(&b.p, b.cap);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            ctx.pool.trim();
+            ctx.pool.shrink(0);
             b.cap = bytes;
             e = hipMalloc(&b.p, b.cap);
         }

@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <exception>
+#include <list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -41,8 +42,9 @@ struct Error {
 // Freed device blocks of a context, kept for its next allocations: a one-shot
 // call makes and drops a dozen buffers, and hipMalloc/hipFree of them cost
 // 0.3-0.5 ms per call, 20 ms and more with a radiance buffer of gigabytes.
-// Bounded (kPoolShare of the device's memory), emptied when an allocation
-// would not fit the context's budget or the device, and with the context.
+// Bounded (kPoolShare of the device's memory, the oldest blocks go first) and
+// given back: as far as an allocation would not fit the context's budget
+// beside them, all of them when the device refuses one, and with the context.
 //
 // A block is taken only for requests of its own capacity (dev_capacity), so a
 // context never holds more of the device for its buffers than the same calls
@@ -58,55 +60,22 @@ struct Error {
 // waits for the device.
 class DevPool {
 public:
-    ~DevPool() { trim(); }
+    ~DevPool() { shrink(0); }
     void set_limit(size_t bytes) { limit_ = bytes; }
-    // A kept block of this capacity, or null.
-    void* take(size_t cap)
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        auto it = free_.find(cap);
-        if (it == free_.end()) return nullptr;
-        void* p = it->second;
-        kept_ -= cap;
-        free_.erase(it);
-        return p;
-    }
-    void put(void* p, size_t cap) noexcept
-    {
-        if (cap <= limit_) {
-            if (kept() + cap > limit_) trim();
-            try {
-                std::lock_guard<std::mutex> lk(mu_);
-                if (kept_ + cap <= limit_) {
-                    free_.emplace(cap, p);
-                    kept_ += cap;
-                    return;
-                }
-            } catch (...) {  // no host memory for the entry
-            }
-        }
-        (void)hipFree(p);
-    }
-    void trim()
-    {
-        std::multimap<size_t, void*> drop;
-        {
-            std::lock_guard<std::mutex> lk(mu_);
-            drop.swap(free_);
-            kept_ = 0;
-        }
-        for (auto& kv : drop) (void)hipFree(kv.second);
-    }
-    size_t kept()
-    {
-        std::lock_guard<std::mutex> lk(mu_);
-        return kept_;
-    }
+    void* take(size_t cap);                 // the block last kept, or null
+    void put(void* p, size_t cap) noexcept;
+    void shrink(size_t keep);               // frees the oldest beyond `keep` bytes
 
 private:
+    struct Block {
+        void* p;
+        size_t cap;
+    };
     std::mutex mu_;
-    std::multimap<size_t, void*> free_;  // capacity -> block
+    std::list<Block> age_;                                    // oldest first
+    std::multimap<size_t, std::list<Block>::iterator> size_;  // by capacity
     size_t kept_ = 0, limit_ = 0;
+    void drop_oldest(size_t keep, std::list<Block>& out);     // with mu_ held
 };
 constexpr size_t kPoolShare = 32;  // of the device's memory: 9 of 288 GB
 
