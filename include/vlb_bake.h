@@ -221,8 +221,11 @@ int32_t     vlb_abi_version(void);
  * selection, queues and pools become one HIP device + one stream.
  * hbm_budget_bytes == 0 means "all free memory".  The context keeps freed
  * device blocks for its next calls (at most 1/32 of the device's memory, never
- * against a request that would not fit beside them). */
+ * against a request of this or another context of the process that would not
+ * fit beside them); vlb_ctx_trim gives them back to the device, for other
+ * allocators and processes. */
 vlb_status  vlb_ctx_create(int32_t device, uint64_t hbm_budget_bytes, vlb_ctx** out);
+vlb_status  vlb_ctx_trim(vlb_ctx* ctx);
 /* Frees the context's scenes and device buffers.  VLB_ERR_INVALID (and
  * nothing freed) while plans, batches or servers made from it are alive:
  * destroy those first. */

@@ -119,3 +119,21 @@ def test_oldest_kept_blocks_go_first():
         held = _free_bytes()
     kept = _free_bytes() - held
     assert size[1] + size[2] <= kept <= limit + (64 << 20)
+
+
+def test_kept_blocks_are_given_back():
+    """What a context keeps is the device's again after trim(), and is no
+    reason for another context of the process to run out of memory."""
+    with vlb.Context() as c, vlb.Context(hbm_budget=1 << 50) as other:
+        sid = c.upload_scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32))
+        rays, p = 131072, vlb.Params(probes=np.zeros((8, 3), np.float32), rays=64)
+        want = c.bake(sid, p)
+        before = _free_bytes()
+        _plans(c, sid, 1, rays)[0].destroy()                  # 1.5 GiB
+        assert before - _free_bytes() >= 12 * 1024 * rays
+        c.trim()
+        assert before - _free_bytes() <= 64 << 20
+        _plans(c, sid, 1, rays)[0].destroy()
+        d = other.alloc(_free_bytes() + (512 << 20))          # a third of what is kept
+        other.free(d)
+        assert np.array_equal(c.bake(sid, p), want)

@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <list>
 #include <numeric>
+#include <set>
 #include <vector>
 
 #include "vlb_internal.hpp"
@@ -18,6 +19,34 @@ using namespace vlb;
 
 namespace vlb {
 
+namespace {
+// The process's pools.  Never destroyed: a context may outlive static objects.
+struct PoolList {
+    std::mutex mu;
+    std::set<DevPool*> pools;
+};
+PoolList& pool_list()
+{
+    static PoolList* l = new PoolList();
+    return *l;
+}
+}  // namespace
+
+DevPool::DevPool()
+{
+    PoolList& l = pool_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.pools.insert(this);
+}
+DevPool::~DevPool()
+{
+    {
+        PoolList& l = pool_list();
+        std::lock_guard<std::mutex> lk(l.mu);
+        l.pools.erase(this);
+    }
+    shrink(0);
+}
 void* DevPool::take(size_t cap)
 {
     std::lock_guard<std::mutex> lk(mu_);
@@ -71,6 +100,12 @@ void DevPool::shrink(size_t keep)
     }
     for (const Block& b : out) (void)hipFree(b.p);
 }
+void DevPool::trim_all()
+{
+    PoolList& l = pool_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    for (DevPool* p : l.pools) p->shrink(0);
+}
 
 DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
 {
@@ -90,7 +125,7 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
         hipError_t e = hipMalloc(&b.p, b.cap);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            ctx.pool.shrink(0);
+            DevPool::trim_all();
             b.cap = bytes;
             e = hipMalloc(&b.p, b.cap);
         }
@@ -1279,6 +1314,17 @@ vlb_status vlb_device_read(vlb_ctx* h, const void* src, size_t bytes, uint32_t g
             VLB_HIP(hipEventElapsedTime(&f, c->ev[0], c->ev[1]));
             *ms = f;
         }
+    });
+}
+
+vlb_status vlb_ctx_trim(vlb_ctx* h)
+{
+    if (!h) return VLB_ERR_INVALID;
+    Context* c = reinterpret_cast<Context*>(h);
+    std::lock_guard<std::recursive_mutex> lk(c->mtx);
+    return guard(c, [&] {
+        VLB_HIP(hipSetDevice(c->device));
+        c->pool.shrink(0);
     });
 }
 

@@ -44,7 +44,8 @@ struct Error {
 // 0.3-0.5 ms per call, 20 ms and more with a radiance buffer of gigabytes.
 // Bounded (kPoolShare of the device's memory, the oldest blocks go first) and
 // given back: as far as an allocation would not fit the context's budget
-// beside them, all of them when the device refuses one, and with the context.
+// beside them, all of them (every context's of the process) when the device
+// refuses one, on vlb_ctx_trim, and with the context.
 //
 // A block is taken only for requests of its own capacity (dev_capacity), so a
 // context never holds more of the device for its buffers than the same calls
@@ -60,11 +61,15 @@ struct Error {
 // waits for the device.
 class DevPool {
 public:
-    ~DevPool() { shrink(0); }
+    DevPool();
+    ~DevPool();
+    DevPool(const DevPool&) = delete;
+    DevPool& operator=(const DevPool&) = delete;
     void set_limit(size_t bytes) { limit_ = bytes; }
     void* take(size_t cap);                 // the block last kept, or null
     void put(void* p, size_t cap) noexcept;
     void shrink(size_t keep);               // frees the oldest beyond `keep` bytes
+    static void trim_all();                 // of every context in the process
 
 private:
     struct Block {

@@ -182,6 +182,7 @@ def _load(path: str = LIB_PATH) -> C.CDLL:
         "vlb_abi_version": (I32, []),
         "vlb_ctx_create": (I32, [I32, U64, P(VP)]),
         "vlb_ctx_destroy": (I32, [VP]),
+        "vlb_ctx_trim": (I32, [VP]),
         "vlb_last_error": (C.c_char_p, [VP]),
         "vlb_device_info": (I32, [VP, P(I32), C.c_char_p, SZ]),
         "vlb_debug_inject": (I32, [VP, I32, I32]),
@@ -912,6 +913,10 @@ class Context:
         return out
 
     # device memory
+    def trim(self):
+        """Gives the device memory of freed buffers, kept for the next calls, back."""
+        self._chk(lib.vlb_ctx_trim(self.h), "ctx_trim")
+
     def alloc(self, nbytes: int) -> int:
         p = C.c_void_p()
         self._chk(lib.vlb_device_alloc(self.h, nbytes, C.byref(p)), "device_alloc")
