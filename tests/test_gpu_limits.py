@@ -137,3 +137,13 @@ def test_kept_blocks_are_given_back():
         d = other.alloc(_free_bytes() + (512 << 20))          # a third of what is kept
         other.free(d)
         assert np.array_equal(c.bake(sid, p), want)
+
+
+@pytest.mark.parametrize("size", [(1 << 64) - 1, (1 << 64) - 4096, (1 << 64) - (3 << 20), 1 << 63])
+def test_requests_near_the_size_limit_are_refused(ctx, size):
+    """Sizes whose rounding to a capacity, or sum with what is in use, wraps."""
+    d = ctx.alloc(4096)
+    with pytest.raises(vlb.VlbError) as e:
+        ctx.alloc(size)
+    assert e.value.status in (vlb.ERR_BUDGET, vlb.ERR_OOM)
+    ctx.free(d)

@@ -111,13 +111,13 @@ DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
 {
     if (bytes == 0) bytes = 16;
     const uint64_t now = ctx.in_use.load();
-    if (ctx.budget && now + bytes > ctx.budget)
+    if (ctx.budget && (now > ctx.budget || bytes > ctx.budget - now))  // no sum that could wrap
         throw Error{VLB_ERR_BUDGET, "request of " + std::to_string(bytes) +
                                         " device bytes exceeds the HBM budget (" +
                                         std::to_string(now) + " of " + std::to_string(ctx.budget) +
                                         " in use)"};
     DevBuf b;
-    b.cap = dev_capacity(bytes);
+    b.cap = std::max(bytes, dev_capacity(bytes));  // bytes: where the rounding wraps
     if (pooled) b.p = ctx.pool.take(b.cap);
     if (!b.p) {
         // kept blocks make room: what is held stays within the budget
