@@ -1,6 +1,7 @@
 """GPU tests of what the library refuses and what it may hold: scene depth,
 bad geometry, device memory budgets and kept device blocks."""
 import ctypes as C
+import os
 
 import numpy as np
 import pytest
@@ -147,3 +148,20 @@ def test_requests_near_the_size_limit_are_refused(ctx, size):
         ctx.alloc(size)
     assert e.value.status in (vlb.ERR_BUDGET, vlb.ERR_OOM)
     ctx.free(d)
+
+
+def test_refused_uploads_leave_nothing_behind(ctx):
+    """Uploads refused for a bad index: the process does not grow.  (An event
+    of the HIP runtime, the smallest thing a call could leave, takes over 200
+    bytes of host memory.)"""
+    v, idx = np.zeros((3, 3), np.float32), np.array([[0, 1, 3]], np.uint32)
+
+    def refused(n):
+        for _ in range(n):
+            with pytest.raises(vlb.VlbError):
+                ctx.upload_scene(v, idx)
+        with open("/proc/self/statm") as f:
+            return int(f.read().split()[1]) * os.sysconf("SC_PAGESIZE")
+
+    before = refused(1000)
+    assert refused(5000) - before < 5000 * 200

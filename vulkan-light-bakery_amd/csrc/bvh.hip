@@ -909,6 +909,14 @@ __global__ void k_collapse(const BNode* __restrict__ n2, const unsigned long lon
 
 inline int nblk(int n, int b = 256) { return (n + b - 1) / b; }
 
+struct Event {
+    hipEvent_t e = nullptr;
+    Event() { VLB_HIP(hipEventCreate(&e)); }
+    Event(const Event&) = delete;
+    Event& operator=(const Event&) = delete;
+    ~Event() { (void)hipEventDestroy(e); }
+};
+
 }  // namespace
 
 void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
@@ -923,9 +931,6 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
         s.depth = 0;
         return;
     }
-    hipEvent_t e0, e1;
-    VLB_HIP(hipEventCreate(&e0));
-    VLB_HIP(hipEventCreate(&e1));
     // uploads
     DevBuf d_xyz = dev_alloc(ctx, (size_t)nverts * 3 * sizeof(float));
     DevBuf d_idx = dev_alloc(ctx, (size_t)n * 3 * sizeof(uint32_t));
@@ -954,7 +959,8 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
         d_alb = dev_alloc(ctx, (size_t)n * 3 * sizeof(float));
         VLB_HIP(hipMemcpyAsync(d_alb.p, albedo, d_alb.bytes, hipMemcpyHostToDevice, st));
     }
-    VLB_HIP(hipEventRecord(e0, st));
+    const Event e0, e1;
+    VLB_HIP(hipEventRecord(e0.e, st));
     DevBuf tri_raw = dev_alloc(ctx, (size_t)n * 3 * sizeof(float4));
     DevBuf lo = dev_alloc(ctx, (size_t)n * sizeof(float4));
     DevBuf hi = dev_alloc(ctx, (size_t)n * sizeof(float4));
@@ -1102,12 +1108,10 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
                                           s.leaf_prims.as<uint32_t>(), tri_raw.as<float4>(),
                                           s.nodes4.as<Node4>(), s.tris.as<float4>());
     VLB_HIP(hipGetLastError());
-    VLB_HIP(hipEventRecord(e1, st));
+    VLB_HIP(hipEventRecord(e1.e, st));
     VLB_HIP(hipStreamSynchronize(st));
     float ms = 0.0f;
-    VLB_HIP(hipEventElapsedTime(&ms, e0, e1));
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    VLB_HIP(hipEventElapsedTime(&ms, e0.e, e1.e));
     s.build_ms = ms;
     s.nnodes = nin;
     s.nnodes4 = n4;
