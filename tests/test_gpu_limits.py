@@ -165,3 +165,23 @@ def test_refused_uploads_leave_nothing_behind(ctx):
 
     before = refused(1000)
     assert refused(5000) - before < 5000 * 200
+
+
+def test_bad_geometry_is_named_where_it_does_not_fit():
+    """Geometry beyond the budget: refused for its first bad index, else its
+    first bad coordinate, else for the budget."""
+    n = 100_000
+    v = np.random.default_rng(0).uniform(-1, 1, (3 * n, 3)).astype(np.float32)
+    idx = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    with vlb.Context(hbm_budget=1 << 20) as c:
+        with pytest.raises(vlb.VlbError) as e:
+            c.upload_scene(v, idx)
+        assert e.value.status == vlb.ERR_BUDGET
+        v[70_000, 1] = np.nan
+        with pytest.raises(vlb.VlbError, match="coordinate .* at 210001$") as e:
+            c.upload_scene(v, idx)
+        assert e.value.status == vlb.ERR_INVALID
+        idx[50_000, 2] = 3 * n
+        with pytest.raises(vlb.VlbError, match="index out of range at 150002$") as e:
+            c.upload_scene(v, idx)
+        assert e.value.status == vlb.ERR_INVALID

@@ -909,6 +909,26 @@ __global__ void k_collapse(const BNode* __restrict__ n2, const unsigned long lon
 
 inline int nblk(int n, int b = 256) { return (n + b - 1) / b; }
 
+// Refuses geometry by its first bad index, else by its first bad coordinate
+// (~0: none).
+void require_good(unsigned long long bad_index, unsigned long long bad_coord)
+{
+    VLB_REQUIRE(bad_index == ~0ull, VLB_ERR_INVALID, "index out of range at " + std::to_string(bad_index));
+    // the BVH4 node grids need finite boxes of bounded magnitude
+    VLB_REQUIRE(bad_coord == ~0ull, VLB_ERR_INVALID,
+                "vertex coordinate not finite or beyond 2^100 at " + std::to_string(bad_coord));
+}
+
+// k_check on the host.
+void require_good_host(const uint32_t* idx, unsigned long long nidx, uint32_t nverts, const float* xyz,
+                       unsigned long long ncoords)
+{
+    unsigned long long bi = 0, bc = 0;
+    while (bi < nidx && idx[bi] < nverts) ++bi;
+    while (bc < ncoords && fabsf(xyz[bc]) <= 0x1p100f) ++bc;
+    require_good(bi < nidx ? bi : ~0ull, bc < ncoords ? bc : ~0ull);
+}
+
 struct Event {
     hipEvent_t e = nullptr;
     Event() { VLB_HIP(hipEventCreate(&e)); }
@@ -932,25 +952,27 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
         return;
     }
     // uploads
-    DevBuf d_xyz = dev_alloc(ctx, (size_t)nverts * 3 * sizeof(float));
-    DevBuf d_idx = dev_alloc(ctx, (size_t)n * 3 * sizeof(uint32_t));
-    DevBuf d_nrm, d_alb;
+    const unsigned long long nidx = (unsigned long long)n * 3, ncoords = (unsigned long long)nverts * 3;
+    DevBuf d_xyz, d_idx, d_nrm, d_alb, d_bad;
+    unsigned long long bad[2] = {~0ull, ~0ull};
+    try {
+        d_xyz = dev_alloc(ctx, ncoords * sizeof(float));
+        d_idx = dev_alloc(ctx, nidx * sizeof(uint32_t));
+        d_bad = dev_alloc(ctx, sizeof bad);
+    } catch (const Error&) {
+        // bad geometry is refused as such also where it does not fit
+        require_good_host(idx, nidx, nverts, xyz, ncoords);
+        throw;
+    }
     VLB_HIP(hipMemcpyAsync(d_xyz.p, xyz, d_xyz.bytes, hipMemcpyHostToDevice, st));
     VLB_HIP(hipMemcpyAsync(d_idx.p, idx, d_idx.bytes, hipMemcpyHostToDevice, st));
-    unsigned long long bad[2] = {~0ull, ~0ull};
-    DevBuf d_bad = dev_alloc(ctx, sizeof bad);
     VLB_HIP(hipMemcpyAsync(d_bad.p, bad, sizeof bad, hipMemcpyHostToDevice, st));
-    k_check<<<std::min(2048, nblk(n)), 256, 0, st>>>(d_idx.as<uint32_t>(), (unsigned long long)n * 3,
-                                                    nverts, d_xyz.as<float>(),
-                                                    (unsigned long long)nverts * 3,
-                                                    d_bad.as<unsigned long long>());
+    k_check<<<std::min(2048, nblk(n)), 256, 0, st>>>(d_idx.as<uint32_t>(), nidx, nverts, d_xyz.as<float>(),
+                                                    ncoords, d_bad.as<unsigned long long>());
     VLB_HIP(hipGetLastError());
     VLB_HIP(hipMemcpyAsync(bad, d_bad.p, sizeof bad, hipMemcpyDeviceToHost, st));
     VLB_HIP(hipStreamSynchronize(st));
-    VLB_REQUIRE(bad[0] == ~0ull, VLB_ERR_INVALID, "index out of range at " + std::to_string(bad[0]));
-    // the BVH4 node grids need finite boxes of bounded magnitude
-    VLB_REQUIRE(bad[1] == ~0ull, VLB_ERR_INVALID,
-                "vertex coordinate not finite or beyond 2^100 at " + std::to_string(bad[1]));
+    require_good(bad[0], bad[1]);
     if (normals) {
         d_nrm = dev_alloc(ctx, (size_t)nverts * 3 * sizeof(float));
         VLB_HIP(hipMemcpyAsync(d_nrm.p, normals, d_nrm.bytes, hipMemcpyHostToDevice, st));
