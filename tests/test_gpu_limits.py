@@ -185,3 +185,35 @@ def test_bad_geometry_is_named_where_it_does_not_fit():
         with pytest.raises(vlb.VlbError, match="index out of range at 150002$") as e:
             c.upload_scene(v, idx)
         assert e.value.status == vlb.ERR_INVALID
+
+
+@pytest.mark.parametrize("prec,per_ray", [(vlb.PREC_FP32, 84), (vlb.PREC_BF16, 84), (vlb.PREC_BF16_FAST, 52)])
+def test_served_direction_sets_fit_a_budget_of_their_tables(prec, per_ray):
+    """A request with a new direction set, served with no more of the budget
+    left than its tables take (16 bytes of direction, 4 of index and the basis
+    row of each ray): it is served, with the coefficients of a bake."""
+    R = 1 << 16                                   # whole slices: no padding rays
+    s = vlb.generate_scene(vlb.SCENE_ROOM, 2)
+    probes = np.random.default_rng(2).uniform([1, 0.5, 1], [9, 3.5, 9], (20, 3)).astype(np.float32)
+    p = vlb.Params(probes=probes, rays=R, precision=prec, lights=[(vlb.LIGHT_DIRECTIONAL, (0.2, -1.0, 0.1), (3.0, 3.0, 3.0))])
+    with vlb.Context() as c:
+        srv = vlb.Server(c, state_budget=1 << 22, step_rays=1 << 16, max_active=4, precision=prec)
+        want = srv.wait(srv.submit(c.upload_scene_dict(s), p))
+        srv.destroy()
+    with vlb.Context(hbm_budget=256 << 20) as c:
+        sid = c.upload_scene_dict(s)
+        srv = vlb.Server(c, state_budget=1 << 22, step_rays=1 << 16, max_active=4, precision=prec)
+        tables = c.alloc(per_ray * R)
+        fill = []
+        for size in (16 << 20, 1 << 20, 1 << 16, 1 << 12):
+            try:
+                while True:
+                    fill.append(c.alloc(size))
+            except vlb.VlbError as e:
+                assert e.status == vlb.ERR_BUDGET
+        c.free(tables)                            # room for them and at most 4095 bytes
+        got = srv.wait(srv.submit(sid, p))
+        srv.destroy()
+        for d in fill:
+            c.free(d)
+    assert np.array_equal(got[0], want[0])

@@ -59,50 +59,44 @@ __device__ uint32_t direction_key(float x, float y, float z)
     return d;
 }
 
-// fibonacci_dirs: y_i = 1 - (2i+1)/R, phi_i = i * pi * (3 - sqrt 5).
-__global__ __launch_bounds__(256) void k_dirs_fibonacci(uint32_t R, double golden, double two_pi,
-                                                        float* __restrict__ xyz,
-                                                        uint32_t* __restrict__ key,
-                                                        uint32_t* __restrict__ val)
-{
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= R) return;
-    const double y = 1.0 - (2.0 * i + 1.0) / (double)R;
-    const double r = sqrt(fmax(0.0, 1.0 - y * y));
-    // fmod(i * golden, two_pi): the remainder is representable, so one FMA
-    // gives it exactly once the quotient is right
-    const double a = (double)i * golden;
-    double q = trunc(a / two_pi);
-    double phi = fma(-q, two_pi, a);
-    if (phi < 0.0) phi = fma(-(q - 1.0), two_pi, a);
-    else if (phi >= two_pi) phi = fma(-(q + 1.0), two_pi, a);
-    const float x = (float)(r * cos(phi)), z = (float)(r * sin(phi));
-    xyz[3 * (size_t)i + 0] = x;
-    xyz[3 * (size_t)i + 1] = (float)y;
-    xyz[3 * (size_t)i + 2] = z;
-    key[i] = direction_key(x, (float)y, z);
-    val[i] = i;
-}
+// How the directions of a set are made, by their canonical index.
+struct DirGen {
+    double golden, two_pi;                  // FIBONACCI (cols null)
+    uint32_t R, W;
+    const float2* cols;                     // EQUIRECT: (cos, sin) of phi_x,
+    const float2* rows;                     // (sin, cos) of theta_y
+};
 
-// equirect_dirs: cols[x] = (cos, sin) of phi_x, rows[y] = (sin, cos) of theta_y.
-__global__ __launch_bounds__(256) void k_dirs_equirect(uint32_t W, uint32_t R,
-                                                       const float2* __restrict__ cols,
-                                                       const float2* __restrict__ rows,
-                                                       float* __restrict__ xyz,
-                                                       uint32_t* __restrict__ key,
-                                                       uint32_t* __restrict__ val)
+__device__ __forceinline__ float3 direction(const DirGen& g, uint32_t i)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= R) return;
-    const uint32_t py = i / W;
-    const float2 cp = cols[i - py * W], st = rows[py];
+    if (!g.cols) {
+        // fibonacci_dirs: y_i = 1 - (2i+1)/R, phi_i = i * pi * (3 - sqrt 5)
+        const double y = 1.0 - (2.0 * i + 1.0) / (double)g.R;
+        const double r = sqrt(fmax(0.0, 1.0 - y * y));
+        // fmod(i * golden, two_pi): the remainder is representable, so one FMA
+        // gives it exactly once the quotient is right
+        const double a = (double)i * g.golden;
+        const double q = trunc(a / g.two_pi);
+        double phi = fma(-q, g.two_pi, a);
+        if (phi < 0.0) phi = fma(-(q - 1.0), g.two_pi, a);
+        else if (phi >= g.two_pi) phi = fma(-(q + 1.0), g.two_pi, a);
+        return make_float3((float)(r * cos(phi)), (float)y, (float)(r * sin(phi)));
+    }
+    // equirect_dirs
+    const uint32_t py = i / g.W;
+    const float2 cp = g.cols[i - py * g.W], st = g.rows[py];
     const float a = st.x * cp.x, b = st.x * cp.y, c = st.y;
     const float l = sqrtf(a * a + b * b + c * c);
-    const float x = a / l, y = c / l, z = b / l;
-    xyz[3 * (size_t)i + 0] = x;
-    xyz[3 * (size_t)i + 1] = y;
-    xyz[3 * (size_t)i + 2] = z;
-    key[i] = direction_key(x, y, z);
+    return make_float3(a / l, c / l, b / l);
+}
+
+__global__ __launch_bounds__(256) void k_ray_keys(DirGen g, uint32_t* __restrict__ key,
+                                                  uint32_t* __restrict__ val)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= g.R) return;
+    const float3 d = direction(g, i);
+    key[i] = direction_key(d.x, d.y, d.z);
     val[i] = i;
 }
 
@@ -119,16 +113,14 @@ __device__ __forceinline__ uint16_t bf16_bits(float f)
     return (uint16_t)(u >> 16);
 }
 
-// Sorted ray r: its direction, canonical index and row of the basis table
-// ([ray octet][coefficient][ray], times the ray's weight over wref); zeros for
-// padding rays and unused coefficients.
-__global__ __launch_bounds__(256) void k_ray_rows(uint32_t R, uint32_t Rpad, int K, int precision,
-                                                  uint32_t W, const float* __restrict__ row_weight,
-                                                  float weight, double wref, ShConst c,
-                                                  const float* __restrict__ xyz,
-                                                  const uint32_t* __restrict__ order,
-                                                  float4* __restrict__ dirs, int* __restrict__ perm,
-                                                  void* __restrict__ ytab)
+// Sorted ray r (canonical index perm[r]; 0 is written for padding rays): its
+// direction, made once more, and its row of the basis table ([ray octet]
+// [coefficient][ray], times the ray's weight over wref); zeros for padding
+// rays.
+__global__ __launch_bounds__(256) void k_ray_rows(DirGen g, uint32_t Rpad, int K, int precision,
+                                                  const float* __restrict__ row_weight, float weight,
+                                                  double wref, ShConst c, float4* __restrict__ dirs,
+                                                  int* __restrict__ perm, void* __restrict__ ytab)
 {
     const uint32_t r = blockIdx.x * 256u + threadIdx.x;
     if (r >= Rpad) return;
@@ -136,12 +128,11 @@ __global__ __launch_bounds__(256) void k_ray_rows(uint32_t R, uint32_t Rpad, int
     double v[16];
 #pragma unroll
     for (int k = 0; k < 16; ++k) v[k] = 0.0;
-    int canon = 0;
-    if (r < R) {
-        const uint32_t i = order[r];
-        canon = (int)i;
-        d4 = make_float4(xyz[3 * (size_t)i], xyz[3 * (size_t)i + 1], xyz[3 * (size_t)i + 2], 1.0f);
-        const float w = row_weight ? row_weight[i / W] : weight;
+    if (r < g.R) {
+        const uint32_t i = (uint32_t)perm[r];
+        const float3 d = direction(g, i);
+        d4 = make_float4(d.x, d.y, d.z, 1.0f);
+        const float w = row_weight ? row_weight[i / g.W] : weight;
         const double wr = (double)w / wref;
         // SH frame: world (x, z, y); order of terms as shaders/sh_common.h:26-152
         const double x = d4.x, y = d4.z, z = d4.y;
@@ -165,9 +156,10 @@ __global__ __launch_bounds__(256) void k_ray_rows(uint32_t R, uint32_t Rpad, int
         }
 #pragma unroll
         for (int k = 0; k < 16; ++k) v[k] *= wr;
+    } else {
+        perm[r] = 0;
     }
     dirs[r] = d4;
-    perm[r] = canon;
     const size_t at = (size_t)(r >> 3) * 128 + (r & 7);
     const size_t lo = (size_t)Rpad * 16;
     const bool bf = precision == VLB_PREC_BF16 || precision == VLB_PREC_BF16_FAST;
@@ -314,32 +306,6 @@ void build_ray_table(Context& ctx, const vlb_bake_params& p, int K, uint32_t RS,
     const bool is16 = p.precision != VLB_PREC_FP32;
     const bool split = p.precision == VLB_PREC_BF16 || p.precision == VLB_PREC_FP16;
 
-    DevBuf xyz = dev_alloc(ctx, (size_t)R * 3 * sizeof(float));
-    SortBufs s(ctx, R, 32);
-    DevBuf trig, roww;
-    float weight = 0.0f;
-    uint32_t W = 1;
-    if (p.dir_mode == VLB_DIRS_FIBONACCI) {
-        weight = (float)(4.0 * M_PI / R);
-        k_dirs_fibonacci<<<blocks(R), 256, 0, st>>>(R, M_PI * (3.0 - sqrt(5.0)), 2.0 * M_PI, xyz.as<float>(),
-                                                    s.key.as<uint32_t>(), s.val.as<uint32_t>());
-    } else {
-        W = p.equirect_w;
-        std::vector<float2> tab(W + p.equirect_h);
-        std::vector<float> wrow(p.equirect_h);
-        equirect_angles(W, p.equirect_h, tab.data(), wrow.data());
-        trig = upload_vec(ctx, tab);
-        roww = upload_vec(ctx, wrow);
-        k_dirs_equirect<<<blocks(R), 256, 0, st>>>(W, R, trig.as<float2>(), trig.as<float2>() + W,
-                                                   xyz.as<float>(), s.key.as<uint32_t>(),
-                                                   s.val.as<uint32_t>());
-        VLB_HIP(hipStreamSynchronize(st));  // tab and wrow are read
-    }
-    VLB_HIP(hipGetLastError());
-    s.sort(R, 32, st);
-    double c[10];
-    sh_constants(p.sh_constants == VLB_SH_EXACT, c);
-    const ShConst sc{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[8], c[9]};
     t.R = R;
     t.RS = RS;
     t.Rpad = Rpad;
@@ -350,9 +316,49 @@ void build_ray_table(Context& ctx, const vlb_bake_params& p, int K, uint32_t RS,
     t.dirs = dev_alloc(ctx, (size_t)Rpad * sizeof(float4));
     t.dir_perm = dev_alloc(ctx, (size_t)Rpad * sizeof(int));
     t.ytab = dev_alloc(ctx, (size_t)Rpad * 16 * (is16 ? sizeof(uint16_t) * (split ? 2 : 1) : sizeof(float)));
-    k_ray_rows<<<blocks(Rpad), 256, 0, st>>>(R, Rpad, K, p.precision, W, roww.as<float>(), weight, wref, sc,
-                                             xyz.as<float>(), s.val2.as<uint32_t>(), t.dirs.as<float4>(),
-                                             t.dir_perm.as<int>(), t.ytab.p);
+
+    // The sort's scratch is the basis table's memory, written last, and its
+    // result the permutation: a table needs no more of the budget than itself
+    // (but for the angles of an equirect grid).
+    auto a256 = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t part = a256((size_t)R * 4);
+    uint32_t *key = nullptr, *val = nullptr, *key2 = nullptr, *order = t.dir_perm.as<uint32_t>();
+    size_t tmp_bytes = 0;
+    VLB_HIP(rocprim::radix_sort_pairs(nullptr, tmp_bytes, key, key2, val, order, (size_t)R, 0, 32, st));
+    DevBuf more;
+    uint8_t* scratch = t.ytab.as<uint8_t>();
+    if (3 * part + tmp_bytes > t.ytab.bytes) {  // a few dozen rays
+        more = dev_alloc(ctx, 3 * part + tmp_bytes);
+        scratch = more.as<uint8_t>();
+    }
+    key = reinterpret_cast<uint32_t*>(scratch);
+    val = reinterpret_cast<uint32_t*>(scratch + part);
+    key2 = reinterpret_cast<uint32_t*>(scratch + 2 * part);
+
+    DirGen g{M_PI * (3.0 - sqrt(5.0)), 2.0 * M_PI, R, 1, nullptr, nullptr};
+    DevBuf trig, roww;
+    float weight = 0.0f;
+    if (p.dir_mode == VLB_DIRS_FIBONACCI) {
+        weight = (float)(4.0 * M_PI / R);
+    } else {
+        g.W = p.equirect_w;
+        std::vector<float2> tab((size_t)g.W + p.equirect_h);
+        std::vector<float> wrow(p.equirect_h);
+        equirect_angles(g.W, p.equirect_h, tab.data(), wrow.data());
+        trig = upload_vec(ctx, tab);
+        roww = upload_vec(ctx, wrow);
+        g.cols = trig.as<float2>();
+        g.rows = g.cols + g.W;
+        VLB_HIP(hipStreamSynchronize(st));  // tab and wrow are read
+    }
+    k_ray_keys<<<blocks(R), 256, 0, st>>>(g, key, val);
+    VLB_HIP(hipGetLastError());
+    VLB_HIP(rocprim::radix_sort_pairs(scratch + 3 * part, tmp_bytes, key, key2, val, order, (size_t)R, 0, 32, st));
+    double c[10];
+    sh_constants(p.sh_constants == VLB_SH_EXACT, c);
+    const ShConst sc{c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7], c[8], c[9]};
+    k_ray_rows<<<blocks(Rpad), 256, 0, st>>>(g, Rpad, K, p.precision, roww.as<float>(), weight, wref, sc,
+                                             t.dirs.as<float4>(), t.dir_perm.as<int>(), t.ytab.p);
     VLB_HIP(hipGetLastError());
 }
 
