@@ -183,7 +183,10 @@ typedef struct vlb_bake_params {
                                       /*   idle lanes; 25..36 as 1..12 with  */
                                       /*   shadow rays visiting BVH children */
                                       /*   far first (same results); 0 =     */
-                                      /*   autotuned choice, else 12         */
+                                      /*   autotuned choice, else 12, or for */
+                                      /*   direct light and few rays (up to  */
+                                      /*   1024 per compute unit) a kernel   */
+                                      /*   for small launches                */
     uint32_t         reserved[2];
 } vlb_bake_params;
 
@@ -208,7 +211,8 @@ typedef struct vlb_bake_stats {
     double   merge_ms;         /* FP64 merge kernel     /  timed executes */
     double   total_ms;         /* whole execute on the device             */
     uint32_t tiles;
-    uint32_t grid;
+    uint32_t grid;             /* trace kernel's workgroups: the variant's */
+                               /* own, after an execute those launched  */
     uint32_t rays_per_slice;
     uint32_t slices;
     uint32_t timed_runs;       /* executes averaged (since set_timing(1)) */
@@ -306,7 +310,9 @@ vlb_status  vlb_plan_count(vlb_plan* plan);
  * bounds x shadow order, and the wavefront kernels) on this plan's real
  * workload, `iters` runs each, keeps the fastest
  * for the plan and remembers it for later plans on the same scene and ray
- * count.  *chosen (may be NULL) receives the trace_variant picked. */
+ * count.  *chosen (may be NULL) receives the trace_variant picked; 12 where
+ * it is the library's kernel for small launches (nothing is remembered then:
+ * plans left at 0 run it by themselves). */
 vlb_status  vlb_plan_autotune(vlb_plan* plan, uint32_t iters, uint32_t* chosen);
 vlb_status  vlb_plan_stats(vlb_plan* plan, vlb_bake_stats* out);
 vlb_status  vlb_plan_destroy(vlb_plan* plan);

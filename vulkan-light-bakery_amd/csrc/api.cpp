@@ -260,14 +260,20 @@ void apply_variant(Context& ctx, Plan& pl, uint32_t v)
     }
 }
 
-// The trace + shade stage of the plan's variant.
+// The trace + shade stage of the plan's variant.  Small launches have a kernel
+// of their own where the variant is left to the library; one that the caller
+// or an autotuner picked is what runs.
 void launch_trace_stage(Plan& pl, bool record, bool count, hipStream_t st)
 {
-    if (pl.wave) launch_wave(pl.args, record, count, pl.wgrid, st);
-    else launch_trace(pl.args, record, count, record || count ? 0 : pl.occ, pl.far, pl.grid,
-                     pl.ctx->num_cus, st);
+    if (pl.wave) {
+        launch_wave(pl.args, record, count, pl.wgrid, st);
+        return;
+    }
+    const int per = pl.default_variant ? trace_small_launch(pl.args, pl.ctx->num_cus) : 0;
+    const int grid = launch_trace(pl.args, record, count, record || count ? 0 : pl.occ, pl.far, pl.grid,
+                                  per, st);
+    if (!record && !count) pl.stats.grid = (uint32_t)grid;
 }
-
 
 
 void build_plan(Context& ctx, Scene& sc, const vlb_bake_params& p, Plan& pl)
@@ -906,9 +912,8 @@ vlb_status vlb_plan_autotune(vlb_plan* h, uint32_t iters, uint32_t* chosen)
         const uint32_t cand[] = {1,  2,  3,  4,  7,  8,  11, 12, 25, 26, 27, 28,
                                  31, 32, 35, 36, 13, 14, 15, 16, 19, 20, 23, 24};
         double best = 1e30;
-        uint32_t best_v = pl->variant;
-        for (uint32_t v : cand) {
-            apply_variant(c, *pl, v);
+        uint32_t best_v = kFusedDefault;
+        const auto time_stage = [&] {
             launch_trace_stage(*pl, false, false, st);  // warm-up
             VLB_HIP(hipEventRecord(e0, st));
             for (uint32_t i = 0; i < iters; ++i) launch_trace_stage(*pl, false, false, st);
@@ -916,18 +921,35 @@ vlb_status vlb_plan_autotune(vlb_plan* h, uint32_t iters, uint32_t* chosen)
             VLB_HIP(hipEventSynchronize(e1));
             float ms = 0.f;
             VLB_HIP(hipEventElapsedTime(&ms, e0, e1));
-            if (ms < best) {
-                best = ms;
+            if (!(ms < best)) return false;
+            best = ms;
+            return true;
+        };
+        // a small launch: the library's own choice is one more candidate
+        apply_variant(c, *pl, best_v);
+        const bool own = trace_small_launch(pl->args, c.num_cus) != 0;
+        pl->default_variant = own;
+        if (own) (void)time_stage();
+        bool keep = own;
+        pl->default_variant = false;
+        for (uint32_t v : cand) {
+            apply_variant(c, *pl, v);
+            if (time_stage()) {
                 best_v = v;
+                keep = false;
             }
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         apply_variant(c, *pl, best_v);
-        pl->default_variant = false;
+        pl->default_variant = keep;
         // a pick made with the indirect term on does not carry over to
         // direct-only plans of the scene
-        if (!pl->indirect) c.tuned[{pl->scene->id, (uint32_t)pl->args.R}] = best_v;
+        if (!pl->indirect) {
+            const std::pair<uint32_t, uint32_t> key{pl->scene->id, (uint32_t)pl->args.R};
+            if (keep) c.tuned.erase(key);
+            else c.tuned[key] = best_v;
+        }
         if (chosen) *chosen = best_v;
     });
 }

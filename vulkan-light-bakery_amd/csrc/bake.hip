@@ -247,23 +247,24 @@ int trace_grid_size(Context& ctx, int occ, bool far)
 // 93 with 16 rays per wave, 98 with 32, 101 with 64; 262,144 rays 134 against
 // 121; in the 0.5M-triangle terrain 137 against 119, and 181 either way.
 // Beyond that both have the waves they can hold.
-static int small_launch(const BakeArgs& a, int num_cus)
+int trace_small_launch(const BakeArgs& a, int num_cus)
 {
     const long long rays = (long long)a.ntrace * 512, waves = 16ll * num_cus;
+    if (a.sc.ntris >= kNarrowTris || a.sp.ind.coeffs) return 0;
     const int n = rays <= 16 * waves ? 16 : rays <= 64 * waves ? 64 : 0;
     return n && (rays / n + 3) / 4 <= (long long)(a.spill_stride / 256) ? n : 0;
 }
 
-void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid, int num_cus,
-                  hipStream_t st)
+int launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid, int per,
+                 hipStream_t st)
 {
     VLB_REQUIRE(grid % 8 == 0, VLB_ERR_INVALID, "trace grid must be a multiple of 8");
     const bool wide = a.sc.ntris >= kNarrowTris;  // else record64's short form
-    const int per = small_launch(a, num_cus);
-    if (per && !record && !count && !far && !wide && !a.sp.ind.coeffs) {
-        k_trace_small<<<(a.ntrace * 512 / per + 3) / 4, 256, 0, st>>>(a, per);
+    if (per && !record && !count) {
+        grid = (a.ntrace * 512 / per + 3) / 4;
+        k_trace_small<<<grid, 256, 0, st>>>(a, per);
         VLB_HIP(hipGetLastError());
-        return;
+        return grid;
     }
     k_zero_ctr8<<<1, 64, 0, st>>>(a.wctr);
     // no more workgroups than take one set of rays per wave (64 probes x 1024
@@ -295,6 +296,7 @@ void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far,
     else if (occ == 6) k_trace<false, false, 6, false><<<grid, 256, 0, st>>>(a);
     else k_trace<false, false, 0, false><<<grid, 256, 0, st>>>(a);
     VLB_HIP(hipGetLastError());
+    return grid;
 }
 
 void launch_project(const BakeArgs& a, int precision, int grid, hipStream_t st)

@@ -473,8 +473,12 @@ void build_scene_bvh(Context& ctx, Scene& s, const float* xyz, uint32_t nverts,
                      const float* albedo);
 // bake.hip
 int  trace_grid_size(Context& ctx, int occ, bool far);
-void launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid,
-                  int num_cus, hipStream_t stream);
+// Rays per wave of the kernel for small launches, or 0 where it does not
+// apply (launch_trace's `per`).
+int  trace_small_launch(const BakeArgs& a, int num_cus);
+// Returns the workgroups launched.
+int  launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid, int per,
+                  hipStream_t stream);
 void launch_project(const BakeArgs& a, int precision, int grid, hipStream_t stream);
 void launch_copy_f32(float* dst, const float* src, size_t n, hipStream_t stream);
 // wave.hip
