@@ -109,3 +109,18 @@ def test_autotuned_small_plans(ctx, room):
         if grid == own:
             assert v == 12
     assert _run(ctx, sid, _params(64, 1024, trace_variant=12))[1] != own
+
+
+@pytest.mark.parametrize("P,R", [(16, 64), (64, 1024), (65, 1024), (128, 1024), (129, 1024), (256, 1024), (257, 1024)])
+def test_small_launches_by_their_size(ctx, P, R):
+    """The library's choice around the sizes where its rays per wave change:
+    16, 32 or 64, the fewest that make at most 16 waves per compute unit (4
+    workgroups), then the ordinary kernel."""
+    sid = ctx.upload_scene_dict(vlb.generate_scene(vlb.SCENE_ROOM, 2))   # a scene no autotuner has seen
+    rays, cus = _tiles(P, R) * 512, ctx.device_info()["num_cus"]
+    per = next((n for n in (16, 32, 64) if rays <= n * 16 * cus), None)
+    got, grid = _run(ctx, sid, _params(P, R))
+    ref, ordinary = _run(ctx, sid, _params(P, R, trace_variant=12))
+    ctx.release_scene(sid)
+    assert grid == (-(-rays // (4 * per)) if per else ordinary)
+    assert np.array_equal(_bits(got), _bits(ref))

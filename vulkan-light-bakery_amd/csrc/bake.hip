@@ -240,18 +240,21 @@ int trace_grid_size(Context& ctx, int occ, bool far)
     return (g + 7) & ~7;
 }
 
-// Rays per wave of k_trace_small for this many rays, or 0: k_trace.  Up to 4
-// waves/SIMD either way: 16 rays per wave while that makes no more waves, then
-// 64.  A bake without tables (trace, projection, merge, launches), k_trace
-// against k_trace_small: 65,536 rays in the 11k-triangle room 106 us against
-// 93 with 16 rays per wave, 98 with 32, 101 with 64; 262,144 rays 134 against
-// 121; in the 0.5M-triangle terrain 137 against 119, and 181 either way.
-// Beyond that both have the waves they can hold.
+// Rays per wave of k_trace_small for this many rays, or 0: k_trace.  The
+// fewest of 16, 32 and 64 that make no more than 4 waves/SIMD; beyond 64 both
+// kernels have the waves they can hold.  Trace, projection and merge of a
+// repeated bake in us, k_trace | 16 | 32 | 64 rays per wave:
+//   rays      11k-triangle room       0.5M terrain            2M city
+//    65,536   106 |  91 |  97 | 100   132 | 117 | 124 | 124   100 |  91 |  84 |  91
+//    98,304   123 | 112 | 114 | 120   144 | 142 | 130 | 138   107 | 110 |  96 |  98
+//   131,072   110 | 117 | 110 | 101   162 | 145 | 149 | 152   115 | 128 | 104 | 105
+//   196,608   121 |   - | 117 | 110   181 |   - | 172 | 169   118 |   - | 117 | 109
+//   262,144   132 |   - | 138 | 115   179 |   - | 180 | 179   122 |   - | 140 | 111
 int trace_small_launch(const BakeArgs& a, int num_cus)
 {
     const long long rays = (long long)a.ntrace * 512, waves = 16ll * num_cus;
     if (a.sc.ntris >= kNarrowTris || a.sp.ind.coeffs) return 0;
-    const int n = rays <= 16 * waves ? 16 : rays <= 64 * waves ? 64 : 0;
+    const int n = rays <= 16 * waves ? 16 : rays <= 32 * waves ? 32 : rays <= 64 * waves ? 64 : 0;
     return n && (rays / n + 3) / 4 <= (long long)(a.spill_stride / 256) ? n : 0;
 }
 
