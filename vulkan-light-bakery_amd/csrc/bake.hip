@@ -258,6 +258,15 @@ int trace_small_launch(const BakeArgs& a, int num_cus)
     return n && (rays / n + 3) / 4 <= (long long)(a.spill_stride / 256) ? n : 0;
 }
 
+// k_trace at the occupancy bound `occ`.
+template <bool IND, bool FAR, bool WIDE>
+static void launch_occ(const BakeArgs& a, int occ, int grid, hipStream_t st)
+{
+    if (occ == 8) k_trace<false, false, 8, IND, FAR, WIDE><<<grid, 256, 0, st>>>(a);
+    else if (occ == 6) k_trace<false, false, 6, IND, FAR, WIDE><<<grid, 256, 0, st>>>(a);
+    else k_trace<false, false, 0, IND, FAR, WIDE><<<grid, 256, 0, st>>>(a);
+}
+
 int launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, int grid, int per,
                  hipStream_t st)
 {
@@ -280,24 +289,24 @@ int launch_trace(const BakeArgs& a, bool record, bool count, int occ, bool far, 
     // and issue of its eight corner rays per hit, so 8 waves/SIMD with spills
     // outside the loops beat 3 without (2048 probes x 4096 rays of the
     // 11k-triangle room: 2.9 ms per bounce at 64 VGPRs against 4.1 at 144).
-    if (a.sp.ind.coeffs) {
-        if (record) k_trace<true, false, 0, true><<<grid, 256, 0, st>>>(a);
-        else if (count) k_trace<false, true, 0, true><<<grid, 256, 0, st>>>(a);
-        else if (wide) k_trace<false, false, 0, true, false, true><<<grid, 256, 0, st>>>(a);
-        else if (occ == 8) k_trace<false, false, 8, true><<<grid, 256, 0, st>>>(a);
-        else if (occ == 6) k_trace<false, false, 6, true><<<grid, 256, 0, st>>>(a);
-        else k_trace<false, false, 0, true><<<grid, 256, 0, st>>>(a);
-    } else if (record) k_trace<true, false, 0, false><<<grid, 256, 0, st>>>(a);
-    else if (count && far) k_trace<false, true, 0, false, true><<<grid, 256, 0, st>>>(a);
-    else if (count) k_trace<false, true, 0, false><<<grid, 256, 0, st>>>(a);
-    else if (wide) k_trace<false, false, 0, false, false, true><<<grid, 256, 0, st>>>(a);
-    else if (far) {
-        if (occ == 8) k_trace<false, false, 8, false, true><<<grid, 256, 0, st>>>(a);
-        else if (occ == 6) k_trace<false, false, 6, false, true><<<grid, 256, 0, st>>>(a);
-        else k_trace<false, false, 0, false, true><<<grid, 256, 0, st>>>(a);
-    } else if (occ == 8) k_trace<false, false, 8, false><<<grid, 256, 0, st>>>(a);
-    else if (occ == 6) k_trace<false, false, 6, false><<<grid, 256, 0, st>>>(a);
-    else k_trace<false, false, 0, false><<<grid, 256, 0, st>>>(a);
+    const bool ind = a.sp.ind.coeffs != nullptr;
+    if (record) {
+        if (ind) k_trace<true, false, 0, true><<<grid, 256, 0, st>>>(a);
+        else k_trace<true, false, 0, false><<<grid, 256, 0, st>>>(a);
+    } else if (count) {
+        if (ind) k_trace<false, true, 0, true><<<grid, 256, 0, st>>>(a);
+        else if (far) k_trace<false, true, 0, false, true><<<grid, 256, 0, st>>>(a);
+        else k_trace<false, true, 0, false><<<grid, 256, 0, st>>>(a);
+    } else if (ind) {
+        if (wide) launch_occ<true, false, true>(a, occ, grid, st);
+        else launch_occ<true, false, false>(a, occ, grid, st);
+    } else if (far) {
+        if (wide) launch_occ<false, true, true>(a, occ, grid, st);
+        else launch_occ<false, true, false>(a, occ, grid, st);
+    } else {
+        if (wide) launch_occ<false, false, true>(a, occ, grid, st);
+        else launch_occ<false, false, false>(a, occ, grid, st);
+    }
     VLB_HIP(hipGetLastError());
     return grid;
 }

@@ -126,6 +126,7 @@ void round_add(RoundTable& r, int job, const JobState& js, int pt0, int npt)
     r.hdr.ntrace += npt * js.nch;
     r.hdr.nproj += npt;
     r.hdr.nvis = std::max(r.hdr.nvis, js.desc.nvis);
+    r.wide = r.wide || js.desc.sc.ntris >= kNarrowTris;
     // primary rays of these tiles (padding probes and rays excluded)
     const int nsl = js.rt->nslices;
     for (int pt = pt0; pt < pt0 + npt; ++pt) {
@@ -206,7 +207,7 @@ void RoundBufs::alloc(Context& ctx, size_t cap, int nv, uint32_t dep)
 }
 
 MultiArgs RoundBufs::args(const JobDesc* jobs, const uint8_t* table, const size_t off[3], int map,
-                          int refill, int chunk, int focc, bool far) const
+                          int refill, int chunk, int focc, bool far, bool wide) const
 {
     MultiArgs a;
     memset(&a, 0, sizeof a);
@@ -312,7 +313,8 @@ struct Batch {
     {
         const size_t off[3] = {round_off[r] + parts[r][0], round_off[r] + parts[r][1],
                                round_off[r] + parts[r][2]};
-        return rb.args(jobtab.as<JobDesc>(), table.as<uint8_t>(), off, map, refill, chunk, focc, far);
+        return rb.args(jobtab.as<JobDesc>(), table.as<uint8_t>(), off, map, refill, chunk, focc, far,
+                       rounds[r].wide);
     }
     // E: kset() events to record around the kernels, or null
     void launch_all(bool count, hipStream_t st, hipEvent_t* E = nullptr)
@@ -481,7 +483,6 @@ void build_batch(Context& ctx, const vlb_batch_job* jobs, uint32_t njobs, const 
     }
     b.table = upload_vec(ctx, host);
     b.rb.alloc(ctx, std::max<size_t>(peak, 2), nvis, depth);
-    for (const Scene* sc : b.scenes) b.rb.wide = b.rb.wide || sc->ntris >= kNarrowTris;
     b.ev.assign(2 * Batch::kRing, nullptr);
     for (auto& e : b.ev) VLB_HIP(hipEventCreate(&e));
     b.info.jobs = njobs;
@@ -648,7 +649,7 @@ vlb_status vlb_batch_autotune(vlb_batch* h, uint32_t iters, uint32_t* variant, u
                 bool far;
                 multi_variant(v, map, refill, focc, far);
                 const MultiArgs a = b->rb.args(b->jobtab.as<JobDesc>(), tab.as<uint8_t>(), off, map,
-                                               refill, ch, focc, far);
+                                               refill, ch, focc, far, smp.wide);
                 launch_multi_trace(a, false, b->rb.grid, b->rb.shade_grid, st);  // warm-up
                 VLB_HIP(hipEventRecord(e0, st));
                 for (uint32_t i = 0; i < iters; ++i)

@@ -388,7 +388,8 @@ struct TraceCount {
 // WIDE: any scene.  Without it the byte offset is kept in 32 bits, the form
 // the vector loads take next to a scalar base (one instruction instead of
 // two 64-bit ones and a register pair): for scenes with less than 2^26
-// triangles (kNarrowTris), so that every offset is below 2^32.
+// triangles (kNarrowTris), so that every offset is below 2^32.  At the 8
+// waves/SIMD bound the short form spills 21 VGPRs, the wide one 24.
 constexpr int kNarrowTris = 1 << 26;
 
 template <bool WIDE>

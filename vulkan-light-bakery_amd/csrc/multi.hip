@@ -438,6 +438,15 @@ int multi_grid_size(Context& ctx)
     return (g + 7) & ~7;
 }
 
+// k_fused_jobs at the occupancy bound a.focc.
+template <bool FAR, bool WIDE>
+static void launch_occ(const MultiArgs& a, hipStream_t st)
+{
+    if (a.focc == 8) k_fused_jobs<false, 8, FAR, WIDE><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
+    else if (a.focc == 6) k_fused_jobs<false, 6, FAR, WIDE><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
+    else k_fused_jobs<false, 0, FAR, WIDE><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
+}
+
 void launch_multi_trace(const MultiArgs& a, bool count, int grid, int shade_grid, hipStream_t st)
 {
     VLB_REQUIRE(grid % 8 == 0 && grid > 0, VLB_ERR_INVALID, "multi-job grid must be a multiple of 8");
@@ -448,14 +457,10 @@ void launch_multi_trace(const MultiArgs& a, bool count, int grid, int shade_grid
         VLB_REQUIRE(a.fgrid % 8 == 0 && a.fgrid > 0, VLB_ERR_INVALID, "fused grid must be a multiple of 8");
         if (count && a.far) k_fused_jobs<true, 0, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
         else if (count) k_fused_jobs<true, 0><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-        else if (a.wide) k_fused_jobs<false, 0, false, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-        else if (a.far) {
-            if (a.focc == 8) k_fused_jobs<false, 8, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-            else if (a.focc == 6) k_fused_jobs<false, 6, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-            else k_fused_jobs<false, 0, true><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-        } else if (a.focc == 8) k_fused_jobs<false, 8><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-        else if (a.focc == 6) k_fused_jobs<false, 6><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
-        else k_fused_jobs<false, 0><<<a.fgrid, 256, 0, st>>>(a, a.jobs, a.seg, a.hdr);
+        else if (a.far && a.wide) launch_occ<true, true>(a, st);
+        else if (a.far) launch_occ<true, false>(a, st);
+        else if (a.wide) launch_occ<false, true>(a, st);
+        else launch_occ<false, false>(a, st);
         VLB_HIP(hipGetLastError());
         return;
     }

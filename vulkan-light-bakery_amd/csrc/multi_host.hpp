@@ -59,6 +59,7 @@ struct RoundTable {
     std::vector<Segment> seg;
     std::vector<MergeItem> merge;
     size_t rays = 0;          // primary rays of the round
+    bool wide = false;        // a scene of it has kNarrowTris triangles or more
 };
 // Appends projection tiles [pt0, pt0 + npt) of job `job` to a round.
 void round_add(RoundTable& r, int job, const JobState& js, int pt0, int npt);
@@ -80,15 +81,14 @@ struct RoundBufs {
     int nvis = 0;             // visibility bytes per ray
     uint32_t depth = 0;       // deepest BVH served
     int grid = 0, shade_grid = 0, pgrid = 0, mgrid = 0;
-    bool wide = false;          // a job's scene has kNarrowTris triangles or more
     int fgrid[6] = {};          // fused kernel grids at occupancy 0, 6, 8 (+3: far-first shadows)
     DevBuf rad, hits, vis, wctr, spill, counters;
     void alloc(Context& ctx, size_t cap_tiles, int nvis, uint32_t depth);
     // kernel arguments for the given device tables; focc: -1 for the
     // wavefront kernels, else the fused kernel's occupancy (0, 6, 8); far:
-    // the fused kernel's shadow queries far first
+    // the fused kernel's shadow queries far first; wide: RoundTable::wide
     MultiArgs args(const JobDesc* jobs, const uint8_t* table, const size_t off[3], int map,
-                   int refill, int chunk, int focc, bool far) const;
+                   int refill, int chunk, int focc, bool far, bool wide) const;
 };
 
 // trace_variant -> lane map, refill threshold, fused occupancy and shadow

@@ -23,8 +23,8 @@
 //    step that fails before launch (an injected failure) fails only the
 //    requests whose work it held.  A request holds a use of its scene from
 //    submit until it is done, so the scene cannot be released under it.
-// One hipGraph, captured once, runs every step: the step's counts live in
-// device memory.  A request's coefficients are a function of the request
+// One hipGraph, captured once, runs every step (another those that hold a
+// scene of 2^26 triangles or more): the step's counts live in device memory.  A request's coefficients are a function of the request
 // alone (fixed tile -> partial-sum slot map, fixed merge order), so they
 // are the same alone and in any mix.
 #include <math.h>
@@ -166,8 +166,9 @@ struct Server {
     int map = 3, refill = 32, chunk = 256, focc = -1;
     bool far = false;
     size_t cap_tiles = 0;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    // the step, and the step of RoundTable::wide, each captured on first use
+    hipGraph_t graph[2] = {nullptr, nullptr};
+    hipGraphExec_t gexec[2] = {nullptr, nullptr};
     InFlight fl[2];
     uint64_t step_no = 0;
     // statistics
@@ -284,18 +285,6 @@ bool Server::admit_one(Request* r, size_t& upload_used, std::vector<Upload>& ups
         // lock order: the server's mutex, then the context's
         std::lock_guard<std::recursive_mutex> lk(ctx->mtx);
         Scene& sc = find_scene(*ctx, r->scene);
-        if (sc.ntris >= kNarrowTris && !rb.wide) {
-            // the first request on such a scene: capture the step again with
-            // the kernel for it
-            rb.wide = true;
-            if (gexec) {
-                VLB_HIP(hipStreamSynchronize(stream));
-                (void)hipGraphExecDestroy(gexec);
-                (void)hipGraphDestroy(graph);
-                gexec = nullptr;
-                graph = nullptr;
-            }
-        }
         bool built = false;
         js.rt = cache.get(*ctx, p, K, RS, &built);
         if (built) VLB_HIP(hipStreamSynchronize(ctx->stream));
@@ -398,9 +387,10 @@ void Server::launch_step(const RoundTable& rt, const std::vector<Upload>& ups, u
     VLB_HIP(hipMemcpyAsync(dtab.p, stg, jobtab_bytes + round_cap_bytes, hipMemcpyHostToDevice, st));
     for (const Upload& u : ups)
         VLB_HIP(hipMemcpyAsync(u.dst, stg + u.src, u.bytes, hipMemcpyHostToDevice, st));
-    if (!gexec) {
+    const int w = rt.wide ? 1 : 0;
+    if (!gexec[w]) {
         const MultiArgs a = rb.args(dtab.as<JobDesc>(), dtab.as<uint8_t>() + jobtab_bytes, off, map, refill, chunk,
-                                    focc, far);
+                                    focc, far, rt.wide);
         VLB_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         try {
             launch_multi_trace(a, false, rb.grid, rb.shade_grid, st);
@@ -412,10 +402,10 @@ void Server::launch_step(const RoundTable& rt, const std::vector<Upload>& ups, u
             if (g) (void)hipGraphDestroy(g);
             throw;
         }
-        VLB_HIP(hipStreamEndCapture(st, &graph));
-        VLB_HIP(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
+        VLB_HIP(hipStreamEndCapture(st, &graph[w]));
+        VLB_HIP(hipGraphInstantiate(&gexec[w], graph[w], nullptr, nullptr, 0));
     }
-    VLB_HIP(hipGraphLaunch(gexec, st));
+    VLB_HIP(hipGraphLaunch(gexec[w], st));
     for (Request* r : finishing)
         VLB_HIP(hipMemcpyAsync(res_host + r->res_off, r->js.desc.out, r->res_bytes, hipMemcpyDeviceToHost, st));
     VLB_HIP(hipEventRecord(f.e1, st));
@@ -597,8 +587,10 @@ void destroy_server(Server* s)
     s->cv_sched.notify_all();
     if (s->thr.joinable()) s->thr.join();
     if (s->stream) (void)hipStreamSynchronize(s->stream);
-    if (s->gexec) (void)hipGraphExecDestroy(s->gexec);
-    if (s->graph) (void)hipGraphDestroy(s->graph);
+    for (hipGraphExec_t g : s->gexec)
+        if (g) (void)hipGraphExecDestroy(g);
+    for (hipGraph_t g : s->graph)
+        if (g) (void)hipGraphDestroy(g);
     for (InFlight& f : s->fl) {
         if (f.e0) (void)hipEventDestroy(f.e0);
         if (f.e1) (void)hipEventDestroy(f.e1);
