@@ -2,6 +2,7 @@
 bad geometry, device memory budgets and kept device blocks."""
 import ctypes as C
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -217,3 +218,51 @@ def test_served_direction_sets_fit_a_budget_of_their_tables(prec, per_ray):
         for d in fill:
             c.free(d)
     assert np.array_equal(got[0], want[0])
+
+
+def test_blocks_given_back_while_others_work():
+    """trim() in a loop beside bakes, a server and another context's bakes:
+    everyone's results are those of a quiet run."""
+    s = vlb.generate_scene(vlb.SCENE_ROOM, 2)
+    rng = np.random.default_rng(9)
+    sets = [rng.uniform([1, 0.5, 1], [9, 3.5, 9], (n, 3)).astype(np.float32) for n in (30, 200, 500)]
+    prm = [vlb.Params(probes=q, rays=640, rays_per_slice=640) for q in sets]
+    with vlb.Context() as c, vlb.Context() as other:
+        sid, oid = c.upload_scene_dict(s), other.upload_scene_dict(s)
+        want = [c.bake(sid, p) for p in prm]
+        errors, stop = [], threading.Event()
+
+        def run(f):
+            try:
+                f()
+            except BaseException as e:  # reported by the main thread
+                errors.append(e)
+
+        def bakes(ctx, sid):
+            for _ in range(15):
+                for p, w in zip(prm, want):
+                    assert np.array_equal(ctx.bake(sid, p), w)
+
+        def serves():
+            for _ in range(3):
+                srv = vlb.Server(c, step_rays=1 << 15, state_budget=1 << 24)
+                ids = [srv.submit(sid, p) for p in prm * 3]
+                got = [srv.wait(i)[0] for i in ids]
+                srv.destroy()
+                assert all(np.array_equal(g, w) for g, w in zip(got, want * 3))
+
+        def trims():
+            while not stop.is_set():
+                c.trim()
+                other.trim()
+
+        work = [threading.Thread(target=run, args=(f,)) for f in
+                (lambda: bakes(c, sid), lambda: bakes(other, oid), serves)]
+        trimmer = threading.Thread(target=run, args=(trims,))
+        for t in work + [trimmer]:
+            t.start()
+        for t in work:
+            t.join()
+        stop.set()
+        trimmer.join()
+    assert not errors, errors
