@@ -46,10 +46,10 @@ __global__ void k_zero_ctr8(unsigned long long* c)
 // (tile_map, a.map) sets how many neighbouring probes x directions (probes
 // Morton sorted, directions on a Hilbert curve) one wave covers.
 // OCC > 0 asks the compiler for OCC waves per SIMD (VGPR budget 512/OCC).
-// At 8 waves/SIMD the arguments read per set of rays (kernel_args) leave 20
-// spilled VGPRs instead of 31 and 72 B of scratch per lane instead of 176:
-// 2048 probes x 4096 rays of the 11k-triangle room 0.855 against 0.871 ms per
-// bake, 16,384 x 16,384 of a 1.15M-triangle terrain 33.8 against 34.35.
+// At 8 waves/SIMD the arguments read per set of rays (kernel_args) leave 11
+// spilled VGPRs fewer (21 are left, 76 B of scratch per lane): 2048 probes x
+// 4096 rays of the 11k-triangle room 0.855 against 0.871 ms per bake, 16,384 x
+// 16,384 of a 1.15M-triangle terrain 33.8 against 34.35.
 // IND: plans with the multi-bounce term.  FAR: shadow queries visit children
 // far first (same radiance; fewer node visits on some scenes).
 template <bool RECORD, bool COUNT, int OCC, bool IND, bool FAR = false,

@@ -118,9 +118,10 @@ constexpr int kCtrStride = 16;
 // 0.92 ms per bake against 0.87.  Sharing what is known by more than a
 // workgroup costs more than it saves (flags per XCD in memory: 1.0 ms;
 // accesses to one line from all waves serialise), and looking only into some
-// of the other XCDs' ranges leaves the launch unbalanced (terrain +3%).  In the
-// multi-job kernel, with its arguments read per set of rays: 24 jobs over
-// three scenes 69.7 ms against 69.4, a burst of 20 requests 41.4 against 40.9.
+// of the other XCDs' ranges leaves the launch unbalanced (terrain +3%).  The
+// multi-job kernel took it over together with arguments read per set of rays
+// (kernel_args): 24 jobs over three scenes 69.5 ms instead of 69.9, a burst of
+// 20 requests 41.2 instead of 41.5.
 struct WorkRanges {
     unsigned long long* ctr;
     size_t nitems, per;

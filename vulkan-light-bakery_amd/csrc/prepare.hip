@@ -6,9 +6,9 @@
 // On the host these were the larger part of a one-shot bake: 97 ms of a 113 ms
 // bake of 343 probes x 785,500 equirect rays (a double-precision basis of 16
 // functions and a sort per ray), most of a millisecond at 4096 rays.  Here
-// each is one thread per ray or probe around a radix sort, bound by launch
-// latency at a few thousand rays and by the table writes (80 B per ray in
-// FP32) at millions: 0.3 ms for 785,500 rays.
+// each is one thread per ray or probe around a library sort, bound by launch
+// latency at a few thousand rays and by the sort's passes at a million: 0.18
+// ms for 785,500 rays (keys 11 us, sort 150, rows 17).
 //
 // Every value is computed by the operation sequence of the host code it
 // replaces (no contraction, correctly rounded divide and square root, the
