@@ -266,3 +266,13 @@ def test_blocks_given_back_while_others_work():
         stop.set()
         trimmer.join()
     assert not errors, errors
+
+
+def test_a_new_context_counts_kept_blocks_as_free():
+    """The default budget is the device's free memory: what another context
+    keeps of it is not missing there."""
+    with vlb.Context() as c:
+        sid = c.upload_scene(np.zeros((0, 3), np.float32), np.zeros((0, 3), np.uint32))
+        _plans(c, sid, 1, 131072)[0].destroy()                # 1.5 GiB kept
+        with vlb.Context() as other:
+            other.free(other.alloc(_free_bytes() + (512 << 20)))

@@ -47,6 +47,12 @@ DevPool::~DevPool()
     }
     shrink(0);
 }
+void DevPool::set_device(int device, size_t limit_bytes)
+{
+    std::lock_guard<std::mutex> lk(mu_);
+    device_ = device;
+    limit_ = limit_bytes;
+}
 void* DevPool::take(size_t cap)
 {
     std::lock_guard<std::mutex> lk(mu_);
@@ -105,6 +111,17 @@ void DevPool::trim_all()
     PoolList& l = pool_list();
     std::lock_guard<std::mutex> lk(l.mu);
     for (DevPool* p : l.pools) p->shrink(0);
+}
+size_t DevPool::kept_on(int device)
+{
+    PoolList& l = pool_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    size_t sum = 0;
+    for (DevPool* p : l.pools) {
+        std::lock_guard<std::mutex> pk(p->mu_);
+        if (p->device_ == device) sum += p->kept_;
+    }
+    return sum;
 }
 
 DevBuf dev_alloc(Context& ctx, size_t bytes, bool pooled)
@@ -528,8 +545,9 @@ vlb_status vlb_ctx_create(int32_t device, uint64_t hbm_budget_bytes, vlb_ctx** o
         c->name = prop.gcnArchName;
         size_t freeb = 0, total = 0;
         VLB_HIP(hipMemGetInfo(&freeb, &total));
-        c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)freeb;
-        c->pool.set_limit(total / kPoolShare);
+        // what other contexts keep makes room when asked for: it is free
+        c->budget = hbm_budget_bytes ? hbm_budget_bytes : (uint64_t)(freeb + DevPool::kept_on(device));
+        c->pool.set_device(device, total / kPoolShare);
         VLB_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         for (auto& e : c->ev) VLB_HIP(hipEventCreate(&e));
         c->sky_scratch = skybox_scratch_init(device);

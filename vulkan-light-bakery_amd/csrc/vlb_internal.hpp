@@ -65,11 +65,12 @@ public:
     ~DevPool();
     DevPool(const DevPool&) = delete;
     DevPool& operator=(const DevPool&) = delete;
-    void set_limit(size_t bytes) { limit_ = bytes; }
+    void set_device(int device, size_t limit_bytes);
     void* take(size_t cap);                 // the block last kept, or null
     void put(void* p, size_t cap) noexcept;
     void shrink(size_t keep);               // frees the oldest beyond `keep` bytes
     static void trim_all();                 // of every context in the process
+    static size_t kept_on(int device);      // by every context in the process
 
 private:
     struct Block {
@@ -80,6 +81,7 @@ private:
     std::list<Block> age_;                                    // oldest first
     std::multimap<size_t, std::list<Block>::iterator> size_;  // by capacity
     size_t kept_ = 0, limit_ = 0;
+    int device_ = -1;
     void drop_oldest(size_t keep, std::list<Block>& out);     // with mu_ held
 };
 constexpr size_t kPoolShare = 32;  // of the device's memory: 9 of 288 GB
