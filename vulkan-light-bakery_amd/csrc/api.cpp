@@ -535,8 +535,11 @@ vlb_status vlb_ctx_create(int32_t device, uint64_t hbm_budget_bytes, vlb_ctx** o
         return VLB_ERR_NO_DEVICE;
     }
     if (device < 0 || device >= n) return VLB_ERR_INVALID;
-    Context* c = new Context();
-    vlb_status s = guard(c, [&] {
+    Context* c = nullptr;
+    // joins the process's pools, which allocates: no exception leaves here
+    vlb_status s = guard(nullptr, [&] { c = new Context(); });
+    if (s != VLB_OK) return s;
+    s = guard(c, [&] {
         c->device = device;
         VLB_HIP(hipSetDevice(device));
         hipDeviceProp_t prop;
