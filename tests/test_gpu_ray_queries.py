@@ -64,3 +64,29 @@ def test_any_direction_length_and_far_origins(ctx, floor, dist, length):
         assert want[0][0] >= 0 and want[1][0] == t
         got = ctx.trace_closest(sid, org[i], d[i], t, tmax)
         assert got[0][0] == want[0][0] and got[1][0] == t
+
+
+@pytest.mark.parametrize("length", [1e-32, 1e-30, 1e-20, 1e20, 1e30])
+def test_directions_at_the_ends_of_the_float_range(ctx, floor, length):
+    """Distances up to 10^32 and down to 10^-30: the oracle's hits."""
+    sid, o = floor
+    org, d = _rays(2.0, length)
+    tmax = np.float32(3e38)
+    ref = o.trace_closest(org, d, 0.0, tmax, brute=True)
+    assert (ref[0] >= 0).sum() > 100
+    got = ctx.trace_closest(sid, org, d, 0.0, tmax)
+    for g, r in zip(got, ref):
+        assert np.array_equal(g, r)
+
+
+def test_zero_directions_hit_nothing(ctx, floor):
+    """... and take no longer than the rays of a usual call (a rejected box
+    ends each at the root or a few nodes below)."""
+    sid, o = floor
+    org = np.random.default_rng(1).uniform(-1, 1, (100_000, 3)).astype(np.float32)
+    org[:1000] = 0.0
+    d = np.zeros_like(org)
+    d[::2] = -0.0
+    for tmax in (np.float32(1e30), np.float32(np.inf)):
+        assert (ctx.trace_closest(sid, org, d, 0.0, tmax)[0] == -1).all()
+        assert not ctx.trace_occluded(sid, org, d, np.full(len(org), tmax), 0.0).any()

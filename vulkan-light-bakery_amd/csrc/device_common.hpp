@@ -300,7 +300,7 @@ __host__ __device__ __forceinline__ float box_margin(float maxabs)
 // a power of two (rounded down, the margin has room), not below 1.
 __device__ __forceinline__ float wt_scale(const WtRay& w)
 {
-    return fmaxf(1.0f, fminf(0x1p58f, __uint_as_float(__float_as_uint(w.Sz) & 0x7F800000u)));
+    return fmaxf(1.0f, fminf(0x1p100f, __uint_as_float(__float_as_uint(w.Sz) & 0x7F800000u)));
 }
 
 __device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, const WtRay& w, float maxabs,
@@ -310,9 +310,10 @@ __device__ __forceinline__ SlabRay slab_setup(const float3& o, const float3& d, 
     const float m = fmaxf(maxabs, fmaxf(fabsf(o.x), fmaxf(fabsf(o.y), fabsf(o.z))));
     // a component this small against the largest moves the ray by less than
     // the margin over the whole scene; the second bound keeps unit / d and
-    // o / d finite
+    // o / d finite, the third a zero direction from meeting every box
     const float dm = fmaxf(fabsf(d.x), fmaxf(fabsf(d.y), fabsf(d.z)));
-    const float dmin = fmaxf(fminf(1e-20f, dm * 0x1p-46f), fmaxf(m, 64.0f) * 0x1p-126f);
+    const float dmin = fmaxf(fmaxf(fminf(1e-20f, dm * 0x1p-46f), fminf(dm * 0x1p-18f, m * 0x1p-126f)),
+                             0x1p-126f);
     const float dx = fabsf(d.x) < dmin ? copysignf(dmin, d.x) : d.x;
     const float dy = fabsf(d.y) < dmin ? copysignf(dmin, d.y) : d.y;
     const float dz = fabsf(d.z) < dmin ? copysignf(dmin, d.z) : d.z;
